@@ -41,15 +41,18 @@ typedef struct rg_weights* rg_weights_t;
 
 /* Tuning of the build.  Zero fields select the defaults. */
 typedef struct rg_tuning {
-    int32_t edges_per_lane; /* sweep edges walked by one lane (default 16) */
+    int32_t edges_per_lane; /* sweep edges walked by one lane, in every pass
+                               (default: per pass, by the expected work) */
     int32_t block;          /* threads per block of the walk kernels (128; a
                                multiple of 64, at most 512) */
     int32_t flags;          /* RG_TUNE_TIMINGS: record per-phase times;
                                RG_TUNE_GUESS_OUTSIDE, RG_TUNE_ROW_WAVES: test
                                hooks */
     int32_t stage_per_edge; /* triples staged per sweep edge by the counting
-                               walk (default 8); chunks that emit more are
-                               walked a second time */
+                               walk (default: from the expected work, 8 when
+                               edges_per_lane is given; 16 edges per lane
+                               when only this is given); chunks that emit
+                               more are walked a second time */
 } rg_tuning;
 
 #define RG_TUNE_TIMINGS 1

@@ -22,6 +22,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <memory>
 #include <string>
@@ -589,16 +590,18 @@ __global__ __launch_bounds__(WALK_MAX_BLOCK) void k_chunk_start(const Build* __r
     const ChunkRef r = chunk_of_thread(B, t - B.thread_gbase);
     if (!r.valid || r.c == 0) return;
     start[B.chunk_gbase + r.g] =
-        guess_outside ? STATE_OUTSIDE : chunk_start_guess(pass_of_wave(B, r), r.row, r.c * B.K);
+        guess_outside ? STATE_OUTSIDE : [&] {
+            const Pass& P = pass_of_wave(B, r);
+            return chunk_start_guess(P, r.row, r.c * P.K);
+        }();
 }
 
 // ---- walks ---------------------------------------------------------------
 
-__device__ inline void chunk_range(const Build& B, const Pass& P, int64_t c,
-                                   int64_t* k0, int64_t* k1)
+__device__ inline void chunk_range(const Pass& P, int64_t c, int64_t* k0, int64_t* k1)
 {
-    *k0 = c * B.K;
-    int64_t e = *k0 + B.K;
+    *k0 = c * P.K;
+    int64_t e = *k0 + P.K;
     *k1 = e < P.nk - 1 ? e : P.nk - 1;
     if (*k1 < *k0) *k1 = *k0;
 }
@@ -620,7 +623,7 @@ __global__ __launch_bounds__(WALK_MAX_BLOCK) void k_walk_count(const Build* __re
     const Pass& P = pass_of_wave(B, r);
     const int64_t g = B.chunk_gbase + r.g;
     int64_t k0, k1;
-    chunk_range(B, P, r.c, &k0, &k1);
+    chunk_range(P, r.c, &k0, &k1);
     StageSink sink{0, t, cap, stage, hist + (B.cell_gbase >> 6), r.p, ngroups_all, {}};
     end[g] = walk_chunk(B, P, r.row, k0, k1, start[g], sink);
     sink.flush();
@@ -663,7 +666,7 @@ __global__ __launch_bounds__(WALK_MAX_BLOCK) void k_fixup(const Build* __restric
         if (truth == STATE_FAILED) break;
         if (start[g] == truth) continue;
         int64_t k0, k1;
-        chunk_range(B, P, c, &k0, &k1);
+        chunk_range(P, c, &k0, &k1);
         UncountSink undo{hist, p, ngroups_all, {}};
         (void)walk_chunk(B, P, row, k0, k1, start[g], undo);
         undo.flush();
@@ -720,7 +723,7 @@ __global__ __launch_bounds__(WALK_MAX_BLOCK) void k_restage(const Build* __restr
     if (count[g] <= cap) return;
     const Pass& P = pass_of_wave(B, r);
     int64_t k0, k1;
-    chunk_range(B, P, r.c, &k0, &k1);
+    chunk_range(P, r.c, &k0, &k1);
     // (a capacity-mode build sizes the buffer in advance: a chunk past its
     // end keeps nothing, and the build's flag reports it)
     const int64_t room = ov_cap - ov_off[g];
@@ -1862,6 +1865,91 @@ __global__ void k_graph_jobs(JobDesc* __restrict__ jobs, const int32_t* __restri
     jobs[j].w = v_out + bases[2 * k];
 }
 
+// The split of the sweep rows into chunks, one walk thread each, and the
+// triples staged per thread.
+//
+// A chunk is a serial chain of dependent loads and divisions, whose time grows
+// with its triples (t of them), and costs a start search, whose time grows
+// with the number of chunks (all triples W / t): their sum is least at a t
+// that grows as sqrt(W).  A pass's edges emit about 2 (1 + c) triples each
+// when they cross c static cell edges, c from the grids' cell counts (they
+// are taken to cover each other, at a mean angle), and a pass's chunk is as
+// many edges as make t.  Build times, 16 edges for every pass -> this rule:
+//   67 x 190 -> 81 x 125 vertices   813 -> 389 us (the walk alone 469 -> 68)
+//   129^2 -> 101^2                  721 -> 322
+//   513^2 -> 385^2                  692 -> 485 (2 edges 483, 4 edges 478)
+//   1025^2 -> 769^2                1013 -> 930 (4 edges 939, 8 edges 922)
+// and from about 2000^2 on t is at its bound, MAX_TRIPLES, and the chunks
+// are the 16 edges they were.  Coarse sweeps over fine static grids get
+// shorter chunks than the others, so that one staging capacity, 1.8 times
+// the expected triples, serves all: with 8 triples per edge for every pass
+// chunks of mixed batches overflowed and walked twice (64 pairs of 33 to
+// 1025 vertices per axis: the build 6.84 -> 5.56 ms).
+//
+// An explicit edges_per_lane or stage_per_edge applies to every pass as given
+// (a missing one of the two is 16 edges, or 8 triples).
+struct WalkShape {
+    static constexpr double MAX_TRIPLES = 72;
+    static constexpr int64_t MAX_EDGES = 32, MIN_CAP = 16, MAX_CAP = 128;
+    int64_t K;           // edges per chunk of every pass; 0: by expected work
+    double target = 1;   // expected triples of a chunk
+    int64_t cap;         // triples staged per walk thread
+
+    struct Dims {
+        int64_t rows, edges;  // sweep rows, edges per row
+        double per_edge;      // expected triples per edge
+    };
+
+    static Dims dims(const rg_pair_desc& d, int p)
+    {
+        const bool in = p >= 2;
+        const int64_t nxs = in ? d.nxi : d.nxo, nys = in ? d.nyi : d.nyo;
+        const int64_t nxt = in ? d.nxo : d.nxi, nyt = in ? d.nyo : d.nyi;
+        Dims q;
+        q.rows = (p & 1) ? nxs : nys;
+        q.edges = ((p & 1) ? nys : nxs) - 1;
+        // 2 / pi: the mean of |cos| and |sin| over the angle
+        const double c = 0.64 * (double)(nxt - 1 + nyt - 1) / (double)q.edges;
+        q.per_edge = 2 * (1 + c);
+        return q;
+    }
+
+    WalkShape(const rg_pair_desc* pairs, int64_t npairs, int64_t edges, int64_t per_edge)
+    {
+        if (edges > 0 || per_edge > 0) {
+            K = edges > 0 ? edges : 16;
+            cap = K * (per_edge > 0 ? per_edge : 8);
+            return;
+        }
+        K = 0;
+        double work = 0;
+        for (int64_t k = 0; k < npairs; k++)
+            for (int p = 0; p < 4; p++) {
+                const Dims q = dims(pairs[k], p);
+                work += (double)q.rows * (double)q.edges * q.per_edge;
+            }
+        target = std::min(std::sqrt(work) / 105, MAX_TRIPLES);
+        double most = 0;
+        for (int64_t k = 0; k < npairs; k++)
+            for (int p = 0; p < 4; p++)
+                most = std::max(most, (double)edges_per_chunk(pairs[k], p) *
+                                          dims(pairs[k], p).per_edge);
+        cap = std::min(MAX_CAP, std::max(MIN_CAP, (int64_t)(1.8 * most) + 1));
+    }
+
+    // Edges per chunk of pass p of a pair: the target's, spread evenly over
+    // the chunks of a row.
+    int64_t edges_per_chunk(const rg_pair_desc& d, int p) const
+    {
+        if (K > 0) return K;
+        const Dims q = dims(d, p);
+        int64_t e = (int64_t)(target / q.per_edge + 0.5);
+        e = std::max<int64_t>(1, std::min({e, MAX_EDGES, q.edges}));
+        const int64_t chunks = (q.edges + e - 1) / e;
+        return (q.edges + chunks - 1) / chunks;
+    }
+};
+
 int build_batched(const rg_pair_desc* pairs, int64_t npairs,
                   const rg_tuning* tuning, rg_weights** out, hipStream_t s,
                   CaptureCaps* caps);
@@ -1897,7 +1985,7 @@ int build_batched(const rg_pair_desc* pairs, int64_t npairs,
         if (d.nxi * d.nyi >= INT32_MAX || d.nxo * d.nyo >= INT32_MAX)
             return fail(RG_ERR_ARGUMENT, "more than 2^31 - 1 vertices in one grid" + at);
     }
-    int64_t K = 16, stage_per_edge = 8;
+    int64_t K = 0, stage_per_edge = 0;  // 0: chosen below
     int block = 128;
     bool timings = false;
     int32_t flags = 0;
@@ -1990,6 +2078,8 @@ int build_batched(const rg_pair_desc* pairs, int64_t npairs,
         S.nsup = sup_pf[g + 1] - sup_pf[g];
     }
 
+    const WalkShape shape(pairs, npairs, K, stage_per_edge);
+
     std::vector<PairCells> pcs(npairs);
     std::vector<Build> builds(npairs);
     std::vector<int64_t> wave_pf(npairs + 1), row_pf(npairs + 1),
@@ -2010,7 +2100,7 @@ int build_batched(const rg_pair_desc* pairs, int64_t npairs,
         P.cell_gbase = cell_tot;
         P.out_gbase = out_tot;
         Build& B = builds[k];
-        B.K = K;
+        B.K = 0;
         int64_t chunk = 0, rows = 0, threads = 0;
         for (int p = 0; p < 4; p++) {
             Pass& Q = B.pass[p];
@@ -2030,7 +2120,9 @@ int build_batched(const rg_pair_desc* pairs, int64_t npairs,
             Q.axis = axis;
             Q.sweep_input = sweep_input;
             Q.st = sweep_input ? sg[2 * k + 1] : sg[2 * k];
-            Q.cpr = std::max<int64_t>(1, (Q.nk - 1 + K - 1) / K);
+            Q.K = shape.edges_per_chunk(d, p);
+            Q.cpr = std::max<int64_t>(1, (Q.nk - 1 + Q.K - 1) / Q.K);
+            B.K = std::max(B.K, Q.K);
             Q.chunk_base = chunk;
             Q.thread_base = threads;
             B.row_base[p] = rows;
@@ -2207,7 +2299,7 @@ int build_batched(const rg_pair_desc* pairs, int64_t npairs,
     tm.mark();  // 2
 
     // ---- count (staging the triples)
-    const int64_t cap = K * stage_per_edge;
+    const int64_t cap = shape.cap;
     DevBuf<Triple> stage;
     RG_TRY(stage.alloc((size_t)thr_tot * cap, s));
     k_walk_count<<<grid_for(thr_tot, block), block, 0, s>>>(

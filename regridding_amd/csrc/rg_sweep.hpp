@@ -72,6 +72,7 @@ struct Pass {
     int32_t axis;            // 0: aligned view is the transpose
     int32_t sweep_input;     // 1: sweep = input grid, static = output grid
     StaticGrid st;
+    int64_t K;               // edges per chunk of this pass
     int64_t chunk_base;      // global id of the first chunk of this pass
     int64_t cpr;             // chunks per row
     int64_t thread_base;     // first walk thread of this pass
@@ -79,7 +80,7 @@ struct Pass {
 
 struct Build {
     Pass pass[4];            // F axis 0, F axis 1, T axis 0, T axis 1
-    int64_t K;               // edges per chunk
+    int64_t K;               // edges per chunk (the most of any pass)
     int64_t nchunks;
     int64_t nrows_total;
     int64_t row_base[4];     // id of the first row of each pass
