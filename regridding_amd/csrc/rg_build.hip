@@ -1877,8 +1877,10 @@ __global__ void k_graph_jobs(JobDesc* __restrict__ jobs, const int32_t* __restri
 // many edges as make t.  Build times, 16 edges for every pass -> this rule:
 //   67 x 190 -> 81 x 125 vertices   813 -> 389 us (the walk alone 469 -> 68)
 //   129^2 -> 101^2                  721 -> 322
+//   257^2 -> 193^2                  610 -> 354 (2 edges 359)
 //   513^2 -> 385^2                  692 -> 485 (2 edges 483, 4 edges 478)
 //   1025^2 -> 769^2                1013 -> 930 (4 edges 939, 8 edges 922)
+// (below ONE_EDGE_WORK triples, about 270^2 -> 200^2, every chunk is one edge)
 // and from about 2000^2 on t is at its bound, MAX_TRIPLES, and the chunks
 // are the 16 edges they were.  Coarse sweeps over fine static grids get
 // shorter chunks than the others, so that one staging capacity, 1.8 times
@@ -1889,7 +1891,7 @@ __global__ void k_graph_jobs(JobDesc* __restrict__ jobs, const int32_t* __restri
 // An explicit edges_per_lane or stage_per_edge applies to every pass as given
 // (a missing one of the two is 16 edges, or 8 triples).
 struct WalkShape {
-    static constexpr double MAX_TRIPLES = 72;
+    static constexpr double MAX_TRIPLES = 72, ONE_EDGE_WORK = 1e6;
     static constexpr int64_t MAX_EDGES = 32, MIN_CAP = 16, MAX_CAP = 128;
     int64_t K;           // edges per chunk of every pass; 0: by expected work
     double target = 1;   // expected triples of a chunk
@@ -1928,7 +1930,7 @@ struct WalkShape {
                 const Dims q = dims(pairs[k], p);
                 work += (double)q.rows * (double)q.edges * q.per_edge;
             }
-        target = std::min(std::sqrt(work) / 105, MAX_TRIPLES);
+        target = work < ONE_EDGE_WORK ? 1 : std::min(std::sqrt(work) / 105, MAX_TRIPLES);
         double most = 0;
         for (int64_t k = 0; k < npairs; k++)
             for (int p = 0; p < 4; p++)
