@@ -193,7 +193,8 @@ enum : int64_t {
     RG_SEARCH_BRUTE = -2,    // the reference falls back to index_of_point_brute
 };
 
-// _grids.py:356-463 index_of_point_secant without its brute-force fallback:
+// _grids.py:356-463 index_of_point_secant without its brute-force fallback,
+// statement by statement (what secant_search below is checked against):
 // returns the flat cell index, RG_SEARCH_OUTSIDE, or RG_SEARCH_BRUTE when
 // the reference would scan every cell (singular Jacobian or 100 iterations
 // without a decision).  The caller runs the exhaustive search cooperatively.
@@ -234,83 +235,157 @@ RG_HD int64_t index_secant(const double* __restrict__ x,
     return RG_SEARCH_BRUTE;
 }
 
-// The cell search over an interleaved (x, y) vertex array: the same
-// arithmetic as bilinear / cell_contains / index_local / index_secant on
-// the separate arrays, with one 16-byte load per vertex instead of two.
-RG_HD double2 bilinear_xy(const double2* __restrict__ a, int64_t nx, int64_t ny, double x,
-                          double y)
-{
-    int64_t x0 = floor_i64(x), y0 = floor_i64(y);
-    if (x0 < 0) x0 = 0;
-    else if (x0 > nx - 2) x0 = nx - 2;
-    if (y0 < 0) y0 = 0;
-    else if (y0 > ny - 2) y0 = ny - 2;
-    const double2 a00 = gload(a, x0 * ny + y0);
-    const double2 a01 = gload(a, x0 * ny + y0 + 1);
-    const double2 a10 = gload(a, (x0 + 1) * ny + y0);
-    const double2 a11 = gload(a, (x0 + 1) * ny + y0 + 1);
-    double dx = x - (double)x0;
-    double dy = y - (double)y0;
-    double w00 = (1 - dx) * (1 - dy);
-    double w01 = (1 - dx) * dy;
-    double w10 = dx * (1 - dy);
-    double w11 = dx * dy;
-    double2 r;
-    r.x = (a00.x * w00) + (a01.x * w01) + (a10.x * w10) + (a11.x * w11);
-    r.y = (a00.y * w00) + (a01.y * w01) + (a10.y * w10) + (a11.y * w11);
-    return r;
-}
+// ---- the same search, reading each vertex once -------------------------------
+//
+// index_secant above evaluates the bilinear map three times per iteration
+// and the cell test from memory, 32 loads in three dependent round trips, and
+// tests the 3 x 3 block cell by cell.  secant_search returns the same answer
+// from the same arithmetic: an iteration loads its cell's four corners once
+// for the map, its two differences (which leave the cell only near its
+// edge) and the cell test, and the block's vertices are requested together.
 
-RG_HD bool cell_contains_xy(const double2* __restrict__ xy, int64_t ny, int64_t i, int64_t j,
-                            double px, double py)
+// Vertex access: index -> (x, y).
+struct VertexXY {  // interleaved vertices
+    const double2* xy;
+    RG_HD double2 operator()(int64_t i) const { return gload(xy, i); }
+};
+struct VertexArrays {
+    const double* x;
+    const double* y;
+    RG_HD double2 operator()(int64_t i) const
+    {
+        double2 v;
+        v.x = gload(x, i);
+        v.y = gload(y, i);
+        return v;
+    }
+};
+
+// The cell (i, j) with corners c0..c3 = (i, j) (i + 1, j) (i + 1, j + 1)
+// (i, j + 1) contains the point: the sum of cell_contains.
+//
+// Most cells asked about lie clearly beside the point, and then the sum is
+// zero: every term is zero where all corners lie strictly above or all
+// strictly below it; with all corners strictly on one side in x, each edge
+// across the point's height counts by its direction alone and the closed
+// polygon's directions cancel.  (An edge's side is computed from its
+// intersection, so x must clear the point by more than the rounding; whether
+// it crosses from a product of the heights, which must not vanish; neither
+// may overflow.)
+RG_HD bool quad_contains(double2 c0, double2 c1, double2 c2, double2 c3, double px, double py)
 {
-    int64_t a = i * ny + j, b = (i + 1) * ny + j;
-    const double2 v0 = gload(xy, a), v1 = gload(xy, b), v2 = gload(xy, b + 1),
-                  v3 = gload(xy, a + 1);
+    const double b0 = c0.y - py, b1 = c1.y - py, b2 = c2.y - py, b3 = c3.y - py;
+    if ((b0 > 0 && b1 > 0 && b2 > 0 && b3 > 0) || (b0 < 0 && b1 < 0 && b2 < 0 && b3 < 0))
+        return false;
+    const double h0 = __builtin_fabs(b0), h1 = __builtin_fabs(b1);
+    const double h2 = __builtin_fabs(b2), h3 = __builtin_fabs(b3);
+    const double tiny = 1e-150, huge = 1e150;
+    if (h0 > tiny && h1 > tiny && h2 > tiny && h3 > tiny && (h0 + h1) + (h2 + h3) < huge) {
+        const double a0 = c0.x - px, a1 = c1.x - px, a2 = c2.x - px, a3 = c3.x - px;
+        const double lo = fmin(fmin(a0, a1), fmin(a2, a3)), hi = fmax(fmax(a0, a1), fmax(a2, a3));
+        // (fmin and fmax pass over a NaN; the sum does not)
+        if (__builtin_fabs((a0 + a1) + (a2 + a3)) < huge &&
+            ((lo > 0 && lo > 1e-6 * hi) || (hi < 0 && hi < 1e-6 * lo)))
+            return false;
+    }
     double w = 0;
-    w += winding_term(px, py, v3.x, v3.y, v0.x, v0.y);
-    w += winding_term(px, py, v0.x, v0.y, v1.x, v1.y);
-    w += winding_term(px, py, v1.x, v1.y, v2.x, v2.y);
-    w += winding_term(px, py, v2.x, v2.y, v3.x, v3.y);
+    w += winding_term(px, py, c3.x, c3.y, c0.x, c0.y);
+    w += winding_term(px, py, c0.x, c0.y, c1.x, c1.y);
+    w += winding_term(px, py, c1.x, c1.y, c2.x, c2.y);
+    w += winding_term(px, py, c2.x, c2.y, c3.x, c3.y);
     return w != 0;
 }
 
-RG_HD int64_t index_local_xy(const double2* __restrict__ xy, int64_t nx, int64_t ny,
-                             int64_t i0, int64_t j0, double px, double py)
-{
-    int64_t ncx = nx - 1, ncy = ny - 1;
-    int64_t ia = i0 - 1 > 0 ? i0 - 1 : 0, ib = i0 + 2 < ncx ? i0 + 2 : ncx;
-    int64_t ja = j0 - 1 > 0 ? j0 - 1 : 0, jb = j0 + 2 < ncy ? j0 + 2 : ncy;
-    for (int64_t ii = ia; ii < ib; ii++)
-        for (int64_t jj = ja; jj < jb; jj++)
-            if (cell_contains_xy(xy, ny, ii, jj, px, py)) return ii * ncy + jj;
-    return -1;
-}
-
-RG_HD int64_t index_secant_xy(const double2* __restrict__ xy, int64_t nx, int64_t ny,
-                              double px, double py)
+// index_secant with the result as a row and a column: 0 and (*ci, *cj), or
+// RG_SEARCH_OUTSIDE, or RG_SEARCH_BRUTE.
+template <class V>
+RG_HD int64_t secant_search(const V& vtx, int64_t nx, int64_t ny, double px, double py,
+                            int64_t* ci, int64_t* cj)
 {
     const double h = 1e-3;
-    int64_t ncx = nx - 1, ncy = ny - 1;
+    const int64_t ncx = nx - 1, ncy = ny - 1;
+    const double last_x = (double)(nx - 2), last_y = (double)(ny - 2);
     double i = (double)nx / 2;
     double j = (double)ny / 2;
     for (int it = 0; it < 100; it++) {
-        const double2 v = bilinear_xy(xy, nx, ny, i, j);
+        // the cell of (i, j), clamped into the grid (NaN: the first one)
+        const double fi = __builtin_floor(i), fj = __builtin_floor(j);
+        const double x0 = !(fi > 0) ? 0 : (fi > last_x ? last_x : fi);
+        const double y0 = !(fj > 0) ? 0 : (fj > last_y ? last_y : fj);
+        const int64_t a = (int64_t)x0 * ny + (int64_t)y0;
+        const double2 c00 = vtx(a), c01 = vtx(a + 1), c10 = vtx(a + ny), c11 = vtx(a + ny + 1);
+        const auto blend = [](double2 v00, double2 v01, double2 v10, double2 v11, double dx,
+                              double dy) {
+            const double w00 = (1 - dx) * (1 - dy);
+            const double w01 = (1 - dx) * dy;
+            const double w10 = dx * (1 - dy);
+            const double w11 = dx * dy;
+            double2 r;
+            r.x = (v00.x * w00) + (v01.x * w01) + (v10.x * w10) + (v11.x * w11);
+            r.y = (v00.y * w00) + (v01.y * w01) + (v10.y * w10) + (v11.y * w11);
+            return r;
+        };
+        // the map at (u, v), from the corners at hand where that is the same cell
+        const auto map = [&](double u, double v) {
+            const double fu = __builtin_floor(u), fv = __builtin_floor(v);
+            const double u0 = !(fu > 0) ? 0 : (fu > last_x ? last_x : fu);
+            const double v0 = !(fv > 0) ? 0 : (fv > last_y ? last_y : fv);
+            if (u0 == x0 && v0 == y0) return blend(c00, c01, c10, c11, u - x0, v - y0);
+            const int64_t b = (int64_t)u0 * ny + (int64_t)v0;
+            return blend(vtx(b), vtx(b + 1), vtx(b + ny), vtx(b + ny + 1), u - u0, v - v0);
+        };
+        const double2 v = blend(c00, c01, c10, c11, i - x0, j - y0);
         const double xv = v.x, yv = v.y;
-        int64_t i0 = floor_i64(i), j0 = floor_i64(j);
-        double ex = xv - px;
-        double ey = yv - py;
-        if (i0 >= 0 && j0 >= 0 && i0 < ncx && j0 < ncy &&
-            cell_contains_xy(xy, ny, i0, j0, px, py)) {
-            int64_t c = index_local_xy(xy, nx, ny, i0, j0, px, py);
-            return c >= 0 ? c : RG_SEARCH_OUTSIDE;
+        const double ex = xv - px;
+        const double ey = yv - py;
+        const bool in = fi >= 0 && fj >= 0 && fi < (double)ncx && fj < (double)ncy &&
+                        quad_contains(c00, c10, c11, c01, px, py);
+        if (in || (__builtin_fabs(ex) < 1e-10 && __builtin_fabs(ey) < 1e-10)) {
+            // the lowest-index cell of the 3 x 3 block around (fi, fj) that
+            // contains the point: its 4 x 4 vertices row by row, clamped
+            // into the grid (cells outside it are passed over).  (A point
+            // the cell itself contains needs only the cells before it.)
+            if (!(fi >= -2 && fj >= -2 && fi <= (double)ncx && fj <= (double)ncy))
+                return RG_SEARCH_OUTSIDE;  // no cell of the block is in the grid
+            const int64_t i0 = (int64_t)fi, j0 = (int64_t)fj;
+            double2 lo[4], hi[4];
+            const auto row = [&](int64_t r, double2* to) {
+                const int64_t rr = r < 0 ? 0 : (r > nx - 1 ? nx - 1 : r);
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const int64_t cc = j0 - 1 + q;
+                    to[q] = vtx(rr * ny + (cc < 0 ? 0 : (cc > ny - 1 ? ny - 1 : cc)));
+                }
+            };
+            row(i0 - 1, lo);
+            row(i0, hi);
+#pragma unroll
+            for (int r = 0; r < 3; r++) {
+                const int64_t ii = i0 - 1 + r;
+#pragma unroll
+                for (int q = 0; q < 3; q++) {
+                    const int64_t jj = j0 - 1 + q;
+                    if (in && r == 1 && q == 1) {
+                        *ci = i0;
+                        *cj = j0;
+                        return 0;
+                    }
+                    if (ii >= 0 && ii < ncx && jj >= 0 && jj < ncy &&
+                        quad_contains(lo[q], hi[q], hi[q + 1], lo[q + 1], px, py)) {
+                        *ci = ii;
+                        *cj = jj;
+                        return 0;
+                    }
+                }
+                if (r == 2) break;
+#pragma unroll
+                for (int q = 0; q < 4; q++) lo[q] = hi[q];
+                row(i0 + 1 + r, hi);
+            }
+            return RG_SEARCH_OUTSIDE;
         }
-        if (__builtin_fabs(ex) < 1e-10 && __builtin_fabs(ey) < 1e-10) {
-            int64_t c = index_local_xy(xy, nx, ny, i0, j0, px, py);
-            return c >= 0 ? c : RG_SEARCH_OUTSIDE;
-        }
-        const double2 vi = bilinear_xy(xy, nx, ny, i + h, j);
-        const double2 vj = bilinear_xy(xy, nx, ny, i, j + h);
+        const double2 vi = map(i + h, j);
+        const double2 vj = map(i, j + h);
         double dx_di = (vi.x - xv) / h;
         double dx_dj = (vj.x - xv) / h;
         double dy_di = (vi.y - yv) / h;
@@ -323,6 +398,15 @@ RG_HD int64_t index_secant_xy(const double2* __restrict__ xy, int64_t nx, int64_
         j -= dj;
     }
     return RG_SEARCH_BRUTE;
+}
+
+// secant_search over interleaved vertices, with index_secant's result.
+RG_HD int64_t index_secant_xy(const double2* __restrict__ xy, int64_t nx, int64_t ny,
+                              double px, double py)
+{
+    int64_t ci = 0, cj = 0;
+    const int64_t r = secant_search(VertexXY{xy}, nx, ny, px, py, &ci, &cj);
+    return r == 0 ? ci * (ny - 1) + cj : r;
 }
 
 }  // namespace rg

@@ -16,40 +16,51 @@ namespace rg {
 int launch_area(const double* x, const double* y, int64_t nx, int64_t ny,
                 double* out, hipStream_t s);
 
-// One lane per point: the secant iteration of the reference.  Points the
-// reference would hand to the exhaustive search are marked for k_cells_brute.
-__global__ void k_cells_secant(const double* __restrict__ x,
-                               const double* __restrict__ y, int64_t nx,
-                               int64_t ny, const double* __restrict__ px,
-                               const double* __restrict__ py, int64_t n,
-                               int64_t* __restrict__ cell)
+constexpr int CELLS_BLOCK = 128;
+
+// One lane per point: the secant iteration of the reference, its cell written
+// as (i, j) or (INT64_MAX, INT64_MAX).  Points the reference would hand to
+// the exhaustive search are marked RG_SEARCH_BRUTE for k_cells_brute: in
+// `mark` (every entry written) when there is one, else in their own row.
+// 2.36 M points in a 1025^2 vertex grid: 228 us reading every vertex where it
+// is used, 154 reading it once (secant_search).
+__global__ __launch_bounds__(CELLS_BLOCK) void k_cells_secant(
+    const double* __restrict__ x, const double* __restrict__ y, int64_t nx, int64_t ny,
+    const double* __restrict__ px, const double* __restrict__ py, int64_t n,
+    int64_t* __restrict__ ij, int64_t* __restrict__ mark)
 {
     const int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (q >= n) return;
-    cell[q] = index_secant(x, y, nx, ny, px[q], py[q]);
+    int64_t ci = INT64_MAX, cj = INT64_MAX;
+    const int64_t r = secant_search(VertexArrays{x, y}, nx, ny, px[q], py[q], &ci, &cj);
+    if (mark) mark[q] = r;
+    ij[2 * q] = !mark && r == RG_SEARCH_BRUTE ? RG_SEARCH_BRUTE : ci;
+    ij[2 * q + 1] = cj;
 }
 
-// One wavefront per point: exhaustive lowest-index search for the points
-// marked RG_SEARCH_BRUTE; then flat index -> (i, j) or (INT64_MAX, INT64_MAX).
-__global__ void k_cells_finish(const double* __restrict__ x,
-                               const double* __restrict__ y, int64_t nx,
-                               int64_t ny, const double* __restrict__ px,
-                               const double* __restrict__ py, int64_t n,
-                               const int64_t* __restrict__ cell,
-                               int64_t* __restrict__ ij)
+// The exhaustive lowest-index search for the marked points, one at a time
+// over a wavefront.  A wavefront looks at `per` points: one while that many
+// wavefronts fill the chip (a marked point costs a pass over the grid), up to
+// 64 of a long list (2.36 M points, none marked: a wavefront each took 217 us,
+// 64 each 6).
+__global__ __launch_bounds__(256) void k_cells_brute(
+    const double* __restrict__ x, const double* __restrict__ y, int64_t nx, int64_t ny,
+    const double* __restrict__ px, const double* __restrict__ py, int64_t n, int per,
+    int64_t* __restrict__ ij, const int64_t* __restrict__ mark)
 {
-    const int64_t q = grid_wave();
+    const int64_t q0 = grid_wave() * per;
     const int lane = threadIdx.x & 63;
-    if (q >= n) return;
-    int64_t c = cell[q];
-    if (c == RG_SEARCH_BRUTE) c = wave_brute(x, y, nx, ny, px[q], py[q], lane);
-    if (lane == 0) {
-        if (c >= 0) {
-            ij[2 * q] = c / (ny - 1);
-            ij[2 * q + 1] = c % (ny - 1);
-        } else {
-            ij[2 * q] = INT64_MAX;
-            ij[2 * q + 1] = INT64_MAX;
+    if (q0 >= n) return;  // uniform
+    const int64_t ql = q0 + lane;
+    uint64_t marked = __ballot(lane < per && ql < n &&
+                               (mark ? mark[ql] : ij[2 * ql]) == RG_SEARCH_BRUTE);
+    while (marked) {  // uniform
+        const int64_t q = q0 + __builtin_ctzll(marked);
+        marked &= marked - 1;
+        const int64_t c = wave_brute(x, y, nx, ny, px[q], py[q], lane);
+        if (lane == 0) {
+            ij[2 * q] = c >= 0 ? c / (ny - 1) : INT64_MAX;
+            ij[2 * q + 1] = c >= 0 ? c % (ny - 1) : INT64_MAX;
         }
     }
 }
@@ -116,15 +127,16 @@ int check_find_cells(const double* x, const double* y, int64_t nx, int64_t ny,
     return RG_OK;
 }
 
-// The two kernels of the cell search; `cell` holds one int64 per point
-// between them (every entry written by the first before the second reads it).
 int launch_find_cells(const double* x, const double* y, int64_t nx, int64_t ny,
                       const double* px, const double* py, int64_t n,
-                      int64_t* cell, int64_t* cell_ij, hipStream_t s)
+                      int64_t* cell_ij, int64_t* mark, hipStream_t s)
 {
-    k_cells_secant<<<grid_for(n, 128), 128, 0, s>>>(x, y, nx, ny, px, py, n, cell);
-    k_cells_finish<<<grid_for(n * 64, 256), 256, 0, s>>>(x, y, nx, ny, px, py, n,
-                                                         cell, cell_ij);
+    k_cells_secant<<<grid_for(n, CELLS_BLOCK), CELLS_BLOCK, 0, s>>>(x, y, nx, ny, px, py, n,
+                                                                    cell_ij, mark);
+    int per = 1;
+    while (per < 64 && n / (2 * per) >= 8192) per *= 2;
+    k_cells_brute<<<grid_for((n + per - 1) / per * 64, 256), 256, 0, s>>>(x, y, nx, ny, px, py, n,
+                                                                          per, cell_ij, mark);
     RG_HIP(hipGetLastError());
     return RG_OK;
 }
@@ -140,7 +152,7 @@ int launch_find_cells(const double* x, const double* y, int64_t nx, int64_t ny,
 // memory.  Its device address is looked up once per device, with that device
 // current, and kept; calls on one GPU share the array, so calls that
 // overlap on one GPU race (issue them on one stream).  Nothing in it needs
-// clearing: the secant kernel writes every entry the finishing kernel reads.
+// clearing: the secant kernel writes every entry the exhaustive one reads.
 static __device__ __align__(256) int64_t scratch[RG_FIND_CELLS_NOALLOC_MAX];
 
 namespace {
@@ -192,10 +204,7 @@ int rg_find_cells_2d(const double* x, const double* y, int64_t nx, int64_t ny,
 {
     if (n == 0) return RG_OK;
     RG_TRY(check_find_cells(x, y, nx, ny, px, py, cell_ij));
-    hipStream_t s = (hipStream_t)stream;
-    DevBuf<int64_t> cell;
-    RG_TRY(cell.alloc(n, s));
-    return launch_find_cells(x, y, nx, ny, px, py, n, cell.p, cell_ij, s);
+    return launch_find_cells(x, y, nx, ny, px, py, n, cell_ij, nullptr, (hipStream_t)stream);
 }
 
 int rg_find_cells_2d_noalloc(const double* x, const double* y, int64_t nx,
@@ -212,8 +221,7 @@ int rg_find_cells_2d_noalloc(const double* x, const double* y, int64_t nx,
                         " points per call; search them in slices");
     int64_t* cell = nullptr;
     RG_TRY(find_cells_scratch(&cell));
-    return launch_find_cells(x, y, nx, ny, px, py, n, cell, cell_ij,
-                             (hipStream_t)stream);
+    return launch_find_cells(x, y, nx, ny, px, py, n, cell_ij, cell, (hipStream_t)stream);
 }
 
 int rg_find_indices_1d(const double* x_input, int64_t m,
