@@ -46,8 +46,8 @@ typedef struct rg_tuning {
     int32_t block;          /* threads per block of the walk kernels (128; a
                                multiple of 64, at most 512) */
     int32_t flags;          /* RG_TUNE_TIMINGS: record per-phase times;
-                               RG_TUNE_GUESS_OUTSIDE, RG_TUNE_ROW_WAVES: test
-                               hooks */
+                               RG_TUNE_GUESS_OUTSIDE, RG_TUNE_ROW_WAVES,
+                               RG_TUNE_REDUCE_GENERAL: test hooks */
     int32_t stage_per_edge; /* triples staged per sweep edge by the counting
                                walk (default: from the expected work, 8 when
                                edges_per_lane is given; 16 edges per lane
@@ -64,6 +64,10 @@ typedef struct rg_tuning {
  * per lane) whatever the row count, where a build with few rows takes one
  * row per wavefront; the result is the same bits. */
 #define RG_TUNE_ROW_WAVES 4
+/* Test hook: every 64-cell group takes the general reduction, which is
+ * otherwise for groups too large, or with keys too wide, to sort in registers;
+ * the result is the same bits, only slower. */
+#define RG_TUNE_REDUCE_GENERAL 8
 
 /* Counters and (optionally) phase times of a build. */
 typedef struct rg_build_stats {

@@ -6,13 +6,13 @@
 //   start     chunk 0 of every row: the reference's row start (wavefront per
 //             row); chunk c > 0: a guessed start from the cell search
 //   count     every chunk walks, counts its triples, records its end state,
-//             adds its triples to the (input cell, pass) histogram and stages
+//             adds its triples to the (cell group, pass) histogram and stages
 //             up to `cap` (cin, cout, term) triples per walk thread
 //   fixup     per row: chunks whose start differs from the predecessor's end
 //             are walked again from the true state (histogram corrected,
 //             staging rewritten)
 //   emit      scans give each chunk its first emission ordinal and each
-//             (cell, pass) its bucket; staged triples are scattered into the
+//             (group, pass) its bucket; staged triples are scattered into the
 //             buckets as (out << 32 | ordinal, term) records; chunks whose
 //             triples overflowed the staging walk a third time
 //   reduce    per group of 64 input cells (in LDS): divide by the input cell
@@ -36,17 +36,19 @@ namespace rg {
 
 // ---- atomics usable from the shared walk code ----------------------------
 
-// Triples are bucketed by sweep pass and by group of 64 consecutive input
-// cells (every pair's cell space is padded to a multiple of 64, so a group
-// belongs to one pair), pass-major: bucket (pass p, group g) at slot
-// p * G + g (G groups in all).  The histogram of buckets is small enough to
-// stay in cache, a walk's consecutive triples mostly fall in one bucket, and
-// the scatter claims whole runs of records per bucket.  Each record carries
-// its cell within the group in a side array of bytes; the reduction splits
-// the group by cell.
+// Triples are bucketed by group of 64 consecutive input cells (every pair's
+// cell space is padded to a multiple of 64, so a group belongs to one pair)
+// and by sweep pass, group-major: bucket 4 g + p, so that a group's records
+// are one range.  (One bucket per group would do for the reduction; but then
+// the four passes of a small build's walk contend for its few counters: 57 ->
+// 81 us for a 67 x 190 -> 81 x 125 vertex pair, its scatter 22 -> 36.)  The
+// histogram of buckets is small enough to stay in cache, a walk's consecutive
+// triples mostly fall in one bucket, and the scatter claims whole runs of
+// records per bucket.  Each record carries its cell within the group in a side
+// array of bytes; the reduction splits the group by cell.
 
 // Histogram increments are combined in registers: a walk's consecutive
-// triples mostly fall in one or two (cell, pass) buckets (the static cell of
+// triples mostly fall in one or two buckets (the static cell of
 // a sweep over the output grid; the left and right cells of an input edge),
 // so two pending (bucket, count) entries replace most atomics.
 struct HistCache {
@@ -85,9 +87,7 @@ struct StageSink {
     int32_t n;
     int64_t g, cap;
     Triple* __restrict__ stage;
-    int32_t* __restrict__ hist;
-    int32_t p;
-    int64_t ps;  // bucket (pass p, cell c) is hist[p * ps + (c >> 6)]
+    int32_t* __restrict__ hist;  // of the pass: the bucket of cell c is hist[4 (c >> 6)]
     HistCache hc;
     __device__ void emit(int64_t cin, int64_t cout, double a)
     {
@@ -101,19 +101,17 @@ struct StageSink {
                                         (u32x4*)&stage[stage_index(g, n, cap)]);
         }
         n++;
-        hc.add(hist, (int32_t)(p * ps + (cin >> 6)), 1);
+        hc.add(hist, (int32_t)(4 * (cin >> 6)), 1);
     }
     __device__ void flush() { hc.flush(hist); }
 };
 
 struct UncountSink {
     int32_t* hist;
-    int32_t p;
-    int64_t ps;
     HistCache hc;
     __device__ void emit(int64_t cin, int64_t, double)
     {
-        hc.add(hist, (int32_t)(p * ps + (cin >> 6)), -1);
+        hc.add(hist, (int32_t)(4 * (cin >> 6)), -1);
     }
     __device__ void flush() { hc.flush(hist); }
 };
@@ -608,7 +606,7 @@ __device__ inline void chunk_range(const Pass& P, int64_t c, int64_t* k0, int64_
 
 __global__ __launch_bounds__(WALK_MAX_BLOCK) void k_walk_count(const Build* __restrict__ builds,
                              const int32_t* __restrict__ pair_of_wave,
-                             int64_t nthreads_all, int64_t ngroups_all,
+                             int64_t nthreads_all,
                              const int32_t* __restrict__ start,
                              int32_t* __restrict__ end,
                              int32_t* __restrict__ count,
@@ -624,7 +622,7 @@ __global__ __launch_bounds__(WALK_MAX_BLOCK) void k_walk_count(const Build* __re
     const int64_t g = B.chunk_gbase + r.g;
     int64_t k0, k1;
     chunk_range(P, r.c, &k0, &k1);
-    StageSink sink{0, t, cap, stage, hist + (B.cell_gbase >> 6), r.p, ngroups_all, {}};
+    StageSink sink{0, t, cap, stage, hist + 4 * (B.cell_gbase >> 6) + r.p, {}};
     end[g] = walk_chunk(B, P, r.row, k0, k1, start[g], sink);
     sink.flush();
     count[g] = sink.n;
@@ -636,7 +634,7 @@ __global__ __launch_bounds__(WALK_MAX_BLOCK) void k_walk_count(const Build* __re
 // chunk order (a fix can change the end state the next link compares with).
 __global__ __launch_bounds__(WALK_MAX_BLOCK) void k_fixup(const Build* __restrict__ builds,
                         const int32_t* __restrict__ pair_of_row,
-                        int64_t nrows_all, int64_t ngroups_all,
+                        int64_t nrows_all,
                         int32_t* __restrict__ start,
                         int32_t* __restrict__ end, int32_t* __restrict__ count,
                         int32_t* __restrict__ hist_all, int32_t* __restrict__ nfix,
@@ -658,7 +656,7 @@ __global__ __launch_bounds__(WALK_MAX_BLOCK) void k_fixup(const Build* __restric
         if (c >= 1 && start[g0 + c] != end[g0 + c - 1]) bad = true;
     }
     if (__ballot(bad) == 0 || lane != 0) return;
-    int32_t* hist = hist_all + (B.cell_gbase >> 6);
+    int32_t* hist = hist_all + 4 * (B.cell_gbase >> 6) + p;
     int32_t fixes = 0;
     for (int64_t c = 1; c < P.cpr; c++) {
         const int64_t g = g0 + c;
@@ -667,11 +665,11 @@ __global__ __launch_bounds__(WALK_MAX_BLOCK) void k_fixup(const Build* __restric
         if (start[g] == truth) continue;
         int64_t k0, k1;
         chunk_range(P, c, &k0, &k1);
-        UncountSink undo{hist, p, ngroups_all, {}};
+        UncountSink undo{hist, {}};
         (void)walk_chunk(B, P, row, k0, k1, start[g], undo);
         undo.flush();
         StageSink redo{0, B.thread_gbase + thread_of_chunk(P, row, c), cap, stage,
-                       hist, p, ngroups_all, {}};
+                       hist, {}};
         end[g] = walk_chunk(B, P, row, k0, k1, truth, redo);
         redo.flush();
         count[g] = redo.n;
@@ -782,7 +780,7 @@ struct ScatTable {
 
 __global__ __launch_bounds__(WALK_MAX_BLOCK) void k_scatter(const Build* __restrict__ builds,
                           const int32_t* __restrict__ pair_of_wave,
-                          int64_t nthreads_all, int64_t ngroups_all,
+                          int64_t nthreads_all,
                           const int32_t* __restrict__ count,
                           const Triple* __restrict__ stage, int64_t cap,
                           const Triple* __restrict__ ovbuf,
@@ -801,8 +799,8 @@ __global__ __launch_bounds__(WALK_MAX_BLOCK) void k_scatter(const Build* __restr
     const Build& B = build_of_thread(builds, pair_of_wave, t);
     const ChunkRef r = chunk_of_thread(B, t - B.thread_gbase);
     const int64_t g = B.chunk_gbase + r.g;
-    // every lane of the wave sweeps one pass: the bucket row is wave-uniform
-    uint32_t* cursor = cursor_all + (B.cell_gbase >> 6) + (int64_t)r.p * ngroups_all;
+    // the pass's cursors: every lane of the wave sweeps one pass
+    uint32_t* cursor = cursor_all + 4 * (B.cell_gbase >> 6) + r.p;
     int32_t n = r.valid ? count[g] : 0;
     const uint32_t ord = r.valid ? (uint32_t)chunk_off[g] : 0;
     const Triple* ov = n > cap ? ovbuf + ov_off[g] : nullptr;
@@ -864,7 +862,7 @@ __global__ __launch_bounds__(WALK_MAX_BLOCK) void k_scatter(const Build* __restr
             const int h = lane * (SCAT_HT / 64) + u;
             c4[u] = H.key[h] >= 0 ? H.cnt[h] : 0;
             b4[u] = 0;
-            if (c4[u] > 0) b4[u] = atomicAdd(&cursor[H.key[h]], (uint32_t)c4[u]);
+            if (c4[u] > 0) b4[u] = atomicAdd(&cursor[4 * H.key[h]], (uint32_t)c4[u]);
             sum += c4[u];
         }
         int32_t o = wave_exclusive(sum, lane);
@@ -886,7 +884,7 @@ __global__ __launch_bounds__(WALK_MAX_BLOCK) void k_scatter(const Build* __restr
                 H.rslot[i] = (uint8_t)slot[k];
                 H.rc[i] = (uint8_t)(e[k].cin & 63);
             } else {
-                const uint32_t pos = atomicAdd(&cursor[e[k].cin >> 6], 1u);
+                const uint32_t pos = atomicAdd(&cursor[4 * (e[k].cin >> 6)], 1u);
                 if (pos < n_rec)
                     put_record(rec, rcell, pos, e[k].cin, e[k].cout, ord + (uint32_t)(q0 + k),
                                e[k].a);
@@ -923,73 +921,19 @@ __global__ __launch_bounds__(WALK_MAX_BLOCK) void k_scatter(const Build* __restr
 // ---- reduce and CSR ------------------------------------------------------
 
 // Coalescing, one wavefront per group of 64 consecutive input cells.  The
-// group's records sit in four pass ranges (the buckets are pass-major), in
-// claim order, each with its cell byte.  The wave counts them per cell in
-// LDS (the cell-major offsets of the group's output, written to cell_off),
-// places them cell-major in LDS, and each lane divides its cell's terms by
-// the cell area, sorts them and reduces equal outputs (bucket_reduce); the
-// wave writes the group's unique (out, weight) pairs packed, in row order,
-// from the group's first offset.  A group beyond the LDS share is first
-// copied cell-major into `red` (global), then goes through LDS in runs of
-// consecutive cells, each cell reduced in place at its own offset (the
-// group is then marked unpacked); a single cell beyond the share is left to
-// k_bucket_long.
+// group's records sit together, in claim order, each with its cell byte.
+// k_reduce_cells sorts and reduces
+// each cell on one lane's registers and writes the group's unique (out,
+// weight) pairs packed, in row order, from the group's first offset.  What its
+// instances do not take (a cell of more than 64 records, a pair of more than
+// 8, keys too wide to sort as doubles) goes to k_reduce_heavy, which takes
+// the group in LDS-sized runs of consecutive cells, each packed at its run's
+// start (the group is then marked unpacked); a single cell beyond the LDS
+// share is left to k_bucket_long.
 // Bits of the flag word (counters[8]) of a capacity-mode build (graph
 // capture): which fixed capacity the data exceeded, or that the build failed.
 constexpr int32_t CAP_TRIPLES = 1, CAP_OVERFLOW = 2, CAP_WEIGHTS = 4, CAP_FAILED = 8,
                   CAP_MISMATCH = 16;
-
-// wavefronts per block: one, so that the blocks pack the LDS more finely (a
-// block's 16.6 KiB per wavefront: nine wavefronts per CU instead of eight
-// in blocks of two; 0.547 -> 0.511 ms at 2049^2 -> 1537^2, the 256-pair
-// batch's reduce phase 7.31 -> 7.11 ms)
-constexpr int RED_WAVES = 1;
-constexpr int HEAVY_WAVES = 2;  // k_reduce_heavy's
-constexpr int RED_CAP = 1024;    // LDS entries per wavefront (16 KiB)
-constexpr int RED_NET = 16;      // largest cell sorted in registers
-// the lane-strided layout of a group whose cells all fit RED_NET entries
-// puts entry j of cell c at j * 64 + c: RED_NET rows of 64 must fit
-static_assert(RED_CAP >= RED_NET * 64, "the lane-strided layout needs RED_NET * 64 entries");
-
-// One cell's terms: divided by the cell area (and weighted), sorted by key
-// in registers through a network of N, written back in place.
-template <int N, int ST = 1>
-__device__ inline void sort_cell_in_registers(uint64_t* K, double* V, int32_t n, double vol,
-                                              const double* wi, int64_t i)
-{
-    uint64_t k[N];
-    double v[N];
-#pragma unroll
-    for (int j = 0; j < N; j++) {
-        k[j] = ~(uint64_t)0;  // padding sorts last
-        v[j] = 0;
-        if (j < n) {
-            k[j] = K[j * ST];
-            v[j] = weight_of(V[j * ST], vol, wi, i);
-        }
-    }
-    sort_network<N, uint64_t>(k, v);
-#pragma unroll
-    for (int j = 0; j < N; j++)
-        if (j < n) {
-            K[j * ST] = k[j];
-            V[j * ST] = v[j];
-        }
-}
-
-// Records of one group (all passes): the group totals that give the
-// group-major output offsets.
-__global__ void k_group_counts(const int64_t* __restrict__ bucket_off, int64_t n_groups,
-                               int32_t* __restrict__ cnt)
-{
-    const int64_t g = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (g >= n_groups) return;
-    int64_t t = 0;
-#pragma unroll
-    for (int p = 0; p < 4; p++)
-        t += bucket_off[p * n_groups + g + 1] - bucket_off[p * n_groups + g];
-    cnt[g] = (int32_t)t;
-}
 
 // One reduced entry (output cell `out`, weight) of a group: stored with its
 // arrival rank among the entries of its output row (the high word of the
@@ -1028,203 +972,389 @@ __device__ inline void put_reduced_cell(KV* __restrict__ dst, const uint64_t* K,
     }
 }
 
-// The records of one group, reached through its four pass ranges: their
-// total (the group's count, of which group_off is the exclusive scan) and
-// the end of the last range, which ends last (the records sit pass-major).
-struct GroupRecs {
-    int64_t ps0, ps1, ps2, ps3, e0, e1, e2, total, end;
-    __device__ GroupRecs(const int64_t* __restrict__ bucket_off, int64_t n_groups, int64_t grp)
+// ---- cells sorted in registers ------------------------------------------------
+//
+// A record's key -- output cell, emission ordinal -- and its place in its
+// cell's slots make one integer below 2^61, which, offset by 2^62, is the bit
+// pattern of a positive normal double: such doubles order as the integers do,
+// so a comparator of the sorting network is v_min_f64 and v_max_f64, two
+// instructions where comparing and exchanging 64-bit keys with their values
+// takes eleven.  The values stay behind and are fetched by the sorted keys'
+// slots.
+struct KeyBits {
+    int ord, out;  // widths of the ordinal and of the output cell; 0: they do not fit
+    static constexpr int SLOT = 6;
+    __device__ uint64_t encode(uint64_t key, int slot) const
     {
-        ps0 = bucket_off[grp];
-        ps1 = bucket_off[n_groups + grp];
-        ps2 = bucket_off[2 * n_groups + grp];
-        ps3 = bucket_off[3 * n_groups + grp];
-        e0 = bucket_off[grp + 1] - ps0;
-        e1 = e0 + bucket_off[n_groups + grp + 1] - ps1;
-        e2 = e1 + bucket_off[2 * n_groups + grp + 1] - ps2;
-        end = bucket_off[3 * n_groups + grp + 1];
-        total = e2 + end - ps3;
+        // (a capacity-mode build past its capacity may hold wider ordinals:
+        // cut, so that the output cell stays in range)
+        const uint64_t o = key & (((uint64_t)1 << ord) - 1);
+        return (uint64_t)1 << 62 | ((key >> 32) << ord | o) << SLOT | (uint64_t)slot;
     }
-    // position of record q of the concatenated pass ranges
-    __device__ int64_t src(int64_t q) const
+    __device__ uint32_t output(uint64_t code) const
     {
-        return q < e0 ? ps0 + q : q < e1 ? ps1 + (q - e0) : q < e2 ? ps2 + (q - e1)
-                                                               : ps3 + (q - e2);
+        return (uint32_t)(code >> (ord + SLOT)) & (uint32_t)(((uint64_t)1 << out) - 1);
     }
 };
 
-// Groups whose records fit the LDS share; a larger group is listed for
-// k_reduce_heavy.
-__global__ __launch_bounds__(RED_WAVES * 64) void k_reduce_groups(
-    const int64_t* __restrict__ bucket_off, int64_t n_groups,
-    const int64_t* __restrict__ group_off, const KV* __restrict__ rec,
-    const uint8_t* __restrict__ rcell, KV* __restrict__ red,
-    int64_t* __restrict__ cell_off, const double* __restrict__ vol_in,
-    const double* __restrict__ wi, int32_t* __restrict__ nnz_row,
-    int32_t* __restrict__ group_mode, int32_t* __restrict__ long_list,
-    int32_t* __restrict__ n_long, int32_t* __restrict__ heavy_list,
-    int32_t* __restrict__ n_heavy, const PairCells* __restrict__ pcs,
-    const int32_t* __restrict__ pair_of_group, int32_t* __restrict__ hist_out_all,
-    int64_t red_cap, int32_t* __restrict__ cap_flag)
+// Batcher's odd-even merge sort of N doubles in registers (for N below a
+// power of two, that power's network without the comparators beyond N).
+template <int N>
+__device__ inline void sort_doubles(double* k)
 {
-    __shared__ uint64_t sk[RED_WAVES][RED_CAP];
-    __shared__ double sv[RED_WAVES][RED_CAP];
-    __shared__ int32_t scnt[RED_WAVES][64];
-    const int wid = block_wave(), lane = threadIdx.x & 63;
-    if (blockIdx.x == 0 && threadIdx.x == 0) cell_off[n_groups * 64] = group_off[n_groups];
-    const int64_t grp = (int64_t)blockIdx.x * RED_WAVES + wid;
-    if (grp >= n_groups) return;  // uniform per wavefront; no block barriers below
-    // requested first, with the group's offsets: the cell areas and the
-    // pair's output-cell base, which the records do not decide
-    const double vol = vol_in[grp * 64 + lane];
+#pragma unroll
+    for (int p = 1; p < N; p <<= 1) {
+#pragma unroll
+        for (int q = p; q > 0; q >>= 1) {
+#pragma unroll
+            for (int j = q % p; j + q < N; j += 2 * q) {
+#pragma unroll
+                for (int i = 0; i < q; i++) {
+                    const int a = i + j, b = i + j + q;
+                    if (b < N && a / (2 * p) == b / (2 * p)) {
+                        const double lo = fmin(k[a], k[b]);
+                        k[b] = fmax(k[a], k[b]);
+                        k[a] = lo;
+                    }
+                }
+            }
+        }
+    }
+}
+
+// One group's slots: entry d of cell c at d * 64 + c, so the lanes (one per
+// cell) touch consecutive words at every step.  Keys first, then values.  Row
+// N and the upper counters take what the lanes past the last record write:
+// every step is the same instructions for all lanes, so the steps of several
+// records overlap (a branch per record made each wait for its own LDS reads
+// and division).
+template <int N>
+struct CellSlots {
+    double slot[(N + 1) * 64];
+    double vol[64], wt[64];
+    int32_t cnt[128];
+};
+
+// What both the group kernels and the code below need of a build.
+struct RedArgs {
+    const int64_t* bucket_off;  // first record of group g at 4 g (4 n_groups + 1)
+    const KV* rec;
+    const uint8_t* rcell;
+    KV* red;
+    int64_t* cell_off;
+    const double* vol;
+    const double* wi;
+    int32_t* nnz_row;
+    int32_t* group_mode;
+    const PairCells* pcs;
+    const int32_t* pair_of_group;
+    int32_t* hist_out;
+    KeyBits bits;
+};
+
+// The cells of one group, at most M records each: sorted, reduced and
+// written.  The slots hold the keys; values() writes the weighted terms over
+// them.  Class 3, with nothing written, if a run is too long for a sequential
+// sum (numpy's pairwise order from 8 further terms on) or the group has more
+// unique pairs than the slots take packed.
+//
+// The unique pairs are packed in LDS before they are written, and each lane
+// asks for the rank of one of them in its output row: neighbours in that
+// order are neighbours in the output grid, so a wavefront's atomics fall in
+// few lines.  (They are carried out at the memory, 27 G lines/s for returning
+// ones at random addresses; asked for cell by cell from the registers, one
+// line each, they took 290 us of the reduction's 750 at 2049^2 -> 1537^2.)
+template <int M, int N, class Values>
+__device__ inline int reduce_sorted(const RedArgs& A, double* __restrict__ slot, int64_t grp,
+                                    int64_t base, int32_t* __restrict__ hist_out, int n,
+                                    const Values& values)
+{
+    const int lane = threadIdx.x & 63;
+    double k[M];
+#pragma unroll
+    for (int j = 0; j < M; j++)
+        k[j] = j < n ? slot[j * 64 + lane] : __builtin_bit_cast(double, 0x7fe0000000000000ull);
+    sort_doubles<M>(k);
+    // the first record of each run of one output; from here on a record is
+    // its output and its slot
+    uint64_t heads = 0;
+    uint32_t out[M];
+    uint8_t from[M];
+#pragma unroll
+    for (int j = 0; j < M; j++) {
+        const uint64_t c = __builtin_bit_cast(uint64_t, k[j]);
+        out[j] = A.bits.output(c);
+        from[j] = (uint8_t)(c & 63);  // (0 past the cell's last)
+        if (j < n && (j == 0 || out[j] != out[j > 0 ? j - 1 : 0])) heads |= (uint64_t)1 << j;
+    }
+    uint64_t more = ~heads & (n < 64 ? ((uint64_t)1 << n) - 1 : ~(uint64_t)0);
+    more &= more >> 1;
+    more &= more >> 2;
+    more &= more >> 4;
+    const int m = __popcll(heads);
+    const int dst = wave_exclusive(m, lane);
+    const int pairs = __builtin_amdgcn_readlane(dst + m, 63);
+    constexpr int room = (N + 1) * 64 * 8 / 12;  // packed pairs the slots take
+    if (__ballot(more != 0) || pairs > room) return 3;  // uniform
+    wave_sync_lds();  // every lane has its keys: the slots take the values
+    values();
+    wave_sync_lds();
+    double v[M];
+#pragma unroll
+    for (int j = 0; j < M; j++) v[j] = slot[(int)from[j] * 64 + lane];
+    wave_sync_lds();  // every lane has its values: the slots take the pairs
+    // each run: its first term plus the sum of the others from -0.0
+    double* const pv = slot;
+    uint32_t* const po = reinterpret_cast<uint32_t*>(slot + room);
+    int at = dst - 1;
+    double first = 0, rest = -0.0;
+    bool one = true;
+#pragma unroll
+    for (int j = 0; j < M; j++) {
+        const bool head = heads >> j & 1;
+        if (head) {
+            if (j > 0) pv[at] = one ? first : first + rest;
+            po[++at] = out[j];
+        }
+        first = head ? v[j] : first;
+        rest = head ? -0.0 : (j < n ? rest + v[j] : rest);
+        one = head || (one && j >= n);
+    }
+    if (n > 0) pv[at] = one ? first : first + rest;
+    wave_sync_lds();
+    for (int e = lane; e < pairs; e += 64) {
+        const uint32_t o = po[e];
+        KV r;
+        r.key = (uint64_t)o | (uint64_t)(uint32_t)atomicAdd(&hist_out[o], 1) << 32;
+        r.val = pv[e];
+        A.red[base + e] = r;
+    }
+    const int64_t i = grp * 64 + lane;
+    A.nnz_row[i] = m;
+    if (lane == 0) A.group_mode[grp] = 0;
+    return 0;
+}
+
+// The instance a group takes, by its records and its largest cell: 0
+// (k_reduce_cells), 1 and 2 (k_reduce_listed), 3 (k_reduce_heavy).
+constexpr int CELLS_U = 16, CELLS_N = 24, LIST1_U = 24, LIST1_N = 32, LIST2_U = 48, LIST2_N = 64;
+
+__device__ inline int group_class(int64_t total, int nmax)
+{
+    return total <= CELLS_U * 64 && nmax <= CELLS_N   ? 0
+           : total <= LIST1_U * 64 && nmax <= LIST1_N ? 1
+           : total <= LIST2_U * 64 && nmax <= LIST2_N ? 2
+                                                      : 3;
+}
+
+__device__ inline int wave_max(int v)
+{
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o, 64));
+    return v;
+}
+
+// One group of at most U * 64 records and N per cell: 0, or with nothing but
+// cell offsets written the class it takes instead.  All records are requested
+// together, U per lane, and their values wait in registers.
+template <int U, int N>
+__device__ inline int reduce_group(const RedArgs& A, CellSlots<N>& S, int64_t grp)
+{
+    const int lane = threadIdx.x & 63;
+    const int64_t i = grp * 64 + lane;
+    // requested first, with the group's offsets: what the records do not decide
+    const double vol = A.vol[i], wt = A.wi ? A.wi[i] : 1.0;
     int32_t* const hist_out =
-        hist_out_all + pcs[__builtin_amdgcn_readfirstlane(pair_of_group[grp])].out_gbase;
-    // every offset of the group takes part in the first test, so they are
-    // requested together (a load first used after a test is not issued
-    // before it: one round trip per test)
-    const int64_t base = group_off[grp];
-    const GroupRecs G(bucket_off, n_groups, grp);
-    const int64_t total = G.total;
-    if (base + total > red_cap || G.end > red_cap) {
+        A.hist_out + A.pcs[__builtin_amdgcn_readfirstlane(A.pair_of_group[grp])].out_gbase;
+    const int64_t base = A.bucket_off[4 * grp];
+    const int total = (int)(A.bucket_off[4 * grp + 4] - base);
+    if (total == 0) {  // uniform
+        A.cell_off[i] = base;
+        A.nnz_row[i] = 0;
+        if (lane == 0) A.group_mode[grp] = 0;
+        return 0;
+    }
+    S.cnt[lane] = 0;
+    S.vol[lane] = vol;
+    S.wt[lane] = wt;
+    wave_sync_lds();
+    // (a lane past the last record reads the last one)
+    const KV* const rec = A.rec + base;
+    const uint8_t* const rcell = A.rcell + base;
+    const auto src = [&](int u) {
+        const int q = lane + 64 * u;
+        return (uint32_t)(q < total ? q : total - 1);
+    };
+    // the records' cells, counted; the count's returning atomic gives each
+    // record its slot
+    int place[U];
+    KV rr[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) place[u] = rcell[src(u)];
+    // (read once, with nontemporal loads: through the caches the records evict
+    // what the groups in flight re-read)
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+#pragma unroll
+    for (int u = 0; u < U; u++)
+        rr[u] = __builtin_bit_cast(KV,
+                                   __builtin_nontemporal_load((const u32x4*)&rec[src(u)]));
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        const bool is = lane + 64 * u < total;
+        const int c = is ? place[u] : lane;
+        const int d = atomicAdd(&S.cnt[is ? c : 64 + lane], 1);
+        place[u] = c | (is ? d : N) << 6;
+    }
+    wave_sync_lds();
+    const int n = S.cnt[lane];
+    const int nmax = wave_max(n);
+    if (nmax > N) return group_class(total, nmax);  // uniform
+    A.cell_off[i] = base + wave_exclusive(n, lane);
+#pragma unroll
+    for (int u = 0; u < U; u++)
+        S.slot[place[u]] = __builtin_bit_cast(double, A.bits.encode(rr[u].key, place[u] >> 6));
+    wave_sync_lds();
+    const auto values = [&] {
+#pragma unroll
+        for (int u0 = 0; u0 < U; u0 += 2) {  // two divisions at a time (registers)
+            double a[2];
+#pragma unroll
+            for (int u = 0; u < 2; u++) a[u] = rr[u0 + u].val / S.vol[place[u0 + u] & 63];
+            if (A.wi) {
+#pragma unroll
+                for (int u = 0; u < 2; u++) a[u] *= S.wt[place[u0 + u] & 63];
+            }
+#pragma unroll
+            for (int u = 0; u < 2; u++) S.slot[place[u0 + u]] = a[u];
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+#define RG_SORTED(M) reduce_sorted<M, N>(A, S.slot, grp, base, hist_out, n, values)
+    if constexpr (N <= 24) {
+        if (nmax <= 8) return RG_SORTED(8);
+        if (nmax <= 16) return RG_SORTED(16);
+        return RG_SORTED(24);
+    } else if constexpr (N <= 32) {
+        if (nmax <= 24) return RG_SORTED(24);
+        return RG_SORTED(32);
+    } else {
+        if (nmax <= 32) return RG_SORTED(32);
+        if (nmax <= 48) return RG_SORTED(48);
+        return RG_SORTED(64);
+    }
+#undef RG_SORTED
+}
+
+// The first pass over all groups, a wavefront each: up to 1024 records and 24
+// per cell (14.3 KiB of LDS: eleven wavefronts per CU).  The class of any
+// other group is left in group_mode (negative) for k_list_groups.
+//
+// The classes follow the sizes the grids' ratio gives: 12 to 15 records a cell
+// (at most 20 to 24) where the output cells are a little larger than the input
+// cells, 18 (28) at equal sizes, 38 (60) at half the size.  With ranking by
+// counting smaller keys beyond 16 records a cell, and a list and a work queue
+// appended to and read by single atomics, the reduction took 1272 us at
+// 2049^2 -> 1537^2 with the grids 0.5 rad apart and 632 at 0.2 rad; now 518
+// and 387; 64 mixed pairs of 33 to 1025 vertices an axis 2036 -> 1109 us.
+// What is left: the records (17 bytes a triple: 0.83 GB, 130 us at the rate
+// plain loads of this form reach) and the ranks' atomics.
+__global__ __launch_bounds__(64, 3) void k_reduce_cells(RedArgs A, int64_t n_groups,
+                                                      int64_t red_cap,
+                                                      int32_t* __restrict__ cap_flag)
+{
+    __shared__ CellSlots<CELLS_N> S;
+    const int lane = threadIdx.x & 63;
+    const int64_t grp = blockIdx.x;
+    const int64_t base = A.bucket_off[4 * grp], end = A.bucket_off[4 * grp + 4];
+    if (grp == 0 && lane == 0) A.cell_off[n_groups * 64] = A.bucket_off[4 * n_groups];
+    if (end > red_cap) {
         // past the records a capacity-mode build holds: nothing of it is kept
-        nnz_row[grp * 64 + lane] = 0;
-        cell_off[grp * 64 + lane] = 0;
+        A.nnz_row[grp * 64 + lane] = 0;
+        A.cell_off[grp * 64 + lane] = 0;
         if (lane == 0) {
-            group_mode[grp] = 0;
+            A.group_mode[grp] = 0;
             atomicOr(cap_flag, CAP_TRIPLES);
         }
         return;
     }
-    if (total > RED_CAP) {
-        if (lane == 0) heavy_list[atomicAdd(n_heavy, 1)] = (int32_t)grp;
-        return;
-    }
-    const int64_t i = grp * 64 + lane;
-    int32_t* C = scnt[wid];
-    // the records are read once, into registers (record q = lane + 64 u of
-    // the concatenated pass ranges), with nontemporal loads: nothing reads
-    // them again, and through the caches they would evict the cell bytes
-    // and offsets of the groups in flight (0.518 -> 0.503 ms at 2049^2 ->
-    // 1537^2)
-    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-    KV rr[RED_CAP / 64];
-    int32_t cc[RED_CAP / 64];
-    C[lane] = 0;
-    wave_sync_lds();
-#pragma unroll
-    for (int u = 0; u < RED_CAP / 64; u++) {
-        const int64_t q = lane + 64 * u;
-        cc[u] = -1;
-        if (q < total) {
-            const int64_t src = G.src(q);
-            cc[u] = rcell[src];
-            rr[u] = __builtin_bit_cast(KV, __builtin_nontemporal_load((const u32x4*)&rec[src]));
-        }
-    }
-    // (the count's returning atomic also gives each record its place in its
-    // cell, used by both layouts below)
-    int32_t dd[RED_CAP / 64];
-#pragma unroll
-    for (int u = 0; u < RED_CAP / 64; u++) dd[u] = cc[u] >= 0 ? atomicAdd(&C[cc[u]], 1) : 0;
-    wave_sync_lds();
-    // records per cell, and the cell-major offsets
-    const int32_t n = C[lane];
-    const int32_t s = wave_exclusive(n, lane);
-    cell_off[i] = base + s;
-    uint64_t* K = sk[wid];
-    double* V = sv[wid];
-    int32_t nmax = n;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) nmax = max(nmax, __shfl_xor(nmax, o, 64));
-    if (nmax <= RED_NET) {
-        // every cell fits RED_NET entries: entry j of cell c sits at
-        // j * 64 + c, so the lanes (one per cell) touch consecutive LDS
-        // words at every step of the sort and the reduction
-#pragma unroll
-        for (int u = 0; u < RED_CAP / 64; u++)
-            if (cc[u] >= 0) {
-                K[dd[u] * 64 + cc[u]] = rr[u].key;
-                V[dd[u] * 64 + cc[u]] = rr[u].val;
-            }
-        wave_sync_lds();
-        if (nmax <= RED_NET / 2)
-            sort_cell_in_registers<RED_NET / 2, 64>(K + lane, V + lane, n, vol, wi, i);
-        else
-            sort_cell_in_registers<RED_NET, 64>(K + lane, V + lane, n, vol, wi, i);
-        bool lr1 = false;  // (a run of at most RED_NET terms is never long)
-        const int64_t m1 = bucket_reduce_sorted(K + lane, V + lane, n, &lr1, 64);
-        const int64_t dst1 = wave_exclusive((int32_t)m1, lane);
-        put_reduced_cell(red + base + dst1, K + lane, V + lane, m1, hist_out, 64);
-        nnz_row[i] = (int32_t)m1;
-        if (lane == 0) group_mode[grp] = 0;
-        return;
-    }
-    wave_sync_lds();
-    // the keys cell-major in LDS; then every record's place in its cell is
-    // the number of smaller keys of its cell (the keys are unique: they hold
-    // the emission ordinal), and the records are written there, weighted
-#pragma unroll
-    for (int u = 0; u < RED_CAP / 64; u++) {
-        const int32_t cs = __shfl(s, cc[u] >= 0 ? cc[u] : lane, 64);
-        if (cc[u] >= 0) K[cs + dd[u]] = rr[u].key;
-    }
-    wave_sync_lds();
-    int32_t pos[RED_CAP / 64];
-#pragma unroll
-    for (int u = 0; u < RED_CAP / 64; u++) {
-        const int32_t ce = cc[u] >= 0 ? cc[u] : lane;
-        const int32_t cs = __shfl(s, ce, 64), cn = __shfl(n, ce, 64);
-        pos[u] = -1;
-        if (cc[u] >= 0) {
-            const uint64_t k = rr[u].key;
-            // four keys requested before any is compared
-            int32_t r = 0, j = cs;
-            const int32_t je = cs + cn;
-            for (; j + 4 <= je; j += 4) {
-                const uint64_t k0 = K[j], k1 = K[j + 1], k2 = K[j + 2], k3 = K[j + 3];
-                r += (k0 < k ? 1 : 0) + (k1 < k ? 1 : 0) + (k2 < k ? 1 : 0) + (k3 < k ? 1 : 0);
-            }
-            for (; j < je; j++) r += K[j] < k ? 1 : 0;
-            pos[u] = cs + r;
-        }
-    }
-    wave_sync_lds();
-#pragma unroll
-    for (int u = 0; u < RED_CAP / 64; u++) {
-        const int32_t ce = cc[u] >= 0 ? cc[u] : lane;
-        const double cv = __shfl(vol, ce, 64);
-        if (pos[u] >= 0) {
-            K[pos[u]] = rr[u].key;
-            V[pos[u]] = weight_of(rr[u].val, cv, wi, grp * 64 + ce);
-        }
-    }
-    wave_sync_lds();
-    bool lr = false;
-    int64_t m = bucket_reduce_sorted(K + s, V + s, n, &lr);
-    if (lr) m = n;  // left sorted, uncompacted, for k_bucket_long
-    const bool packed = __ballot(lr) == 0;
-    // packed destination: exclusive prefix of m over the wave; a group
-    // with a long run keeps the cell starts
-    const int64_t dst = packed ? wave_exclusive((int32_t)m, lane) : s;
-    if (lr) {
-        for (int64_t t = 0; t < m; t++) {  // finished by k_bucket_long
-            KV r;
-            r.key = K[s + t];
-            r.val = V[s + t];
-            red[base + dst + t] = r;
-        }
+    int cls = 3;
+    if (A.bits.out == 0 || end - base > LIST2_U * 64) {
+    } else if (end - base <= CELLS_U * 64) {
+        cls = reduce_group<CELLS_U, CELLS_N>(A, S, grp);
     } else {
-        put_reduced_cell(red + base + dst, K + s, V + s, m, hist_out);
+        const int total = (int)(end - base);
+        const uint8_t* const rcell = A.rcell + base;
+        S.cnt[lane] = 0;
+        wave_sync_lds();
+        for (int q0 = lane; q0 - lane < total; q0 += 64 * 16) {
+            int c[16];
+#pragma unroll
+            for (int u = 0; u < 16; u++)
+                c[u] = rcell[q0 + 64 * u < total ? q0 + 64 * u : total - 1];
+#pragma unroll
+            for (int u = 0; u < 16; u++)
+                atomicAdd(&S.cnt[q0 + 64 * u < total ? c[u] : 64 + lane], 1);
+        }
+        wave_sync_lds();
+        cls = group_class(total, wave_max(S.cnt[lane]));
     }
-    nnz_row[i] = (int32_t)m;
-    if (lr) long_list[atomicAdd(n_long, 1)] = (int32_t)i;
-    if (lane == 0) group_mode[grp] = packed ? 0 : 1;
+    if (cls && lane == 0) A.group_mode[grp] = -cls;
 }
 
-// Groups beyond the LDS share, one wavefront each.  The waves are resident
-// and pull the next group of the list from a counter (a work queue: the
-// heavy groups differ in size by orders of magnitude, so a fixed
-// assignment leaves waves idle behind the one that drew the largest).  The
+// The groups of each class, listed: one atomic per block and class.  (All
+// atomics on one word are carried out one after another, about 12 ns each:
+// appended by their own wavefronts, and taken one by one from a shared
+// counter, the 30 600 listed groups of the 2049^2 -> 1537^2 pair at a large
+// angle cost 360 us each way; this kernel takes 5.)
+constexpr int LIST_BLOCK = 1024;
+
+__global__ __launch_bounds__(LIST_BLOCK) void k_list_groups(
+    const int32_t* __restrict__ group_mode, int64_t n_groups, int32_t* __restrict__ list1,
+    int32_t* __restrict__ n1, int32_t* __restrict__ list2, int32_t* __restrict__ n2,
+    int32_t* __restrict__ list3, int32_t* __restrict__ n3)
+{
+    __shared__ int32_t cnt[3], at[3];
+    const int64_t grp = blockIdx.x * (int64_t)LIST_BLOCK + threadIdx.x;
+    const int lane = threadIdx.x & 63;
+    if (threadIdx.x < 3) cnt[threadIdx.x] = 0;
+    __syncthreads();
+    const int cls = grp < n_groups ? -group_mode[grp] : 0;
+    int32_t mine = 0;  // place among the block's groups of the same class
+    for (int c = 1; c <= 3; c++) {
+        const uint64_t m = __ballot(cls == c);
+        int32_t w = 0;
+        if (lane == 0 && m) w = atomicAdd(&cnt[c - 1], __popcll(m));
+        w = __shfl(w, 0, 64);
+        if (cls == c) mine = w + __popcll(m & (((uint64_t)1 << lane) - 1));
+    }
+    __syncthreads();
+    if (threadIdx.x < 3 && cnt[threadIdx.x])
+        at[threadIdx.x] =
+            atomicAdd(threadIdx.x == 0 ? n1 : threadIdx.x == 1 ? n2 : n3, cnt[threadIdx.x]);
+    __syncthreads();
+    if (cls == 1) list1[at[0] + mine] = (int32_t)grp;
+    if (cls == 2) list2[at[1] + mine] = (int32_t)grp;
+    if (cls == 3) list3[at[2] + mine] = (int32_t)grp;
+}
+
+// The listed groups of one class, in turn over resident wavefronts.
+template <int U, int N>
+__global__ __launch_bounds__(64, N > 32 ? 1 : 2) void k_reduce_listed(
+    RedArgs A, const int32_t* __restrict__ list, const int32_t* __restrict__ n_list,
+    int32_t* __restrict__ heavy_list, int32_t* __restrict__ n_heavy)
+{
+    __shared__ CellSlots<N> S;
+    const int lane = threadIdx.x & 63;
+    const int32_t nl = *n_list;
+    for (int32_t h = blockIdx.x; h < nl; h += gridDim.x) {
+        const int64_t grp = list[h];
+        if (reduce_group<U, N>(A, S, grp) && lane == 0)  // (a long run: rare)
+            heavy_list[atomicAdd(n_heavy, 1)] = (int32_t)grp;
+        wave_sync_lds();  // LDS reuse by the next group
+    }
+}
+
+// The groups left over, one wavefront each, in turn over resident waves.  The
 // cells' counts give their cell-major offsets in `red` (the group is marked
 // unpacked); the cells are then taken in runs of consecutive cells that fit
 // the LDS share.  For each run the wave places the records of the run's
@@ -1239,8 +1369,9 @@ __global__ __launch_bounds__(RED_WAVES * 64) void k_reduce_groups(
 // HEAVY_UNROLL loads per lane in flight, each record written over its own
 // source slot: two short dependent chains per run instead of one per
 // record.
-constexpr int HEAVY_CAP = RED_CAP;  // LDS entries per wavefront
-constexpr int HEAVY_UNROLL = 4;  // records loaded per lane at once
+constexpr int HEAVY_WAVES = 2;   // wavefronts per block
+constexpr int HEAVY_CAP = 1024;  // LDS entries per wavefront (16 KiB)
+constexpr int HEAVY_UNROLL = 3;  // records loaded per lane at once
 constexpr int HEAVY_SCAN = 8;    // cell bytes requested per lane at once
 // A group's cell bytes are kept in LDS from the counting scan when it has at
 // most this many records (most heavy groups), so the scans of its runs read
@@ -1248,14 +1379,13 @@ constexpr int HEAVY_SCAN = 8;    // cell bytes requested per lane at once
 constexpr int HEAVY_CELLB = 2048;
 
 __global__ __launch_bounds__(HEAVY_WAVES * 64) void k_reduce_heavy(
-    const int64_t* __restrict__ bucket_off, int64_t n_groups,
-    const int64_t* __restrict__ group_off, const KV* __restrict__ rec,
+    const int64_t* __restrict__ bucket_off, const KV* __restrict__ rec,
     const uint8_t* __restrict__ rcell, KV* __restrict__ red,
     int64_t* __restrict__ cell_off, const double* __restrict__ vol_in,
     const double* __restrict__ wi, int32_t* __restrict__ nnz_row,
     int32_t* __restrict__ group_mode, int32_t* __restrict__ long_list,
     int32_t* __restrict__ n_long, const int32_t* __restrict__ heavy_list,
-    const int32_t* __restrict__ n_heavy, int32_t* __restrict__ heavy_next,
+    const int32_t* __restrict__ n_heavy,
     const PairCells* __restrict__ pcs, const int32_t* __restrict__ pair_of_group,
     int32_t* __restrict__ hist_out_all)
 {
@@ -1273,21 +1403,11 @@ __global__ __launch_bounds__(HEAVY_WAVES * 64) void k_reduce_heavy(
     uint8_t* CB = scb[wid];  // the group's cell bytes, by record
     constexpr int U = HEAVY_CAP / 64;
     const int32_t nh = *n_heavy;
-    // the next list position, requested one group ahead
-    int32_t hn = 0;
-    if (lane == 0) hn = atomicAdd(heavy_next, 1);
-    for (;;) {
-        // (all lanes are active here: the first active lane is lane 0, and
-        // the group's tables are then read with scalar loads)
-        const int32_t h = __builtin_amdgcn_readfirstlane(hn);
-        if (h >= nh) break;  // uniform per wavefront
-        if (lane == 0) hn = atomicAdd(heavy_next, 1);
+    for (int32_t h = blockIdx.x * HEAVY_WAVES + wid; h < nh; h += gridDim.x * HEAVY_WAVES) {
         const int64_t grp = heavy_list[h];
         const int64_t i = grp * 64 + lane;
         const double vol = vol_in[i];
-        const int64_t base = group_off[grp];
-        const GroupRecs G(bucket_off, n_groups, grp);
-        const int64_t total = G.total;
+        const int64_t base = bucket_off[4 * grp], total = bucket_off[4 * grp + 4] - base;
         int32_t* hist_out =
             hist_out_all + pcs[__builtin_amdgcn_readfirstlane(pair_of_group[grp])].out_gbase;
         const bool cached = total <= HEAVY_CELLB;
@@ -1297,7 +1417,7 @@ __global__ __launch_bounds__(HEAVY_WAVES * 64) void k_reduce_heavy(
             int32_t cb[HEAVY_SCAN];
 #pragma unroll
             for (int u = 0; u < HEAVY_SCAN; u++)
-                cb[u] = q0 + 64 * u < total ? rcell[G.src(q0 + 64 * u)] : -1;
+                cb[u] = q0 + 64 * u < total ? rcell[base + q0 + 64 * u] : -1;
 #pragma unroll
             for (int u = 0; u < HEAVY_SCAN; u++)
                 if (cb[u] >= 0) {
@@ -1321,9 +1441,8 @@ __global__ __launch_bounds__(HEAVY_WAVES * 64) void k_reduce_heavy(
                 if (lane == 0) C[0] = 0;
                 wave_sync_lds();
                 for (int64_t q = lane; q < total; q += 64) {
-                    const int64_t src = G.src(q);
-                    if ((cached ? CB[q] : rcell[src]) == c)
-                        red[base + sb + atomicAdd(&C[0], 1)] = rec[src];
+                    if ((cached ? CB[q] : rcell[base + q]) == c)
+                        red[base + sb + atomicAdd(&C[0], 1)] = rec[base + q];
                 }
                 if (lane == c) {  // (k_bucket_long takes the cell's size from nnz_row)
                     nnz_row[i] = n;
@@ -1343,13 +1462,13 @@ __global__ __launch_bounds__(HEAVY_WAVES * 64) void k_reduce_heavy(
 #pragma unroll
                 for (int u = 0; u < HEAVY_SCAN; u++) {
                     const int64_t q = q0 + 64 * u;
-                    cb[u] = q < total ? (cached ? CB[q] : rcell[G.src(q)]) : -1;
+                    cb[u] = q < total ? (cached ? CB[q] : rcell[base + q]) : -1;
                 }
 #pragma unroll
                 for (int u = 0; u < HEAVY_SCAN; u++)
                     if (cb[u] >= c && cb[u] < d) {
                         const int32_t p = atomicAdd(&C[cb[u]], 1);
-                        SRC[p] = G.src(q0 + 64 * u);
+                        SRC[p] = base + q0 + 64 * u;
                         SC[p] = (uint8_t)cb[u];
                     }
             }
@@ -1399,6 +1518,7 @@ __global__ __launch_bounds__(HEAVY_WAVES * 64) void k_reduce_heavy(
                     ve[u] = weight_of(V[e], cv, wi, grp * 64 + ce);
                     pe[u] = cs + r;
                 }
+                __builtin_amdgcn_sched_barrier(0);  // (one record's at a time: registers)
             }
             wave_sync_lds();
 #pragma unroll
@@ -1712,6 +1832,20 @@ int fill_zero(int32_t* p, int64_t n, hipStream_t s)
                  s>>>(p, 0, n);
     RG_HIP(hipGetLastError());
     return RG_OK;
+}
+
+// The widths of the reduction's keys for T triples and `most_out` output
+// cells of a pair; none if they and a slot exceed the 61 bits there are.
+KeyBits key_bits(int64_t T, int64_t most_out)
+{
+    const auto width = [](int64_t values) {  // bits of 0 .. values - 1, at least one
+        int b = 1;
+        while (b < 63 && ((int64_t)1 << b) < values) b++;
+        return b;
+    };
+    KeyBits k = {width(T), width(most_out)};
+    if (k.ord + k.out + KeyBits::SLOT > 61) k = {0, 0};
+    return k;
 }
 
 int launch_segments(const int64_t* prefix, int n, int64_t nunits, int32_t* out,
@@ -2280,8 +2414,8 @@ int build_batched(const rg_pair_desc* pairs, int64_t npairs,
     RG_TRY(hist.alloc(4 * n_groups, s));
     // anomalies, fixups, failed/overflow, long runs, restaged chunks, heavy
     // groups; words 6-7: the triples beyond the staging capacity (64-bit);
-    // word 8: capacity bits of a capacity-mode build; word 9: the heavy
-    // groups' work-queue cursor
+    // word 8: capacity bits of a capacity-mode build; words 10-11: the counts
+    // of the reduction's two lists
     RG_TRY(counters.alloc(12, s));
     RG_TRY(fill_zero(hist.p, 4 * n_groups, s));
     RG_TRY(fill_zero(counters.p, 12, s));
@@ -2305,14 +2439,14 @@ int build_batched(const rg_pair_desc* pairs, int64_t npairs,
     DevBuf<Triple> stage;
     RG_TRY(stage.alloc((size_t)thr_tot * cap, s));
     k_walk_count<<<grid_for(thr_tot, block), block, 0, s>>>(
-        d_builds, pair_of_wave.p, thr_tot, n_groups, start.p, end.p, count.p, hist.p,
+        d_builds, pair_of_wave.p, thr_tot, start.p, end.p, count.p, hist.p,
         stage.p, cap);
     RG_HIP(hipGetLastError());
     tm.mark();  // 3
 
     // ---- fix-up
     k_fixup<<<grid_for(row_tot * 64, 256), 256, 0, s>>>(
-        d_builds, pair_of_row.p, row_tot, n_groups, start.p, end.p, count.p, hist.p,
+        d_builds, pair_of_row.p, row_tot, start.p, end.p, count.p, hist.p,
         counters.p + 1, counters.p + 2, stage.p, cap);
     RG_HIP(hipGetLastError());
     DevBuf<int64_t> chunk_off, bucket_off;
@@ -2390,7 +2524,7 @@ int build_batched(const rg_pair_desc* pairs, int64_t npairs,
     }
     k_scatter<<<grid_for(thr_tot, SCAT_BLOCK), SCAT_BLOCK, (SCAT_BLOCK / 64) * sizeof(ScatTable),
                 s>>>(
-        d_builds, pair_of_wave.p, thr_tot, n_groups, count.p, stage.p, cap, ovbuf.p,
+        d_builds, pair_of_wave.p, thr_tot, count.p, stage.p, cap, ovbuf.p,
         ov_off.p, ov_tot, chunk_off.p, cursor, rec.p, rcell.p, (uint32_t)T, counters.p + 2);
     RG_HIP(hipGetLastError());
     tm.mark();  // 6
@@ -2401,38 +2535,45 @@ int build_batched(const rg_pair_desc* pairs, int64_t npairs,
 
     // ---- reduce -> CSR by input
     DevBuf<int32_t> nnz_row, long_list, group_mode;
-    DevBuf<int64_t> row_off, cell_off, group_off;
+    DevBuf<int64_t> row_off, cell_off;
     DevBuf<KV> red;
     RG_TRY(nnz_row.alloc(cell_tot, s));
     RG_TRY(long_list.alloc(cell_tot, s));
     RG_TRY(group_mode.alloc(n_groups, s));
     RG_TRY(row_off.alloc(cell_tot + 1, s));
     RG_TRY(cell_off.alloc(cell_tot + 1, s));
-    RG_TRY(group_off.alloc(n_groups + 1, s));
     RG_TRY(red.alloc(T, s));
-    // group-major offsets of the reduction's output (group_mode as scratch)
-    k_group_counts<<<grid_for(n_groups, 256), 256, 0, s>>>(bucket_off.p, n_groups,
-                                                           group_mode.p);
-    RG_HIP(hipGetLastError());
-    RG_TRY(scan_i32_to_i64(group_mode.p, group_off.p, n_groups, s));
     tm.mark();  // 7
     DevBuf<int32_t> heavy_list, hist_out;
     RG_TRY(heavy_list.alloc(n_groups, s));
     // entries per output row (the reductions also keep each entry's rank)
     RG_TRY(hist_out.alloc(out_tot, s));
     RG_TRY(fill_zero(hist_out.p, out_tot, s));
-    k_reduce_groups<<<(unsigned)((n_groups + RED_WAVES - 1) / RED_WAVES),
-                      RED_WAVES * 64, 0, s>>>(bucket_off.p, n_groups, group_off.p, rec.p,
-                                              rcell.p, red.p, cell_off.p, vol.p, wi_all.p,
-                                              nnz_row.p, group_mode.p, long_list.p,
-                                              counters.p + 3, heavy_list.p, counters.p + 5,
-                                              d_pcs, pair_of_ing.p, hist_out.p, T,
-                                              counters.p + 8);
+    int64_t most_out = 1;
+    for (int64_t k = 0; k < npairs; k++) most_out = std::max(most_out, pcs[k].n_out);
+    const RedArgs red_args = {bucket_off.p, rec.p,        rcell.p, red.p,         cell_off.p,
+                              vol.p,        wi_all.p,     nnz_row.p, group_mode.p, d_pcs,
+                              pair_of_ing.p, hist_out.p,
+                              (flags & RG_TUNE_REDUCE_GENERAL) ? KeyBits{0, 0}
+                                                               : key_bits(T, most_out)};
+    DevBuf<int32_t> list1, list2;
+    RG_TRY(list1.alloc(n_groups, s));
+    RG_TRY(list2.alloc(n_groups, s));
+    k_reduce_cells<<<(unsigned)n_groups, 64, 0, s>>>(red_args, n_groups, T, counters.p + 8);
+    k_list_groups<<<grid_for(n_groups, LIST_BLOCK), LIST_BLOCK, 0, s>>>(
+        group_mode.p, n_groups, list1.p, counters.p + 10, list2.p, counters.p + 11, heavy_list.p,
+        counters.p + 5);
+    // (twice the resident wavefronts, eight and four per CU by LDS, even out
+    // the groups' differences: 309 -> 290 us at 2049^2 -> 1537^2)
+    k_reduce_listed<LIST1_U, LIST1_N><<<4096, 64, 0, s>>>(
+        red_args, list1.p, counters.p + 10, heavy_list.p, counters.p + 5);
+    k_reduce_listed<LIST2_U, LIST2_N><<<2048, 64, 0, s>>>(
+        red_args, list2.p, counters.p + 11, heavy_list.p, counters.p + 5);
     // (resident waves: four blocks of two waves per CU fit the LDS)
     k_reduce_heavy<<<1024, HEAVY_WAVES * 64, 0, s>>>(
-        bucket_off.p, n_groups, group_off.p, rec.p, rcell.p, red.p, cell_off.p, vol.p,
+        bucket_off.p, rec.p, rcell.p, red.p, cell_off.p, vol.p,
         wi_all.p, nnz_row.p, group_mode.p, long_list.p, counters.p + 3, heavy_list.p,
-        counters.p + 5, counters.p + 9, d_pcs, pair_of_ing.p, hist_out.p);
+        counters.p + 5, d_pcs, pair_of_ing.p, hist_out.p);
     k_bucket_long<<<256, 64, 0, s>>>(cell_off.p, red.p, vol.p, wi_all.p, long_list.p,
                                    counters.p + 3, nnz_row.p, d_pcs, pair_of_ing.p,
                                    hist_out.p);
