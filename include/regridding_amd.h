@@ -207,7 +207,8 @@ int rg_weights_free(rg_weights_t w);
 int rg_weights_set_shape(rg_weights_t w, int64_t ncx_in, int64_t ncy_in,
                          int64_t ncx_out, int64_t ncy_out);
 
-/* Launch shape of the apply kernels (process-wide; 0 keeps the current
+/* Launch shape of the apply kernels that stage input patches (several images
+ * of weights with 65536 outputs or more; process-wide; 0 keeps the current
  * value): tile_w output cells along the last axis per tile row of a
  * 256-cell tile for the FP64 forward apply, twice that (up to 256) for FP32
  * values and for the adjoint (default 16; negative: same widths, staged

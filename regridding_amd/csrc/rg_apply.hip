@@ -5,26 +5,26 @@
 // storage order (sorted by (input, output)).  Each output therefore receives
 // its terms in ascending input order, one rounded multiply and one rounded
 // add at a time, starting from +0.0.  The GPU gathers instead: one lane owns
-// one output cell, walks its CSR row (columns ascending) and accumulates in
-// exactly that order, which reproduces the reference bit for bit without
-// atomics.  A lane keeps DB batch accumulators so every weight is loaded once
-// per DB images; batches larger than DB loop over tiles (the row comes from
-// cache the second time).
+// one output cell and adds up its CSR row (columns ascending) in exactly that
+// order, which reproduces the reference bit for bit without atomics.
+//
+// One image, small weights and batched jobs read the entries as they lie and
+// gather from global memory (k_apply, k_apply_jobs).  Several images of large
+// weights stage patches of the input in LDS, DB images at a time, which
+// takes a plan (k_apply_rounds).
 //
 // The adjoint (transpose=1) is the same gather over the CSR by input, whose
 // rows hold the outputs in ascending order: exactly the order in which the
 // reference applies regrid_from_weights(*transpose_weights(w)).
 //
 // Launch layout.  The rows of a CSR are the cells of a 2-D grid.  A block
-// of 256 lanes owns a tile of output cells, tile_w wide along the grid's
-// last axis and 256 / tile_w tall, so the input cells it gathers form one
+// of 256 lanes owns a tile of output cells (with a plan tile_w wide along the
+// grid's last axis and 256 / tile_w tall, otherwise 64 and 4), so the input cells it gathers form one
 // compact patch (a linear run of rows would be a thin band tilted across
 // the input grid, re-fetched by every neighbouring run).  Blocks are
 // renumbered so each of the 8 XCDs of the MI355X (blocks arrive
 // round-robin) sweeps one contiguous band of tiles, keeping the patches of
-// neighbouring tiles in that XCD's L2.  The launch's second dimension is
-// the image group: all tiles of images [0, DB) first, then the next DB, so
-// the gathered footprint per pass is DB images deep.
+// neighbouring tiles in that XCD's L2.
 //
 // The results are stored nontemporal: each is written once and not read
 // back by the launch, so written through the caches they would only evict
@@ -51,39 +51,140 @@ struct ApplyGrid {
     int64_t ntx, ntiles;  // tiles along gy, tiles in total
 };
 
-template <class T, int DB>
+// ---- the apply without a plan ----------------------------------------------
+//
+// A lane that walks its own row reads col and w at a stride of one row (about
+// five entries): every load instruction of the wavefront touches 20 to 30
+// cache lines, and the next entry's the same lines again, which bounds it far
+// below the memory's rate.  Here the wavefront reads the entries of its 64
+// rows as they lie, 64 at a time, gathers x for each (neighbouring lanes hold
+// neighbouring columns), and puts the rounded products into LDS; a lane then
+// adds up its own row's in entry order: the same roundings in the same order.
+// One image of FP64, plain pairs: 1025^2 -> 769^2 21.9 -> 12.4 us, 2049^2 ->
+// 1537^2 74 -> 31 us (6.9 TB/s), its adjoint 62 -> 38 us, adjoint of 1025^2
+// -> 1500^2 83 -> 23 us; eight views of a 1024^2 image, 134 -> 95 us.
+// The wavefronts need no barrier; a block is four of them only so that
+// neighbouring rows share the L1.
+//
+// Entries per lane at a time: 6 (a wavefront's 345 entries at output cells a
+// third larger than the input's are one chunk) at 54 registers; 8 are 66 and
+// 10 are 78 registers and lose 5 % to 10 % where the rows are short, and gain
+// 15 % only where they hold nine or more.
+constexpr int ENTRIES_U = 6;
+constexpr int PROD_SLOTS = 64 * ENTRIES_U + 1;  // the last one is 0
+// Launches of fewer tiles than this split the images over more blocks: 8
+// images of 129^2 -> 101^2 take 7.6 us in 40 blocks, 4.6 us in 320 (any
+// limit from 512 to 4096 measures the same).
+constexpr int64_t SPLIT_TILES = 1024;
+
+// Entries [c0, c0 + 64 * U) of the wavefront's `total` for `images` images:
+// the products go to LDS in entry order, and each lane adds up those of its
+// row, entries [s, e), to y (from 0 where c0 is 0).
+template <class T, int U>
+__device__ inline void apply_entries(const int32_t* __restrict__ col, const T* __restrict__ w,
+                                     const T* __restrict__ x, T* __restrict__ y, int64_t nrows,
+                                     int64_t ncols, int32_t images, int32_t c0, int32_t total,
+                                     int32_t s, int32_t e, bool has_row, T* __restrict__ prod)
+{
+    const int32_t lane = threadIdx.x & 63;
+    uint32_t c[U];
+    T wq[U], xv[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        const uint32_t t = min(c0 + u * 64 + lane, total - 1);
+        c[u] = (uint32_t)col[t];
+        wq[u] = w[t];
+    }
+    s = max(s - c0, 0);
+    e = min(e - c0, 64 * U);
+    const bool stores = c0 ? s < e : has_row;
+    for (int32_t m = 0; m < images; m++) {
+#pragma unroll
+        for (int u = 0; u < U; u++) xv[u] = x[c[u]];
+        __builtin_amdgcn_wave_barrier();  // the last image's products are read
+#pragma unroll
+        for (int u = 0; u < U; u++) prod[u * 64 + lane] = wq[u] * xv[u];
+        x += ncols;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        if (stores) {
+            T acc = c0 ? *y : T(0);
+            // four at a time; past the row's end +0 is added, which changes
+            // no sum (none is -0, as it starts from +0)
+            for (int32_t q = s; q < e; q += 4) {
+                T p[4];
+#pragma unroll
+                for (int u = 0; u < 4; u++) p[u] = prod[q + u < e ? q + u : PROD_SLOTS - 1];
+#pragma unroll
+                for (int u = 0; u < 4; u++) acc = acc + p[u];
+            }
+            __builtin_nontemporal_store(acc, y);
+        }
+        y += nrows;
+    }
+}
+
+// Applies the CSR to one tile and `images` images, a wavefront for each 64
+// consecutive rows and by itself.  A tile is 64 columns of APPLY_BLOCK / 64
+// grid rows at (ib, jb) or, if `flat`, APPLY_BLOCK rows of one long row.
+template <class T>
+__device__ inline void apply_rows(const int32_t* __restrict__ rowptr,
+                                  const int32_t* __restrict__ col, const T* __restrict__ w,
+                                  const T* __restrict__ x, T* __restrict__ y, int64_t nrows,
+                                  int64_t ncols, int32_t images, int64_t gy, int64_t ib,
+                                  int64_t jb, bool flat, T* __restrict__ prod)
+{
+    const int32_t lane = threadIdx.x & 63;
+    const int32_t wave = __builtin_amdgcn_readfirstlane((int32_t)threadIdx.x / 64);
+    const int64_t i = ib + (flat ? 0 : wave), j = jb + (flat ? wave * 64 : 0);
+    const int64_t r0 = i * gy + j;
+    if (r0 >= nrows || j >= gy) return;
+    const int32_t rows = gy - j < 64 ? (int32_t)(gy - j) : 64;
+    // lanes past the last row take that row's end: no entries
+    const int64_t r = r0 + min(lane, rows - 1);
+    int32_t s = rowptr[r];
+    int32_t e = rowptr[r + 1];
+    const bool valid = lane < rows;
+    if (!valid) s = e;
+    const int32_t first = __builtin_amdgcn_readlane(s, 0);
+    const int32_t total = __builtin_amdgcn_readlane(e, 63) - first;
+    s -= first;
+    e -= first;
+    col += first;
+    w += first;
+    y += r;
+    if (lane == 0) prod[PROD_SLOTS - 1] = T(0);
+    if (total == 0) {
+        if (valid)
+            for (int32_t m = 0; m < images; m++) y[m * nrows] = T(0);
+        return;
+    }
+    if (total <= 64 * (ENTRIES_U / 2))
+        apply_entries<T, ENTRIES_U / 2>(col, w, x, y, nrows, ncols, images, 0, total, s, e, valid,
+                                        prod);
+    else
+        for (int32_t c0 = 0; c0 < total; c0 += 64 * ENTRIES_U)
+            apply_entries<T, ENTRIES_U>(col, w, x, y, nrows, ncols, images, c0, total, s, e,
+                                        valid, prod);
+}
+
+template <class T>
 __global__ __launch_bounds__(APPLY_BLOCK) void k_apply(
     const int32_t* __restrict__ rowptr, const int32_t* __restrict__ col,
     const T* __restrict__ w, const T* __restrict__ x, T* __restrict__ y,
-    int64_t nrows, int64_t ncols, int64_t batch, ApplyGrid G)
+    int64_t nrows, int64_t ncols, int64_t batch, int32_t db, ApplyGrid G)
 {
-    const int64_t nb = gridDim.x;  // a multiple of NUM_XCD
-    const int64_t b = blockIdx.x;
-    const int64_t tile = (b % NUM_XCD) * (nb / NUM_XCD) + b / NUM_XCD;
+    __shared__ T prod[APPLY_BLOCK / 64][PROD_SLOTS];
+    const uint32_t nb = gridDim.x;  // a multiple of NUM_XCD
+    const uint32_t b = blockIdx.x;
+    const uint32_t tile = (b % NUM_XCD) * (nb / NUM_XCD) + b / NUM_XCD;
     if (tile >= G.ntiles) return;
-    const int64_t ti = tile / G.ntx, tj = tile % G.ntx;
-    const int64_t i = ti * G.th + threadIdx.x / G.tw;
-    const int64_t j = tj * G.tw + threadIdx.x % G.tw;
-    if (i >= G.gx || j >= G.gy) return;
-    const int64_t r = i * G.gy + j;
-    const int64_t d0 = (int64_t)blockIdx.y * DB;
-    const int64_t nd = batch - d0 < DB ? batch - d0 : DB;
-    const int32_t s = rowptr[r], e = rowptr[r + 1];
-    T acc[DB];
-#pragma unroll
-    for (int q = 0; q < DB; q++) acc[q] = T(0);
-    const T* xb = x + d0 * ncols;
-    for (int32_t q = s; q < e; q++) {
-        const int64_t c = col[q];
-        const T wq = w[q];
-#pragma unroll
-        for (int m = 0; m < DB; m++)
-            if (m < nd) acc[m] = acc[m] + wq * xb[m * ncols + c];
-    }
-    T* yb = y + d0 * nrows + r;
-#pragma unroll
-    for (int m = 0; m < DB; m++)
-        if (m < nd) __builtin_nontemporal_store(acc[m], &yb[m * nrows]);
+    const uint32_t ntx = (uint32_t)G.ntx, ti = tile / ntx, tj = tile % ntx;
+    const int64_t d0 = (int64_t)blockIdx.y * db;
+    const int64_t nd = batch - d0 < db ? batch - d0 : db;
+    apply_rows<T>(rowptr, col, w, x + d0 * ncols, y + d0 * nrows, nrows, ncols, (int32_t)nd, G.gy,
+                  ti * G.th, tj * G.tw, G.th == 1, prod[threadIdx.x / 64]);
 }
 
 // ---- the apply plan -------------------------------------------------------
@@ -455,11 +556,8 @@ __global__ void k_to_f32(const double* __restrict__ a, float* __restrict__ b,
 //
 // Many applies, each with its own weights, in one launch.  Jobs are cut into
 // blocks of one tile of output rows x JOB_DB images; block b finds its job in
-// the jobs' block prefix.  A tile is a compact patch of the output grid (16
-// x 16 cells for 8-byte values), so the inputs its lanes gather are one
-// compact patch too, where runs of 256 consecutive rows gathered along a
-// thin band (the FP64 apply of the 256-pair batch, 1-8 images per pair: 1.71
-// -> 1.51 ms).  The accumulation per output is the one of k_apply.
+// the jobs' block prefix.  The tiles and the accumulation per output are
+// those of k_apply.
 //
 // Blocks are renumbered so each of the 8 XCDs takes one contiguous range of
 // the blocks (blocks arrive round-robin over the XCDs): neighbouring tiles
@@ -470,55 +568,20 @@ __global__ __launch_bounds__(APPLY_BLOCK) void k_apply_jobs(
     const JobDesc* __restrict__ jobs, const int64_t* __restrict__ block_prefix,
     int njobs, int64_t nblocks, const int32_t* __restrict__ abort_flag)
 {
+    __shared__ T prod[APPLY_BLOCK / 64][PROD_SLOTS];
     if (abort_flag && *abort_flag) return;  // uniform: one word for the grid
     const int64_t ng = gridDim.x;  // a multiple of NUM_XCD
     const int64_t b = (blockIdx.x % NUM_XCD) * (ng / NUM_XCD) + blockIdx.x / NUM_XCD;
     if (b >= nblocks) return;
     const JobDesc& J = jobs[seg_of(block_prefix, njobs, b)];
-    const int64_t lt = b - J.block_base;
-    const int64_t grp = lt / J.nrt, tile = lt - grp * J.nrt;
-    const int64_t ti = tile / J.ntx, tj = tile - ti * J.ntx;
-    const int64_t i = ti * J.th + (int32_t)threadIdx.x / J.tw;
-    const int64_t j = tj * J.tw + (int32_t)threadIdx.x % J.tw;
-    if (j >= J.gy) return;
-    const int64_t r = i * J.gy + j;
-    if (r >= J.nrows) return;
-    const int64_t d0 = grp * JOB_DB;
+    const uint32_t lt = (uint32_t)(b - J.block_base), nrt = (uint32_t)J.nrt;
+    const uint32_t ntx = (uint32_t)J.ntx, grp = lt / nrt, tile = lt - grp * nrt;
+    const int64_t ti = tile / ntx, tj = tile % ntx;
+    const int64_t d0 = (int64_t)grp * JOB_DB;
     const int64_t nd = J.batch - d0 < JOB_DB ? J.batch - d0 : JOB_DB;
-    const int32_t* __restrict__ col = J.col;
-    const T* __restrict__ w = (const T*)J.w;
-    const T* __restrict__ xb = (const T*)J.x + d0 * J.ncols;
-    const int64_t ncols = J.ncols;
-    const int32_t s = J.rowptr[r], e = J.rowptr[r + 1];
-    T acc[JOB_DB];
-#pragma unroll
-    for (int m = 0; m < JOB_DB; m++) acc[m] = T(0);
-    int32_t q = s;
-    for (; q + 4 <= e; q += 4) {
-        int64_t c[4];
-        T wq[4];
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-            c[u] = col[q + u];
-            wq[u] = w[q + u];
-        }
-#pragma unroll
-        for (int u = 0; u < 4; u++)
-#pragma unroll
-            for (int m = 0; m < JOB_DB; m++)
-                if (m < nd) acc[m] = acc[m] + wq[u] * xb[m * ncols + c[u]];
-    }
-    for (; q < e; q++) {
-        const int64_t c = col[q];
-        const T wq = w[q];
-#pragma unroll
-        for (int m = 0; m < JOB_DB; m++)
-            if (m < nd) acc[m] = acc[m] + wq * xb[m * ncols + c];
-    }
-    T* yb = (T*)J.y + d0 * J.nrows + r;
-#pragma unroll
-    for (int m = 0; m < JOB_DB; m++)
-        if (m < nd) yb[m * J.nrows] = acc[m];
+    apply_rows<T>(J.rowptr, J.col, (const T*)J.w, (const T*)J.x + d0 * J.ncols,
+                  (T*)J.y + d0 * J.nrows, J.nrows, J.ncols, (int32_t)nd, J.gy, ti * J.th,
+                  tj * J.tw, J.th == 1, prod[threadIdx.x / 64]);
 }
 
 namespace {
@@ -540,7 +603,7 @@ bool g_use_plan = true;
 bool g_rounds = true;  // one block per tile looping over image groups
 std::mutex g_plan_mu;
 
-ApplyGrid make_grid(const int64_t* shape, int64_t nrows, int64_t value_bytes, int dir)
+ApplyGrid make_grid(const int64_t* shape, int64_t nrows, int64_t tile_w)
 {
     ApplyGrid G;
     G.gx = shape[0];
@@ -549,8 +612,31 @@ ApplyGrid make_grid(const int64_t* shape, int64_t nrows, int64_t value_bytes, in
         G.gx = 1;
         G.gy = nrows;
     }
-    G.tw = value_bytes >= 8 && dir == 0 ? g_tile_w : std::min<int64_t>(2 * g_tile_w, APPLY_BLOCK);
+    G.tw = tile_w;
     if (G.gx == 1 || G.tw > G.gy) G.tw = APPLY_BLOCK;
+    G.th = APPLY_BLOCK / G.tw;
+    G.ntx = (G.gy + G.tw - 1) / G.tw;
+    G.ntiles = G.ntx * ((G.gx + G.th - 1) / G.th);
+    return G;
+}
+
+// Tiles of an apply without a plan: 64 columns of four grid rows (16 or 32
+// columns of more rows measure the same).  Grids of narrow rows are taken as
+// one long row, where a block's consecutive rows are a compact patch too; so
+// are rows of unknown shape.
+ApplyGrid gather_grid(const int64_t* shape, int64_t nrows)
+{
+    ApplyGrid G;
+    G.gx = shape[0];
+    G.gy = shape[1];
+    G.tw = 64;
+    // (grids of narrow rows as well: a block's consecutive rows are a compact
+    // patch there)
+    if (G.gx * G.gy != nrows || G.gy < 64) {
+        G.gx = 1;
+        G.gy = nrows;
+        G.tw = APPLY_BLOCK;
+    }
     G.th = APPLY_BLOCK / G.tw;
     G.ntx = (G.gy + G.tw - 1) / G.tw;
     G.ntiles = G.ntx * ((G.gx + G.th - 1) / G.th);
@@ -561,12 +647,15 @@ ApplyGrid make_grid(const int64_t* shape, int64_t nrows, int64_t value_bytes, in
 // on stream s; later applies on other streams must be ordered after it).
 int ensure_plan(rg_weights* W, int dir, int64_t value_bytes, const int32_t* rowptr,
                 const int32_t* col, const ApplyGrid& G, int64_t src_gy,
-                hipStream_t s, rg_weights::Plan** out)
+                int64_t batch, hipStream_t s, rg_weights::Plan** out)
 {
     *out = nullptr;
     // below PLAN_MIN_ROWS outputs the gathered input stays in L2 anyway and
-    // a plan (two kernels and a host wait) would only add latency
-    if (!g_use_plan || G.gx == 1 || W->nnz == 0 || G.gx * G.gy < PLAN_MIN_ROWS)
+    // a plan (two kernels and a host wait) would only add latency; one image
+    // is faster without (2049^2 -> 1537^2 FP64 31 against 37 us, FP32 25
+    // against 30, their adjoints 38 against 49 and 29 against 42; two images
+    // are even, and from four on the plan is faster)
+    if (!g_use_plan || batch == 1 || G.gx == 1 || W->nnz == 0 || G.gx * G.gy < PLAN_MIN_ROWS)
         return RG_OK;
     std::lock_guard<std::mutex> lk(g_plan_mu);
     rg_weights::Plan& P = W->plan[2 * dir + (value_bytes < 8 ? 1 : 0)];
@@ -599,9 +688,17 @@ int launch_apply(rg_weights* W, int dir, const int32_t* rowptr,
                  int64_t src_gy, int64_t batch, hipStream_t s)
 {
     if (nrows == 0 || batch == 0) return RG_OK;
-    const ApplyGrid G = make_grid(shape, nrows, sizeof(T), dir);
+    const int64_t tile_w =
+        sizeof(T) >= 8 && dir == 0 ? g_tile_w : std::min(2 * g_tile_w, APPLY_BLOCK);
+    ApplyGrid G = make_grid(shape, nrows, tile_w);
     rg_weights::Plan* P = nullptr;
-    RG_TRY(ensure_plan(W, dir, sizeof(T), rowptr, col, G, src_gy, s, &P));
+    RG_TRY(ensure_plan(W, dir, sizeof(T), rowptr, col, G, src_gy, batch, s, &P));
+    int32_t sb = 0;
+    if (!P) {
+        G = gather_grid(shape, nrows);
+        sb = (int32_t)std::min<int64_t>(batch, JOB_DB);
+        while (sb > 1 && G.ntiles * ((batch + sb - 1) / sb) < SPLIT_TILES) sb = (sb + 1) / 2;
+    }
     const int64_t nb = (G.ntiles + NUM_XCD - 1) / NUM_XCD * NUM_XCD;
     int db = g_images_per_pass;
     while (db > 1 && db > batch) db >>= 1;
@@ -641,13 +738,8 @@ int launch_apply(rg_weights* W, int dir, const int32_t* rowptr,
         }
 #undef RG_PLANNED
     } else {
-        switch (db) {
-        case 16: k_apply<T, 16><<<g, bl, 0, s>>>(rowptr, col, w, x, y, nrows, ncols, batch, G); break;
-        case 8: k_apply<T, 8><<<g, bl, 0, s>>>(rowptr, col, w, x, y, nrows, ncols, batch, G); break;
-        case 4: k_apply<T, 4><<<g, bl, 0, s>>>(rowptr, col, w, x, y, nrows, ncols, batch, G); break;
-        case 2: k_apply<T, 2><<<g, bl, 0, s>>>(rowptr, col, w, x, y, nrows, ncols, batch, G); break;
-        default: k_apply<T, 1><<<g, bl, 0, s>>>(rowptr, col, w, x, y, nrows, ncols, batch, G); break;
-        }
+        k_apply<T><<<dim3((unsigned)nb, (unsigned)((batch + sb - 1) / sb)), bl, 0, s>>>(
+            rowptr, col, w, x, y, nrows, ncols, batch, sb, G);
     }
     RG_HIP(hipGetLastError());
     return RG_OK;
@@ -753,7 +845,7 @@ int launch_jobs_common(const rg_apply_job* jobs, int64_t njobs, bool f32,
         d.batch = jb.batch;
         if (d.nrows == 0 || d.batch == 0) continue;
         const int64_t* shape = jb.transpose ? W->shape_in : W->shape_out;
-        job_tiles(d, shape[0], shape[1], f32 ? 4 : 8);
+        job_tiles(d, shape[0], shape[1]);
         d.block_base = nblocks;
         prefix.push_back(nblocks);
         nblocks += d.nrt * ((d.batch + JOB_DB - 1) / JOB_DB);
@@ -818,18 +910,15 @@ int apply_jobs_device(const JobDesc* jobs, const int64_t* prefix, int njobs, int
     return RG_OK;
 }
 
-void job_tiles(JobDesc& d, int64_t gx, int64_t gy, int64_t value_bytes)
+void job_tiles(JobDesc& d, int64_t gx, int64_t gy)
 {
-    if (gx * gy != d.nrows) {  // shape unknown: one long row
-        gx = 1;
-        gy = d.nrows;
-    }
-    const int64_t tw = value_bytes >= 8 ? 16 : 32;
-    d.tw = gx == 1 || gy < tw ? APPLY_BLOCK : (int32_t)tw;
-    d.th = APPLY_BLOCK / d.tw;
-    d.gy = gy;
-    d.ntx = (gy + d.tw - 1) / d.tw;
-    d.nrt = d.ntx * ((gx + d.th - 1) / d.th);
+    const int64_t shape[2] = {gx, gy};
+    const ApplyGrid G = gather_grid(shape, d.nrows);
+    d.tw = (int32_t)G.tw;
+    d.th = (int32_t)G.th;
+    d.gy = G.gy;
+    d.ntx = G.ntx;
+    d.nrt = G.ntiles;
 }
 
 }  // namespace rg
