@@ -107,6 +107,12 @@ int rg_memset(void* dst, int value, size_t bytes, void* stream);
 /* Pinned (page-locked) host memory, for asynchronous transfers. */
 int rg_host_alloc(void** ptr, size_t bytes);
 int rg_host_free(void* ptr);
+/* Content digests of n host arrays, to notice a change (not cryptographic):
+ * start begins to hash them, in threads of its own where they are large;
+ * finish waits, writes one digest per array and ends the job.  A started job
+ * is finished exactly once, and the arrays stay until then. */
+int rg_digest_start(const void* const* data, const size_t* bytes, int n, void** job);
+int rg_digest_finish(void* job, uint64_t* digests);
 int rg_stream_create(void** stream);
 int rg_stream_destroy(void* stream);
 int rg_stream_sync(void* stream);

@@ -149,6 +149,8 @@ SIGNATURES = {
     "rg_memcpy_htod": (ctypes.c_int, [_vp, _vp, ctypes.c_size_t, _vp]),
     "rg_memcpy_dtoh": (ctypes.c_int, [_vp, _vp, ctypes.c_size_t, _vp]),
     "rg_memset": (ctypes.c_int, [_vp, ctypes.c_int, ctypes.c_size_t, _vp]),
+    "rg_digest_start": (ctypes.c_int, [_vp, _vp, ctypes.c_int, ctypes.POINTER(_vp)]),
+    "rg_digest_finish": (ctypes.c_int, [_vp, _vp]),
     "rg_stream_create": (ctypes.c_int, [ctypes.POINTER(_vp)]),
     "rg_stream_destroy": (ctypes.c_int, [_vp]),
     "rg_stream_sync": (ctypes.c_int, [_vp]),

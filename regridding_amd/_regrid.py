@@ -59,7 +59,7 @@ def prepare_apply(
 
     Returns a dict with ``flat`` (the per-element weight triples, length D),
     ``values_input`` (D, n_in) float64 C-contiguous, ``values_output`` the
-    (D, *cells_out) zero-filled buffer the result goes to, plus the pieces
+    (D, *cells_out) buffer the result goes to, plus the pieces
     :func:`finish_apply` needs.
     """
     unit = getattr(values_input, "unit", None)
@@ -103,7 +103,8 @@ def prepare_apply(
     values_input = np.broadcast_to(values_input, full_in, subok=True)
 
     if values_output is None:
-        values_output = np.zeros_like(values_input, shape=full_out, dtype=float)
+        # (every element is written by finish_apply or straight into it)
+        values_output = np.empty_like(values_input, shape=full_out, dtype=float)
     else:
         if values_output.shape != full_out:
             raise ValueError(f"{values_output.shape=} should be equal to {full_out}")
@@ -145,7 +146,8 @@ def finish_apply(prep: dict, result: np.ndarray) -> np.ndarray:
     """Write `result` (D, n_out) into the output buffer and restore the
     caller's axis order and units (``_regrid_from_weights.py:152-162``)."""
     out = prep["values_output"]
-    out.reshape(out.shape[0], -1)[...] = result
+    if result is not prep.get("direct"):
+        out.reshape(out.shape[0], -1)[...] = result
     out = out.reshape(*prep["shape_output_moved"])
     out = np.moveaxis(out, prep["axis_output_last"], prep["axis_output"])
     unit, unit_weights = prep["unit"], prep["unit_weights"]
@@ -156,14 +158,15 @@ def finish_apply(prep: dict, result: np.ndarray) -> np.ndarray:
     return out << unit
 
 
-def _handle_for(element, n_in: int, n_out: int) -> tuple[Weights, bool]:
-    ii, io, w = element
-    w = np.asarray(w)
-    if isinstance(ii, np.ndarray) and isinstance(io, np.ndarray):
-        hit = _cache.lookup(ii, io, w)
-        if hit is not None:
-            return hit
-    return import_weights(ii, io, w, n_in, n_out), False
+def _direct_output(prep: dict) -> np.ndarray | None:
+    """The output buffer as a float64 (D, n_out) array that the device's
+    result can be copied into as it is, or None; :func:`finish_apply` then
+    finds the result in place."""
+    out = prep["values_output"]
+    if type(out) is not np.ndarray or out.dtype != np.float64 or not out.flags.writeable:
+        return None
+    prep["direct"] = out.reshape(out.shape[0], prep["n_out"])
+    return prep["direct"]
 
 
 def _block_diagonal(flat, n_in: int, n_out: int):
@@ -178,8 +181,8 @@ def _block_diagonal(flat, n_in: int, n_out: int):
         ii, io, w = flat[d]
         if not (isinstance(ii, np.ndarray) and isinstance(io, np.ndarray)):
             return None
-        hit = _cache.lookup_part(ii, io, np.asarray(w))
-        if hit is None or hit[2] is None:
+        hit = _cache.lookup_block(ii, io, np.asarray(w))
+        if hit is None:
             return None
         handle, transposed, (k, nparts, bi, bo) = hit
         if transposed:
@@ -193,10 +196,13 @@ def _block_diagonal(flat, n_in: int, n_out: int):
     return first
 
 
-def apply_device(handle: Weights, transposed: bool, x: np.ndarray, n_out: int) -> np.ndarray:
-    """(D, n_in) host float64 -> (D, n_out) host float64 through the GPU."""
+def apply_device(handle: Weights, transposed: bool, x: np.ndarray, n_out: int,
+                 out: np.ndarray | None = None) -> np.ndarray:
+    """(D, n_in) host float64 -> (D, n_out) host float64 through the GPU, into
+    `out` where given (C-contiguous, D * n_out values)."""
     D = x.shape[0]
-    out = np.empty((D, n_out))
+    if out is None:
+        out = np.empty((D, n_out))
     if D == 0 or n_out == 0:
         return out
     dx = DeviceArray.from_host(x)
@@ -212,6 +218,28 @@ def _check_sizes(handle: Weights, transposed: bool, n_in: int, n_out: int) -> No
             f"weights relate {hin} input cells to {hout} output cells, but the "
             f"values have {n_in} input cells and {n_out} output cells"
         )
+
+
+def _apply_element(element, x: np.ndarray, n_in: int, n_out: int,
+                   out: np.ndarray | None = None) -> np.ndarray:
+    """One weights triple applied to the rows of `x`."""
+    ii, io, w = element
+    w = np.asarray(w)
+    if isinstance(ii, np.ndarray) and isinstance(io, np.ndarray):
+        hit = _cache.lookup_pending(ii, io, w)
+        if hit is not None:
+            # the arrays are compared with the resident weights meanwhile
+            handle, transposed, pending = hit
+            hin, hout = (handle.n_in, handle.n_out)[:: -1 if transposed else 1]
+            if (hin, hout) == (n_in, n_out):
+                y = apply_device(handle, transposed, x, n_out, out)
+                if pending.unchanged():
+                    return y
+            elif pending.unchanged():
+                _check_sizes(handle, transposed, n_in, n_out)
+    handle = import_weights(ii, io, w, n_in, n_out)
+    _check_sizes(handle, False, n_in, n_out)
+    return apply_device(handle, False, x, n_out, out)
 
 
 def regrid_from_weights(
@@ -239,23 +267,20 @@ def regrid_from_weights(
     if whole is not None:
         # every element is its own block of one handle, in order: one launch
         handle, transposed = whole
-        y = apply_device(handle, transposed, x.reshape(1, D * n_in), D * n_out)
-        return finish_apply(prep, y.reshape(D, n_out))
-    result = np.zeros((D, n_out))
+        out = _direct_output(prep)
+        y = apply_device(handle, transposed, x.reshape(1, D * n_in), D * n_out, out)
+        return finish_apply(prep, out if out is not None else y.reshape(D, n_out))
     # group the elements by weight object: broadcast weights are one object
     groups: dict[int, list[int]] = {}
     for d in range(D):
         groups.setdefault(id(flat[d]), []).append(d)
+    result = None if len(groups) == 1 else np.zeros((D, n_out))
     for ds in groups.values():
-        handle, transposed = _handle_for(flat[ds[0]], n_in, n_out)
-        _check_sizes(handle, transposed, n_in, n_out)
-        idx = np.asarray(ds)
-        block = x if len(ds) == D else np.ascontiguousarray(x[idx])
-        y = apply_device(handle, transposed, block, n_out)
         if len(ds) == D:
-            result = y
+            result = _apply_element(flat[ds[0]], x, n_in, n_out, _direct_output(prep))
         else:
-            result[idx] = y
+            idx = np.asarray(ds)
+            result[idx] = _apply_element(flat[ds[0]], np.ascontiguousarray(x[idx]), n_in, n_out)
     return finish_apply(prep, result)
 
 
