@@ -119,7 +119,7 @@ struct UncountSink {
 // Bucket cursors: cursor[b] starts at the first record of bucket b and each
 // store claims records with a returning atomic (record positions fit in 32
 // bits: a build holds fewer than 2^32 triples).  A store is only
-// bounds-checked against the record count; k_cursor_check then verifies that
+// bounds-checked against the record count; the reduction then verifies that
 // every cursor ended exactly at its bucket's end, which holds iff each
 // bucket received exactly the triples the count walk histogrammed.
 __device__ inline void put_record(KV* __restrict__ rec, uint8_t* __restrict__ rcell,
@@ -153,21 +153,6 @@ struct OverflowSink {
         n++;
     }
 };
-
-__global__ void k_cursor_init(const int64_t* __restrict__ bucket_off,
-                              uint32_t* __restrict__ cursor, int64_t nb)
-{
-    const int64_t b = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (b < nb) cursor[b] = (uint32_t)bucket_off[b];
-}
-
-__global__ void k_cursor_check(const int64_t* __restrict__ bucket_off,
-                               const uint32_t* __restrict__ cursor, int64_t nb,
-                               int32_t* __restrict__ bad)
-{
-    const int64_t b = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (b < nb && (int64_t)cursor[b] != bucket_off[b + 1]) atomicAdd(bad, 1);
-}
 
 // ---- prepare -------------------------------------------------------------
 
@@ -231,21 +216,56 @@ struct PairCells {
     int64_t out_gbase, n_out;  // output cells
 };
 
-// unit -> segment lookup table (pair of a wavefront, row, cell group ...)
-__global__ void k_segments(const int64_t* __restrict__ prefix, int n,
-                           int64_t nunits, int32_t* __restrict__ out)
-{
-    const int64_t u = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (u < nunits) out[u] = seg_of(prefix, n, u);
-}
+// The launches of a small build cost more than their work (a 67 x 190 -> 81 x
+// 125 vertex pair took 43, each 2 to 5 us on the device and as long on the
+// host), so what only has to come before the next kernel shares one: the
+// preparation is k_prepare_vertices, k_prepare_grids, k_grid_boxes and
+// k_starts, where it was 16 launches (that pair, built and applied: 322 -> 258
+// us; 64 mixed pairs 4553 -> 4370 us; 2049^2 -> 1537^2 the same).
+
+// What a build's tables are filled from: the pair of every wavefront, row and
+// cell group (unit -> segment of a prefix), and the words that start at 0.
+struct TableFill {
+    static constexpr int SEGS = 4, ZEROS = 3;
+    const int64_t* prefix[SEGS];
+    int32_t* out[SEGS];
+    int64_t units[SEGS];
+    int32_t* zero[ZEROS];
+    int64_t words[ZEROS];
+    int npairs;
+
+    int64_t items() const
+    {
+        int64_t n = 0;
+        for (int q = 0; q < SEGS; q++) n += units[q];
+        for (int q = 0; q < ZEROS; q++) n += words[q];
+        return n;
+    }
+};
 
 // One block per tile of VTILE vertices of one grid: interleaves the
-// vertices into (x, y) pairs and reduces the tile's bounding box.
-__global__ __launch_bounds__(BBOX_BLOCK) void k_grid_tiles(
+// vertices into (x, y) pairs and reduces the tile's bounding box.  The blocks
+// past the tiles fill the tables, a thread for each item.
+__global__ __launch_bounds__(BBOX_BLOCK) void k_prepare_vertices(
     const GridDesc* __restrict__ grids, const int64_t* __restrict__ tile_prefix,
-    int ngrids, double2* __restrict__ xy_all, double* __restrict__ part)
+    int ngrids, int64_t ntiles, double2* __restrict__ xy_all, double* __restrict__ part,
+    TableFill F)
 {
     const int64_t tile = blockIdx.x;
+    if (tile >= ntiles) {
+        int64_t u = (tile - ntiles) * BBOX_BLOCK + threadIdx.x;
+#pragma unroll
+        for (int q = 0; q < TableFill::SEGS; q++) {
+            if (u >= 0 && u < F.units[q]) F.out[q][u] = seg_of(F.prefix[q], F.npairs, u);
+            u -= F.units[q];
+        }
+#pragma unroll
+        for (int q = 0; q < TableFill::ZEROS; q++) {
+            if (u >= 0 && u < F.words[q]) F.zero[q][u] = 0;
+            u -= F.words[q];
+        }
+        return;
+    }
     const GridDesc& G = grids[seg_of(tile_prefix, ngrids, tile)];
     const int64_t nv = G.nx * G.ny;
     const int64_t v0 = (tile - G.tile_base) * VTILE;
@@ -278,167 +298,13 @@ __global__ __launch_bounds__(BBOX_BLOCK) void k_grid_tiles(
         for (int q = 0; q < 4; q++) part[4 * tile + q] = sh[q][0];
 }
 
-// One block per grid: the bounding box from its tiles' partial boxes.
-__global__ __launch_bounds__(BBOX_BLOCK) void k_grid_bbox(
-    const int64_t* __restrict__ tile_prefix, const double* __restrict__ part,
-    double* __restrict__ bbox_all)
-{
-    const int g = blockIdx.x;
-    const int64_t t0 = tile_prefix[g], t1 = tile_prefix[g + 1];
-    double v[4] = {part[4 * t0], part[4 * t0 + 1], part[4 * t0 + 2], part[4 * t0 + 3]};
-    for (int64_t t = t0 + threadIdx.x; t < t1; t += BBOX_BLOCK) {
-        v[0] = nan_min(v[0], part[4 * t + 0]);
-        v[1] = nan_min(v[1], part[4 * t + 1]);
-        v[2] = nan_max(v[2], part[4 * t + 2]);
-        v[3] = nan_max(v[3], part[4 * t + 3]);
-    }
-    __shared__ double sh[4][BBOX_BLOCK];
-    for (int q = 0; q < 4; q++) sh[q][threadIdx.x] = v[q];
-    __syncthreads();
-    for (int o = BBOX_BLOCK / 2; o > 0; o >>= 1) {
-        if ((int)threadIdx.x < o) {
-            sh[0][threadIdx.x] = nan_min(sh[0][threadIdx.x], sh[0][threadIdx.x + o]);
-            sh[1][threadIdx.x] = nan_min(sh[1][threadIdx.x], sh[1][threadIdx.x + o]);
-            sh[2][threadIdx.x] = nan_max(sh[2][threadIdx.x], sh[2][threadIdx.x + o]);
-            sh[3][threadIdx.x] = nan_max(sh[3][threadIdx.x], sh[3][threadIdx.x + o]);
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0)
-        for (int q = 0; q < 4; q++) bbox_all[4 * g + q] = sh[q][0];
-}
-
-// Boundary polygon and boundary edge table of every grid (each grid has
-// 2(nx-1)+2(ny-1) of both).
-__global__ void k_grid_boundary(const GridDesc* __restrict__ grids,
-                                const int64_t* __restrict__ e_prefix, int ngrids,
-                                int64_t ne_all, double* __restrict__ bpx,
-                                double* __restrict__ bpy, double* __restrict__ be,
-                                int32_t* __restrict__ bcell)
-{
-    const int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (e >= ne_all) return;
-    const GridDesc& G = grids[seg_of(e_prefix, ngrids, e)];
-    const int64_t le = e - G.e_base;
-    const int64_t v = boundary_vertex(G.nx, G.ny, le);
-    bpx[e] = G.x[v];
-    bpy[e] = G.y[v];
-    boundary_edge(G.x, G.y, G.nx, G.ny, le, be + 4 * e, bcell + e);
-}
-
-// The y range of the vertices of each run of 64 boundary-polygon edges
-// (edge k runs from vertex k - 1 to vertex k, edge 0 from the last vertex):
-// a run whose range excludes a point's y adds nothing to its winding number.
-__global__ void k_grid_poly_yranges(const GridDesc* __restrict__ grids,
-                                    const int64_t* __restrict__ pyr_prefix, int ngrids,
-                                    int64_t npyr_all, const double* __restrict__ bpy_all,
-                                    double2* __restrict__ pyr)
-{
-    // one wavefront per run, one lane per edge
-    const int64_t b = grid_wave();
-    const int lane = threadIdx.x & 63;
-    if (b >= npyr_all) return;  // uniform per wavefront
-    const GridDesc& G = grids[seg_of(pyr_prefix, ngrids, b)];
-    const int64_t nbp = 2 * (G.nx - 1) + 2 * (G.ny - 1);
-    const int64_t k = (b - G.pyr_base) * 64 + lane;
-    const double* bpy = bpy_all + G.e_base;
-    double lo = __builtin_huge_val(), hi = -__builtin_huge_val();
-    if (k < nbp) {
-        const int64_t km = k == 0 ? nbp - 1 : k - 1;
-        // fmin/fmax ignore NaN; an edge with a NaN end adds nothing
-        lo = fmin(bpy[km], bpy[k]);
-        hi = fmax(bpy[km], bpy[k]);
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        lo = fmin(lo, __shfl_xor(lo, o, 64));
-        hi = fmax(hi, __shfl_xor(hi, o, 64));
-    }
-    if (lane == 0) pyr[b] = make_double2(lo, hi);
-}
-
-__global__ void k_grid_edge_boxes(const GridDesc* __restrict__ grids,
-                                  const int64_t* __restrict__ blk_prefix,
-                                  int ngrids, int64_t nblk_all,
-                                  const double* __restrict__ be_all,
-                                  Box* __restrict__ bblk)
-{
-    const int64_t b = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (b >= nblk_all) return;
-    const GridDesc& G = grids[seg_of(blk_prefix, ngrids, b)];
-    const int64_t nbe = 2 * (G.nx - 1) + 2 * (G.ny - 1);
-    const int64_t lb = b - G.blk_base;
-    const double* be = be_all + 4 * G.e_base;
-    Box r;
-    r.x0 = r.y0 = __builtin_huge_val();
-    r.x1 = r.y1 = -__builtin_huge_val();
-    const int64_t e1 = (lb + 1) * BND_BLOCK < nbe ? (lb + 1) * BND_BLOCK : nbe;
-    for (int64_t e = lb * BND_BLOCK; e < e1; e++) {
-        const double* q = be + 4 * e;
-        // fmin/fmax ignore NaN; an edge with a NaN end never hits anyway
-        r.x0 = fmin(r.x0, fmin(q[0], q[2]));
-        r.x1 = fmax(r.x1, fmax(q[0], q[2]));
-        r.y0 = fmin(r.y0, fmin(q[1], q[3]));
-        r.y1 = fmax(r.y1, fmax(q[1], q[3]));
-    }
-    bblk[b] = r;
-}
-
-__global__ void k_grid_super_boxes(const GridDesc* __restrict__ grids,
-                                   const int64_t* __restrict__ sup_prefix,
-                                   int ngrids, int64_t nsup_all,
-                                   const Box* __restrict__ bblk_all,
-                                   Box* __restrict__ bsup)
-{
-    const int64_t sidx = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (sidx >= nsup_all) return;
-    const GridDesc& G = grids[seg_of(sup_prefix, ngrids, sidx)];
-    const int64_t nbe = 2 * (G.nx - 1) + 2 * (G.ny - 1);
-    const int64_t nblk = (nbe + BND_BLOCK - 1) / BND_BLOCK;
-    const int64_t ls = sidx - G.sup_base;
-    const Box* bblk = bblk_all + G.blk_base;
-    Box r;
-    r.x0 = r.y0 = __builtin_huge_val();
-    r.x1 = r.y1 = -__builtin_huge_val();
-    const int64_t b1 = (ls + 1) * BND_SUPER < nblk ? (ls + 1) * BND_SUPER : nblk;
-    for (int64_t b = ls * BND_SUPER; b < b1; b++) {
-        r.x0 = fmin(r.x0, bblk[b].x0);
-        r.y0 = fmin(r.y0, bblk[b].y0);
-        r.x1 = fmax(r.x1, bblk[b].x1);
-        r.y1 = fmax(r.y1, bblk[b].y1);
-    }
-    bsup[sidx] = r;
-}
-
-// One thread per grid: the box of all its boundary edges (NaN ends ignored,
-// as in the block boxes) -- a sweep edge that misses it misses every block.
-__global__ void k_grid_boundary_box(const int64_t* __restrict__ sup_prefix, int ngrids,
-                                    const Box* __restrict__ bsup, Box* __restrict__ ball)
-{
-    const int g = blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= ngrids) return;
-    Box r;
-    r.x0 = r.y0 = __builtin_huge_val();
-    r.x1 = r.y1 = -__builtin_huge_val();
-    for (int64_t q = sup_prefix[g]; q < sup_prefix[g + 1]; q++) {
-        r.x0 = fmin(r.x0, bsup[q].x0);
-        r.y0 = fmin(r.y0, bsup[q].y0);
-        r.x1 = fmax(r.x1, bsup[q].x1);
-        r.y1 = fmax(r.y1, bsup[q].y1);
-    }
-    ball[g] = r;
-}
-
-// Input cell areas (and the input weighting, 1 where a pair has none) over
-// the padded global cell space; padding cells get area 1 and weight 1 (they
+// Input cell area (and the input weighting, 1 where a pair has none) of cell c
+// of the padded global cell space; padding cells get area 1 and weight 1 (they
 // receive no triples).
-__global__ void k_pair_cells(const PairCells* __restrict__ pcs,
-                             const int32_t* __restrict__ pair_of_group,
-                             int64_t ncells_all, double* __restrict__ vol,
-                             double* __restrict__ wi_all)
+__device__ inline void pair_cell(const PairCells* __restrict__ pcs,
+                                 const int32_t* __restrict__ pair_of_group, int64_t c,
+                                 double* __restrict__ vol, double* __restrict__ wi_all)
 {
-    const int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (c >= ncells_all) return;
     const PairCells& P = pcs[pair_of_group[c >> 6]];
     const int64_t lc = c - P.cell_gbase;
     double a = 1, w = 1;
@@ -451,6 +317,149 @@ __global__ void k_pair_cells(const PairCells* __restrict__ pcs,
     if (wi_all) wi_all[c] = w;
 }
 
+__device__ inline Box empty_box()
+{
+    Box r;
+    r.x0 = r.y0 = __builtin_huge_val();
+    r.x1 = r.y1 = -__builtin_huge_val();
+    return r;
+}
+
+// (fmin/fmax ignore NaN; an edge with a NaN end never hits anyway)
+__device__ inline void grow_box(Box& r, const Box& b)
+{
+    r.x0 = fmin(r.x0, b.x0);
+    r.y0 = fmin(r.y0, b.y0);
+    r.x1 = fmax(r.x1, b.x1);
+    r.y1 = fmax(r.y1, b.y1);
+}
+
+__device__ inline void grow_box_from_lane(Box& r, int o)
+{
+    Box b;
+    b.x0 = __shfl_xor(r.x0, o, 64);
+    b.y0 = __shfl_xor(r.y0, o, 64);
+    b.x1 = __shfl_xor(r.x1, o, 64);
+    b.y1 = __shfl_xor(r.y1, o, 64);
+    grow_box(r, b);
+}
+
+// One block per super-block of boundary edges, a thread for each edge: the
+// boundary polygon and edge table of every grid (each grid has 2(nx-1)+2(ny-1)
+// of both), the boxes of the edge blocks and super-blocks, and the y range of
+// the vertices of each run of 64 boundary-polygon edges (edge k runs from
+// vertex k - 1 to vertex k, edge 0 from the last vertex): a run whose range
+// excludes a point's y adds nothing to its winding number.  The blocks past
+// the super-blocks compute the input cells' areas, a thread for each cell.
+constexpr int EDGE_THREADS = BND_BLOCK * BND_SUPER;
+static_assert(EDGE_THREADS % 64 == 0 && 64 % BND_BLOCK == 0, "whole wavefronts of whole blocks");
+
+struct EdgeTables {
+    double *bpx, *bpy, *be;
+    int32_t* bcell;
+    Box *bblk, *bsup;
+    double2* pyr;
+};
+
+__global__ __launch_bounds__(EDGE_THREADS) void k_prepare_grids(
+    const GridDesc* __restrict__ grids, const int64_t* __restrict__ sup_prefix, int ngrids,
+    int64_t nsup_all, EdgeTables E, const PairCells* __restrict__ pcs,
+    const int32_t* __restrict__ pair_of_group, int64_t ncells_all, double* __restrict__ vol,
+    double* __restrict__ wi_all)
+{
+    const int64_t sup = blockIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63;
+    if (sup >= nsup_all) {
+        const int64_t c = (sup - nsup_all) * EDGE_THREADS + tid;
+        if (c < ncells_all) pair_cell(pcs, pair_of_group, c, vol, wi_all);
+        return;
+    }
+    const GridDesc& G = grids[seg_of(sup_prefix, ngrids, sup)];
+    const int64_t nbe = 2 * (G.nx - 1) + 2 * (G.ny - 1);
+    const int64_t le = (sup - G.sup_base) * EDGE_THREADS + tid, e = G.e_base + le;
+    Box r = empty_box();
+    double lo = __builtin_huge_val(), hi = -__builtin_huge_val();
+    if (le < nbe) {
+        const int64_t v = boundary_vertex(G.nx, G.ny, le);
+        const double py = G.y[v];
+        E.bpx[e] = G.x[v];
+        E.bpy[e] = py;
+        // (an edge with a NaN end adds nothing to a winding number either)
+        const double pm = G.y[boundary_vertex(G.nx, G.ny, le == 0 ? nbe - 1 : le - 1)];
+        lo = fmin(pm, py);
+        hi = fmax(pm, py);
+        double q[4];
+        int32_t cell;
+        boundary_edge(G.x, G.y, G.nx, G.ny, le, q, &cell);
+#pragma unroll
+        for (int u = 0; u < 4; u++) E.be[4 * e + u] = q[u];
+        E.bcell[e] = cell;
+        r.x0 = fmin(q[0], q[2]);
+        r.x1 = fmax(q[0], q[2]);
+        r.y0 = fmin(q[1], q[3]);
+        r.y1 = fmax(q[1], q[3]);
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        lo = fmin(lo, __shfl_xor(lo, o, 64));
+        hi = fmax(hi, __shfl_xor(hi, o, 64));
+    }
+    if (lane == 0 && le < nbe) E.pyr[G.pyr_base + le / 64] = make_double2(lo, hi);
+#pragma unroll
+    for (int o = 1; o < BND_BLOCK; o <<= 1) grow_box_from_lane(r, o);
+    if (tid % BND_BLOCK == 0 && le < nbe) E.bblk[G.blk_base + le / BND_BLOCK] = r;
+#pragma unroll
+    for (int o = BND_BLOCK; o < 64; o <<= 1) grow_box_from_lane(r, o);
+    __shared__ Box wave_box[EDGE_THREADS / 64];
+    if (lane == 0) wave_box[tid / 64] = r;
+    __syncthreads();
+    if (tid == 0) {
+        for (int w = 1; w < EDGE_THREADS / 64; w++) grow_box(r, wave_box[w]);
+        E.bsup[sup] = r;
+    }
+}
+
+// One block per grid: the bounding box from its tiles' partial boxes, and the
+// box of all its boundary edges (NaN ends ignored, as in the block boxes) -- a
+// sweep edge that misses it misses every block.
+__global__ __launch_bounds__(BBOX_BLOCK) void k_grid_boxes(
+    const int64_t* __restrict__ tile_prefix, const double* __restrict__ part,
+    double* __restrict__ bbox_all, const int64_t* __restrict__ sup_prefix,
+    const Box* __restrict__ bsup, Box* __restrict__ ball)
+{
+    const int g = blockIdx.x;
+    const int64_t t0 = tile_prefix[g], t1 = tile_prefix[g + 1];
+    double v[4] = {part[4 * t0], part[4 * t0 + 1], part[4 * t0 + 2], part[4 * t0 + 3]};
+    for (int64_t t = t0 + threadIdx.x; t < t1; t += BBOX_BLOCK) {
+        v[0] = nan_min(v[0], part[4 * t + 0]);
+        v[1] = nan_min(v[1], part[4 * t + 1]);
+        v[2] = nan_max(v[2], part[4 * t + 2]);
+        v[3] = nan_max(v[3], part[4 * t + 3]);
+    }
+    Box r = empty_box();
+    for (int64_t q = sup_prefix[g] + threadIdx.x; q < sup_prefix[g + 1]; q += BBOX_BLOCK)
+        grow_box(r, bsup[q]);
+    __shared__ double sh[4][BBOX_BLOCK];
+    __shared__ Box box[BBOX_BLOCK];
+    for (int q = 0; q < 4; q++) sh[q][threadIdx.x] = v[q];
+    box[threadIdx.x] = r;
+    __syncthreads();
+    for (int o = BBOX_BLOCK / 2; o > 0; o >>= 1) {
+        if ((int)threadIdx.x < o) {
+            sh[0][threadIdx.x] = nan_min(sh[0][threadIdx.x], sh[0][threadIdx.x + o]);
+            sh[1][threadIdx.x] = nan_min(sh[1][threadIdx.x], sh[1][threadIdx.x + o]);
+            sh[2][threadIdx.x] = nan_max(sh[2][threadIdx.x], sh[2][threadIdx.x + o]);
+            sh[3][threadIdx.x] = nan_max(sh[3][threadIdx.x], sh[3][threadIdx.x + o]);
+            grow_box(box[threadIdx.x], box[threadIdx.x + o]);
+        }
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+        for (int q = 0; q < 4; q++) bbox_all[4 * g + q] = sh[q][0];
+        ball[g] = box[0];
+    }
+}
+
 // ---- start states --------------------------------------------------------
 
 // Row start of the reference (:293-322) for rows_per_wave rows per
@@ -461,13 +470,13 @@ __global__ void k_pair_cells(const PairCells* __restrict__ pcs,
 // puts one row per wavefront while the rows alone do not fill the GPU, and
 // more when they do: a wavefront per row ran each secant search on one lane
 // (the 256-pair batch's build, about a million rows: 20.24 -> 20.04 ms).
-__global__ void k_row_start(const Build* __restrict__ builds,
-                            const int32_t* __restrict__ pair_of_row,
-                            int64_t nrows_all, int32_t* __restrict__ start,
-                            int32_t* __restrict__ anomalies, int rows_per_wave)
+__device__ inline void row_starts(const Build* __restrict__ builds,
+                                  const int32_t* __restrict__ pair_of_row, int64_t wave,
+                                  int64_t nrows_all, int32_t* __restrict__ start,
+                                  int32_t* __restrict__ anomalies, int rows_per_wave)
 {
     const int R = rows_per_wave;  // 1..64, a power of two
-    const int64_t r0 = grid_wave() * R;
+    const int64_t r0 = wave * R;
     const int lane = threadIdx.x & 63;
     if (r0 >= nrows_all) return;  // uniform per wavefront
     // lane j < R owns row r0 + j
@@ -577,12 +586,11 @@ __device__ inline const Pass& pass_of_wave(const Build& B, const ChunkRef& r)
     return B.pass[__builtin_amdgcn_readfirstlane(r.p)];
 }
 
-__global__ __launch_bounds__(WALK_MAX_BLOCK) void k_chunk_start(const Build* __restrict__ builds,
-                              const int32_t* __restrict__ pair_of_wave,
-                              int64_t nthreads_all, int32_t* __restrict__ start,
-                              int guess_outside)
+__device__ inline void chunk_starts(const Build* __restrict__ builds,
+                                    const int32_t* __restrict__ pair_of_wave, int64_t t,
+                                    int64_t nthreads_all, int32_t* __restrict__ start,
+                                    int guess_outside)
 {
-    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (t >= nthreads_all) return;
     const Build& B = build_of_thread(builds, pair_of_wave, t);
     const ChunkRef r = chunk_of_thread(B, t - B.thread_gbase);
@@ -592,6 +600,24 @@ __global__ __launch_bounds__(WALK_MAX_BLOCK) void k_chunk_start(const Build* __r
             const Pass& P = pass_of_wave(B, r);
             return chunk_start_guess(P, r.row, r.c * P.K);
         }();
+}
+
+// The starts of all chunks: row_blocks blocks for the rows' first chunks, the
+// others a thread for each walk thread.
+constexpr int START_BLOCK = 256;
+
+__global__ __launch_bounds__(START_BLOCK) void k_starts(
+    const Build* __restrict__ builds, const int32_t* __restrict__ pair_of_row, int64_t nrows_all,
+    int rows_per_wave, int64_t row_blocks, const int32_t* __restrict__ pair_of_wave,
+    int64_t nthreads_all, int guess_outside, int32_t* __restrict__ start,
+    int32_t* __restrict__ anomalies)
+{
+    if (blockIdx.x < row_blocks)
+        row_starts(builds, pair_of_row, grid_wave(), nrows_all, start, anomalies, rows_per_wave);
+    else
+        chunk_starts(builds, pair_of_wave,
+                     ((int64_t)blockIdx.x - row_blocks) * START_BLOCK + threadIdx.x, nthreads_all,
+                     start, guess_outside);
 }
 
 // ---- walks ---------------------------------------------------------------
@@ -685,10 +711,13 @@ __global__ __launch_bounds__(WALK_MAX_BLOCK) void k_fixup(const Build* __restric
 }
 
 // Triples beyond the staging capacity, per chunk (then scanned into the
-// chunks' ranges of the overflow buffer).
-__global__ void k_overflow_counts(const int32_t* __restrict__ count, int64_t nchunks,
-                                  int64_t cap, int32_t* __restrict__ ov,
-                                  unsigned long long* __restrict__ total)
+// chunks' ranges of the overflow buffer), and the bucket cursors' first
+// values.
+__global__ void k_prepare_emit(const int32_t* __restrict__ count, int64_t nchunks,
+                               int64_t cap, int32_t* __restrict__ ov,
+                               unsigned long long* __restrict__ total,
+                               const int64_t* __restrict__ bucket_off,
+                               uint32_t* __restrict__ cursor, int64_t nb)
 {
     const int64_t g = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     int64_t v = 0;
@@ -696,6 +725,7 @@ __global__ void k_overflow_counts(const int32_t* __restrict__ count, int64_t nch
         v = count[g] > cap ? count[g] - cap : 0;
         ov[g] = (int32_t)v;
     }
+    if (g < nb) cursor[g] = (uint32_t)bucket_off[g];
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
     if ((threadIdx.x & 63) == 0 && v) atomicAdd(total, (unsigned long long)v);
@@ -1260,11 +1290,15 @@ __device__ inline int reduce_group(const RedArgs& A, CellSlots<N>& S, int64_t gr
 // plain loads of this form reach) and the ranks' atomics.
 __global__ __launch_bounds__(64, 3) void k_reduce_cells(RedArgs A, int64_t n_groups,
                                                       int64_t red_cap,
-                                                      int32_t* __restrict__ cap_flag)
+                                                      int32_t* __restrict__ cap_flag,
+                                                      const uint32_t* __restrict__ cursor,
+                                                      int32_t* __restrict__ mismatch)
 {
     __shared__ CellSlots<CELLS_N> S;
     const int lane = threadIdx.x & 63;
     const int64_t grp = blockIdx.x;
+    if (lane < 4 && (int64_t)cursor[4 * grp + lane] != A.bucket_off[4 * grp + lane + 1])
+        atomicAdd(mismatch, 1);
     const int64_t base = A.bucket_off[4 * grp], end = A.bucket_off[4 * grp + 4];
     if (grp == 0 && lane == 0) A.cell_off[n_groups * 64] = A.bucket_off[4 * n_groups];
     if (end > red_cap) {
@@ -1848,15 +1882,6 @@ KeyBits key_bits(int64_t T, int64_t most_out)
     return k;
 }
 
-int launch_segments(const int64_t* prefix, int n, int64_t nunits, int32_t* out,
-                    hipStream_t s)
-{
-    if (nunits == 0) return RG_OK;
-    k_segments<<<grid_for(nunits, 256), 256, 0, s>>>(prefix, n, nunits, out);
-    RG_HIP(hipGetLastError());
-    return RG_OK;
-}
-
 struct PhaseTimer {
     bool on;
     hipStream_t s;
@@ -2297,9 +2322,6 @@ int build_batched(const rg_pair_desc* pairs, int64_t npairs,
     const size_t o_grids = append_table(hb, grids.data(), grids.size());
     const size_t o_pcs = append_table(hb, pcs.data(), pcs.size());
     const size_t o_tile = append_table(hb, tile_pf.data(), tile_pf.size());
-    const size_t o_e = append_table(hb, e_pf.data(), e_pf.size());
-    const size_t o_blk = append_table(hb, blk_pf.data(), blk_pf.size());
-    const size_t o_pyr = append_table(hb, pyr_pf.data(), pyr_pf.size());
     const size_t o_sup = append_table(hb, sup_pf.data(), sup_pf.size());
     const size_t o_wave = append_table(hb, wave_pf.data(), wave_pf.size());
     const size_t o_row = append_table(hb, row_pf.data(), row_pf.size());
@@ -2357,9 +2379,6 @@ int build_batched(const rg_pair_desc* pairs, int64_t npairs,
     const GridDesc* d_grids = (const GridDesc*)(meta.p + o_grids);
     const PairCells* d_pcs = (const PairCells*)(meta.p + o_pcs);
     const int64_t* d_tile = (const int64_t*)(meta.p + o_tile);
-    const int64_t* d_e = (const int64_t*)(meta.p + o_e);
-    const int64_t* d_blk = (const int64_t*)(meta.p + o_blk);
-    const int64_t* d_pyr = (const int64_t*)(meta.p + o_pyr);
     const int64_t* d_sup = (const int64_t*)(meta.p + o_sup);
 
     // ---- prepare
@@ -2368,69 +2387,57 @@ int build_batched(const rg_pair_desc* pairs, int64_t npairs,
     RG_TRY(pair_of_row.alloc(row_tot, s));
     RG_TRY(pair_of_ing.alloc(cell_tot / 64, s));
     RG_TRY(pair_of_outg.alloc(out_tot / 64, s));
-    const int np32 = (int)npairs;
-    RG_TRY(launch_segments((const int64_t*)(meta.p + o_wave), np32, thr_tot / 64,
-                           pair_of_wave.p, s));
-    RG_TRY(launch_segments((const int64_t*)(meta.p + o_row), np32, row_tot,
-                           pair_of_row.p, s));
-    RG_TRY(launch_segments((const int64_t*)(meta.p + o_ing), np32, cell_tot / 64,
-                           pair_of_ing.p, s));
-    RG_TRY(launch_segments((const int64_t*)(meta.p + o_outg), np32, out_tot / 64,
-                           pair_of_outg.p, s));
-    k_grid_tiles<<<(unsigned)tile_tot, BBOX_BLOCK, 0, s>>>(d_grids, d_tile, ng,
-                                                            xy_all.p, part.p);
-    RG_HIP(hipGetLastError());
-    k_grid_bbox<<<(unsigned)ng, BBOX_BLOCK, 0, s>>>(d_tile, part.p, bbox_all.p);
-    RG_HIP(hipGetLastError());
-    k_grid_boundary<<<grid_for(e_tot, 256), 256, 0, s>>>(d_grids, d_e, ng, e_tot,
-                                                         bpx.p, bpy.p, be.p, bcell.p);
-    RG_HIP(hipGetLastError());
-    k_grid_edge_boxes<<<grid_for(blk_tot, 256), 256, 0, s>>>(d_grids, d_blk, ng,
-                                                             blk_tot, be.p, bblk.p);
-    RG_HIP(hipGetLastError());
-    k_grid_poly_yranges<<<grid_for(pyr_tot * 64, 256), 256, 0, s>>>(d_grids, d_pyr, ng,
-                                                                    pyr_tot, bpy.p, pyr.p);
-    RG_HIP(hipGetLastError());
-    k_grid_super_boxes<<<grid_for(sup_tot, 256), 256, 0, s>>>(d_grids, d_sup, ng,
-                                                              sup_tot, bblk.p, bsup.p);
-    RG_HIP(hipGetLastError());
-    k_grid_boundary_box<<<grid_for(ng, 64), 64, 0, s>>>(d_sup, ng, bsup.p, ball.p);
-    RG_HIP(hipGetLastError());
-    DevBuf<double> vol, wi_all;
-    RG_TRY(vol.alloc(cell_tot, s));
-    if (any_wi) RG_TRY(wi_all.alloc(cell_tot, s));
-    k_pair_cells<<<grid_for(cell_tot, 256), 256, 0, s>>>(d_pcs, pair_of_ing.p,
-                                                         cell_tot, vol.p, wi_all.p);
-    RG_HIP(hipGetLastError());
-    tm.mark();  // 1
-
-    // ---- start states
     const int64_t n_groups = cell_tot / 64;  // every pair's cells padded to 64
     if (4 * n_groups >= INT32_MAX) return fail(RG_ERR_ARGUMENT, "too many input cells in one build");
-    DevBuf<int32_t> start, end, count, hist, counters;
-    RG_TRY(start.alloc(chunk_tot, s));
-    RG_TRY(end.alloc(chunk_tot, s));
-    RG_TRY(count.alloc(chunk_tot, s));
-    RG_TRY(hist.alloc(4 * n_groups, s));
     // anomalies, fixups, failed/overflow, long runs, restaged chunks, heavy
     // groups; words 6-7: the triples beyond the staging capacity (64-bit);
     // word 8: capacity bits of a capacity-mode build; words 10-11: the counts
     // of the reduction's two lists
+    DevBuf<int32_t> hist, counters, hist_out;
+    RG_TRY(hist.alloc(4 * n_groups, s));
     RG_TRY(counters.alloc(12, s));
-    RG_TRY(fill_zero(hist.p, 4 * n_groups, s));
-    RG_TRY(fill_zero(counters.p, 12, s));
+    // entries per output row (the reductions also keep each entry's rank)
+    RG_TRY(hist_out.alloc(out_tot, s));
+    const TableFill fills = {
+        {(const int64_t*)(meta.p + o_wave), (const int64_t*)(meta.p + o_row),
+         (const int64_t*)(meta.p + o_ing), (const int64_t*)(meta.p + o_outg)},
+        {pair_of_wave.p, pair_of_row.p, pair_of_ing.p, pair_of_outg.p},
+        {thr_tot / 64, row_tot, cell_tot / 64, out_tot / 64},
+        {hist.p, counters.p, hist_out.p},
+        {4 * n_groups, 12, out_tot},
+        (int)npairs};
+    k_prepare_vertices<<<(unsigned)(tile_tot + grid_for(fills.items(), BBOX_BLOCK)), BBOX_BLOCK, 0,
+                         s>>>(d_grids, d_tile, ng, tile_tot, xy_all.p, part.p, fills);
+    RG_HIP(hipGetLastError());
+    DevBuf<double> vol, wi_all;
+    RG_TRY(vol.alloc(cell_tot, s));
+    if (any_wi) RG_TRY(wi_all.alloc(cell_tot, s));
+    const EdgeTables edges = {bpx.p, bpy.p, be.p, bcell.p, bblk.p, bsup.p, pyr.p};
+    k_prepare_grids<<<(unsigned)(sup_tot + grid_for(cell_tot, EDGE_THREADS)), EDGE_THREADS, 0,
+                      s>>>(d_grids, d_sup, ng, sup_tot, edges, d_pcs, pair_of_ing.p, cell_tot,
+                           vol.p, wi_all.p);
+    RG_HIP(hipGetLastError());
+    k_grid_boxes<<<(unsigned)ng, BBOX_BLOCK, 0, s>>>(d_tile, part.p, bbox_all.p, d_sup, bsup.p,
+                                                     ball.p);
+    RG_HIP(hipGetLastError());
+    tm.mark();  // 1
+
+    // ---- start states
+    DevBuf<int32_t> start, end, count;
+    RG_TRY(start.alloc(chunk_tot, s));
+    RG_TRY(end.alloc(chunk_tot, s));
+    RG_TRY(count.alloc(chunk_tot, s));
     {
         // rows per wavefront: one until the rows fill about 4096 wavefronts
         int rpw = 1;
         while (rpw < 64 && row_tot / (2 * rpw) >= 4096) rpw *= 2;
         if (flags & RG_TUNE_ROW_WAVES) rpw = 64;
         const int64_t waves = (row_tot + rpw - 1) / rpw;
-        k_row_start<<<grid_for(waves * 64, 256), 256, 0, s>>>(d_builds, pair_of_row.p, row_tot,
-                                                              start.p, counters.p + 0, rpw);
+        const int64_t row_blocks = grid_for(waves * 64, START_BLOCK);
+        k_starts<<<(unsigned)(row_blocks + grid_for(thr_tot, START_BLOCK)), START_BLOCK, 0, s>>>(
+            d_builds, pair_of_row.p, row_tot, rpw, row_blocks, pair_of_wave.p, thr_tot,
+            (flags & RG_TUNE_GUESS_OUTSIDE) != 0, start.p, counters.p + 0);
     }
-    RG_HIP(hipGetLastError());
-    k_chunk_start<<<grid_for(thr_tot, block), block, 0, s>>>(
-        d_builds, pair_of_wave.p, thr_tot, start.p, (flags & RG_TUNE_GUESS_OUTSIDE) != 0);
     RG_HIP(hipGetLastError());
     tm.mark();  // 2
 
@@ -2457,8 +2464,10 @@ int build_batched(const rg_pair_desc* pairs, int64_t npairs,
     // triples beyond the staging capacity, per chunk and in all
     DevBuf<int32_t> ov;
     RG_TRY(ov.alloc(chunk_tot, s));
-    k_overflow_counts<<<grid_for(chunk_tot, 256), 256, 0, s>>>(
-        count.p, chunk_tot, cap, ov.p, (unsigned long long*)(counters.p + 6));
+    uint32_t* cursor = (uint32_t*)hist.p;  // reused: one word per bucket
+    k_prepare_emit<<<grid_for(std::max(chunk_tot, 4 * n_groups), 256), 256, 0, s>>>(
+        count.p, chunk_tot, cap, ov.p, (unsigned long long*)(counters.p + 6), bucket_off.p,
+        cursor, 4 * n_groups);
     RG_HIP(hipGetLastError());
     int64_t tot[2];
     int32_t cnt[8] = {};
@@ -2506,9 +2515,6 @@ int build_batched(const rg_pair_desc* pairs, int64_t npairs,
     DevBuf<uint8_t> rcell;
     RG_TRY(rec.alloc(T, s));
     RG_TRY(rcell.alloc(T, s));
-    uint32_t* cursor = (uint32_t*)hist.p;  // reused: one word per bucket
-    k_cursor_init<<<grid_for(4 * n_groups, 256), 256, 0, s>>>(bucket_off.p, cursor,
-                                                              4 * n_groups);
     tm.mark();  // 5
     DevBuf<Triple> ovbuf;
     DevBuf<int64_t> ov_off;
@@ -2528,9 +2534,6 @@ int build_batched(const rg_pair_desc* pairs, int64_t npairs,
         ov_off.p, ov_tot, chunk_off.p, cursor, rec.p, rcell.p, (uint32_t)T, counters.p + 2);
     RG_HIP(hipGetLastError());
     tm.mark();  // 6
-    k_cursor_check<<<grid_for(4 * n_groups, 256), 256, 0, s>>>(
-        bucket_off.p, cursor, 4 * n_groups, counters.p + 2);
-    RG_HIP(hipGetLastError());
     stage.reset();
 
     // ---- reduce -> CSR by input
@@ -2544,11 +2547,8 @@ int build_batched(const rg_pair_desc* pairs, int64_t npairs,
     RG_TRY(cell_off.alloc(cell_tot + 1, s));
     RG_TRY(red.alloc(T, s));
     tm.mark();  // 7
-    DevBuf<int32_t> heavy_list, hist_out;
+    DevBuf<int32_t> heavy_list;
     RG_TRY(heavy_list.alloc(n_groups, s));
-    // entries per output row (the reductions also keep each entry's rank)
-    RG_TRY(hist_out.alloc(out_tot, s));
-    RG_TRY(fill_zero(hist_out.p, out_tot, s));
     int64_t most_out = 1;
     for (int64_t k = 0; k < npairs; k++) most_out = std::max(most_out, pcs[k].n_out);
     const RedArgs red_args = {bucket_off.p, rec.p,        rcell.p, red.p,         cell_off.p,
@@ -2559,7 +2559,8 @@ int build_batched(const rg_pair_desc* pairs, int64_t npairs,
     DevBuf<int32_t> list1, list2;
     RG_TRY(list1.alloc(n_groups, s));
     RG_TRY(list2.alloc(n_groups, s));
-    k_reduce_cells<<<(unsigned)n_groups, 64, 0, s>>>(red_args, n_groups, T, counters.p + 8);
+    k_reduce_cells<<<(unsigned)n_groups, 64, 0, s>>>(red_args, n_groups, T, counters.p + 8,
+                                                   cursor, counters.p + 2);
     k_list_groups<<<grid_for(n_groups, LIST_BLOCK), LIST_BLOCK, 0, s>>>(
         group_mode.p, n_groups, list1.p, counters.p + 10, list2.p, counters.p + 11, heavy_list.p,
         counters.p + 5);
