@@ -26,11 +26,12 @@
 // round-robin) sweeps one contiguous band of tiles, keeping the patches of
 // neighbouring tiles in that XCD's L2.
 //
-// The results are stored nontemporal: each is written once and not read
-// back by the launch, so written through the caches they would only evict
-// the input patches that neighbouring tiles share (at 2049^2 -> 1537^2 and
-// 16 images: FP64 0.210 -> 0.205 ms, FP32 0.130 -> 0.123 ms, FP64 adjoint
-// 0.256 -> 0.248 ms, FP32 adjoint 0.148 -> 0.094 ms).
+// The results are stored nontemporal, where a tile's rows end at cache lines or
+// the images are too many to merge there (launch_apply): each is written once
+// and not read back by the launch, so written through the caches they would
+// only evict the input patches that neighbouring tiles share (at 2049^2 ->
+// 1537^2 and 16 images: FP64 0.239 -> 0.232 ms, FP32 0.164 -> 0.150 ms, FP64
+// adjoint 0.301 -> 0.286 ms, FP32 adjoint 0.212 -> 0.115 ms).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -50,6 +51,17 @@ struct ApplyGrid {
     int64_t tw, th;       // tile shape (tw * th = APPLY_BLOCK)
     int64_t ntx, ntiles;  // tiles along gy, tiles in total
 };
+
+// Stores a result: nontemporal, or (MERGE) through the caches.  (A template,
+// since the compiler joins the two stores of a branch into an ordinary one.)
+template <bool MERGE, class T>
+__device__ inline void store_result(T* y, T v)
+{
+    if constexpr (MERGE)
+        *y = v;
+    else
+        __builtin_nontemporal_store(v, y);
+}
 
 // ---- the apply without a plan ----------------------------------------------
 //
@@ -80,11 +92,12 @@ constexpr int64_t SPLIT_TILES = 1024;
 // Entries [c0, c0 + 64 * U) of the wavefront's `total` for `images` images:
 // the products go to LDS in entry order, and each lane adds up those of its
 // row, entries [s, e), to y (from 0 where c0 is 0).
-template <class T, int U>
+template <bool MERGE, class T, int U>
 __device__ inline void apply_entries(const int32_t* __restrict__ col, const T* __restrict__ w,
                                      const T* __restrict__ x, T* __restrict__ y, int64_t nrows,
                                      int64_t ncols, int32_t images, int32_t c0, int32_t total,
-                                     int32_t s, int32_t e, bool has_row, T* __restrict__ prod)
+                                     int32_t s, int32_t e, bool has_row,
+                                     T* __restrict__ prod)
 {
     const int32_t lane = threadIdx.x & 63;
     uint32_t c[U];
@@ -119,7 +132,7 @@ __device__ inline void apply_entries(const int32_t* __restrict__ col, const T* _
 #pragma unroll
                 for (int u = 0; u < 4; u++) acc = acc + p[u];
             }
-            __builtin_nontemporal_store(acc, y);
+            store_result<MERGE>(y, acc);
         }
         y += nrows;
     }
@@ -128,7 +141,7 @@ __device__ inline void apply_entries(const int32_t* __restrict__ col, const T* _
 // Applies the CSR to one tile and `images` images, a wavefront for each 64
 // consecutive rows and by itself.  A tile is 64 columns of APPLY_BLOCK / 64
 // grid rows at (ib, jb) or, if `flat`, APPLY_BLOCK rows of one long row.
-template <class T>
+template <bool MERGE, class T>
 __device__ inline void apply_rows(const int32_t* __restrict__ rowptr,
                                   const int32_t* __restrict__ col, const T* __restrict__ w,
                                   const T* __restrict__ x, T* __restrict__ y, int64_t nrows,
@@ -161,15 +174,15 @@ __device__ inline void apply_rows(const int32_t* __restrict__ rowptr,
         return;
     }
     if (total <= 64 * (ENTRIES_U / 2))
-        apply_entries<T, ENTRIES_U / 2>(col, w, x, y, nrows, ncols, images, 0, total, s, e, valid,
+        apply_entries<MERGE, T, ENTRIES_U / 2>(col, w, x, y, nrows, ncols, images, 0, total, s, e, valid,
                                         prod);
     else
         for (int32_t c0 = 0; c0 < total; c0 += 64 * ENTRIES_U)
-            apply_entries<T, ENTRIES_U>(col, w, x, y, nrows, ncols, images, c0, total, s, e,
+            apply_entries<MERGE, T, ENTRIES_U>(col, w, x, y, nrows, ncols, images, c0, total, s, e,
                                         valid, prod);
 }
 
-template <class T>
+template <class T, bool MERGE>
 __global__ __launch_bounds__(APPLY_BLOCK) void k_apply(
     const int32_t* __restrict__ rowptr, const int32_t* __restrict__ col,
     const T* __restrict__ w, const T* __restrict__ x, T* __restrict__ y,
@@ -183,7 +196,7 @@ __global__ __launch_bounds__(APPLY_BLOCK) void k_apply(
     const uint32_t ntx = (uint32_t)G.ntx, ti = tile / ntx, tj = tile % ntx;
     const int64_t d0 = (int64_t)blockIdx.y * db;
     const int64_t nd = batch - d0 < db ? batch - d0 : db;
-    apply_rows<T>(rowptr, col, w, x + d0 * ncols, y + d0 * nrows, nrows, ncols, (int32_t)nd, G.gy,
+    apply_rows<MERGE, T>(rowptr, col, w, x + d0 * ncols, y + d0 * nrows, nrows, ncols, (int32_t)nd, G.gy,
                   ti * G.th, tj * G.tw, G.th == 1, prod[threadIdx.x / 64]);
 }
 
@@ -451,7 +464,7 @@ __global__ __launch_bounds__(APPLY_BLOCK) void k_apply_planned(
     T* yb = y + d0 * nrows + r;
 #pragma unroll
     for (int m = 0; m < DB; m++)
-        if (m < nd) __builtin_nontemporal_store(acc[m], &yb[m * nrows]);
+        if (m < nd) store_result<false>(&yb[m * nrows], acc[m]);
 }
 
 // The planned apply with all images in one block: the lane's CSR entries
@@ -459,7 +472,7 @@ __global__ __launch_bounds__(APPLY_BLOCK) void k_apply_planned(
 // images the block stages the input patch in LDS and gathers from it.  The
 // entries and row pointers are read once per launch instead of once per
 // image group, and the blocks (one per tile) stay resident longer.
-template <class T, int DB, int MAXE>
+template <class T, int DB, int MAXE, bool MERGE>
 __global__ __launch_bounds__(APPLY_BLOCK) void k_apply_rounds(
     const int32_t* __restrict__ rowptr, const int32_t* __restrict__ col,
     const uint16_t* __restrict__ off, const int32_t* __restrict__ box,
@@ -538,7 +551,7 @@ __global__ __launch_bounds__(APPLY_BLOCK) void k_apply_rounds(
             T* yb = y + d0 * nrows + r;
 #pragma unroll
             for (int m = 0; m < DB; m++)
-                if (m < nd) __builtin_nontemporal_store(acc[m], &yb[m * nrows]);
+                if (m < nd) store_result<MERGE>(&yb[m * nrows], acc[m]);
         }
         if (fits) __syncthreads();  // the next group overwrites the patch
     }
@@ -579,19 +592,33 @@ __global__ __launch_bounds__(APPLY_BLOCK) void k_apply_jobs(
     const int64_t ti = tile / ntx, tj = tile % ntx;
     const int64_t d0 = (int64_t)grp * JOB_DB;
     const int64_t nd = J.batch - d0 < JOB_DB ? J.batch - d0 : JOB_DB;
-    apply_rows<T>(J.rowptr, J.col, (const T*)J.w, (const T*)J.x + d0 * J.ncols,
+    apply_rows<false, T>(J.rowptr, J.col, (const T*)J.w, (const T*)J.x + d0 * J.ncols,
                   (T*)J.y + d0 * J.nrows, J.nrows, J.ncols, (int32_t)nd, J.gy, ti * J.th,
                   tj * J.tw, J.th == 1, prod[threadIdx.x / 64]);
 }
 
 namespace {
 
-// Tile width of the FP64 forward apply; 4-byte values and the adjoint use
-// tiles twice as wide (up to APPLY_BLOCK).  Tuned on the plain 2049^2 ->
-// 1537^2 pair, 16 images: FP64 forward 16 wide, FP32 32 wide (0.149 ->
-// 0.129 ms forward, 0.181 -> 0.148 ms adjoint against 16); the FP64 adjoint
-// 32 wide (0.252 -> 0.247 ms against 16; its rows are the input cells, and
-// its patches short runs of output rows).
+// Tile width, and how results are stored (launch_apply).  Where the rows of
+// the output are whole cache lines, tiles are 16 wide and stores nontemporal.
+// Elsewhere a tile's row ends in two lines that the neighbouring tiles also
+// write, and a nontemporal store sends each part to memory by itself: while
+// the images fit the Infinity Cache with room to spare, the parts are stored
+// through the caches, which merge them; beyond that, tiles are two or four
+// times as wide (fewer parts), the less the more input cells there are to an
+// output, as a wider tile's patch leaves fewer images per pass.
+// us, 16 wide nontemporal / 32 wide nontemporal / 16 wide merged, 16 images:
+//   500^2 -> 999^2 FP64 73.8 / 52.6 / 35.0 (160 MB)
+//   1400^2 -> 1000^2 adjoint FP32 123 / 89.7 / 57.7 (189 MB)
+//   1200^2 -> 1200^2 FP32 92.7 / 65.4 / 50.7 (184 MB); FP64 138 / 103 / 133 (369 MB)
+//   1400^2 -> 1000^2 adjoint FP64 176 / 127 / 166 (379 MB); 8 images 76.7 / 59.6 / 72.1
+//   900^2 -> 1537^2 adjoint FP64 190 / 348 / 183; 2049^2 -> 1537^2 (whole
+//   lines) FP64 232 / 285 / 239, adjoint 285 / 321 / 301
+//   1500^2 -> 2000^2 FP64, 3 images - / 60 / 81 (150 MB)
+// and FP32 beyond the limit, 16 / 32 / 64 wide nontemporal: 1500^2 -> 2000^2
+//   - / 183 / 154, 1600^2 -> 1600^2 - / 120 / 168, 1700^2 -> 1200^2 102 / 89 / -
+constexpr int64_t LINE = 128;
+constexpr double MERGE_BYTES_8 = 130e6, MERGE_BYTES_4 = 190e6;
 int g_tile_w = 16;
 int g_images_per_pass = 8;
 // staged patch per block above which fewer images are staged per pass: at
@@ -645,7 +672,7 @@ ApplyGrid gather_grid(const int64_t* shape, int64_t nrows)
 
 // The plan of one direction for the current tile shape (made on first use
 // on stream s; later applies on other streams must be ordered after it).
-int ensure_plan(rg_weights* W, int dir, int64_t value_bytes, const int32_t* rowptr,
+int ensure_plan(rg_weights* W, int dir, int widen, const int32_t* rowptr,
                 const int32_t* col, const ApplyGrid& G, int64_t src_gy,
                 int64_t batch, hipStream_t s, rg_weights::Plan** out)
 {
@@ -658,7 +685,7 @@ int ensure_plan(rg_weights* W, int dir, int64_t value_bytes, const int32_t* rowp
     if (!g_use_plan || batch == 1 || G.gx == 1 || W->nnz == 0 || G.gx * G.gy < PLAN_MIN_ROWS)
         return RG_OK;
     std::lock_guard<std::mutex> lk(g_plan_mu);
-    rg_weights::Plan& P = W->plan[2 * dir + (value_bytes < 8 ? 1 : 0)];
+    rg_weights::Plan& P = W->plan[dir][widen];
     if (P.tile_w != G.tw || P.ntiles != G.ntiles) {
         dev_free(P.box);
         dev_free(P.off);
@@ -688,11 +715,20 @@ int launch_apply(rg_weights* W, int dir, const int32_t* rowptr,
                  int64_t src_gy, int64_t batch, hipStream_t s)
 {
     if (nrows == 0 || batch == 0) return RG_OK;
-    const int64_t tile_w =
-        sizeof(T) >= 8 && dir == 0 ? g_tile_w : std::min(2 * g_tile_w, APPLY_BLOCK);
+    const bool lines = shape[0] * shape[1] == nrows && shape[1] * (int64_t)sizeof(T) % LINE == 0;
+    const bool small = (double)batch * (nrows + ncols) * sizeof(T) <=
+                       (sizeof(T) < 8 ? MERGE_BYTES_4 : MERGE_BYTES_8);
+    const bool merge = !lines && small;
+    int widen = 0;
+    if (!lines && !small) {
+        const double c = (double)ncols / (double)nrows;
+        if (sizeof(T) >= 8) widen = c <= 1.75;
+        else widen = c <= 0.75 ? 2 : c <= 2.2;
+    }
+    const int64_t tile_w = std::min(g_tile_w << widen, APPLY_BLOCK);
     ApplyGrid G = make_grid(shape, nrows, tile_w);
     rg_weights::Plan* P = nullptr;
-    RG_TRY(ensure_plan(W, dir, sizeof(T), rowptr, col, G, src_gy, batch, s, &P));
+    RG_TRY(ensure_plan(W, dir, widen, rowptr, col, G, src_gy, batch, s, &P));
     int32_t sb = 0;
     if (!P) {
         G = gather_grid(shape, nrows);
@@ -711,9 +747,21 @@ int launch_apply(rg_weights* W, int dir, const int32_t* rowptr,
         lds = (lds + 255) / 256 * 256;
         if (lds > LDS_BYTES) lds = LDS_BYTES;
         dim3 g1((unsigned)nb);
-#define RG_ROUNDS(D)                                                                   \
-    k_apply_rounds<T, D, 8><<<g1, bl, (size_t)lds, s>>>(                               \
+        // rows of more than 8 entries would read the rest once per image
+        // group: the adjoint of 1025^2 -> 1500^2 (7.6 a row where there are
+        // any, at most 12), 16 images: FP64 265 -> 195 us, FP32 121 -> 93; at
+        // three or four a row the longer row costs 8 %, at five nothing
+        const bool long_rows = W->nnz >= 5 * nrows;
+#define RG_ROUNDS_K(D, E, M)                                                           \
+    k_apply_rounds<T, D, E, M><<<g1, bl, (size_t)lds, s>>>(                            \
         rowptr, col, P->off, P->box, w, x, y, nrows, ncols, src_gy, batch, G, lds)
+#define RG_ROUNDS(D)                                                                   \
+    do {                                                                               \
+        if (long_rows && merge) RG_ROUNDS_K(D, 12, true);                              \
+        else if (long_rows) RG_ROUNDS_K(D, 12, false);                                 \
+        else if (merge) RG_ROUNDS_K(D, 8, true);                                       \
+        else RG_ROUNDS_K(D, 8, false);                                                 \
+    } while (0)
         switch (db) {
         case 16: RG_ROUNDS(16); break;
         case 8: RG_ROUNDS(8); break;
@@ -722,6 +770,7 @@ int launch_apply(rg_weights* W, int dir, const int32_t* rowptr,
         default: RG_ROUNDS(1); break;
         }
 #undef RG_ROUNDS
+#undef RG_ROUNDS_K
     } else if (P) {
         int64_t lds = P->max_cells * db * (int64_t)sizeof(T);
         lds = (lds + 255) / 256 * 256;
@@ -738,8 +787,11 @@ int launch_apply(rg_weights* W, int dir, const int32_t* rowptr,
         }
 #undef RG_PLANNED
     } else {
-        k_apply<T><<<dim3((unsigned)nb, (unsigned)((batch + sb - 1) / sb)), bl, 0, s>>>(
-            rowptr, col, w, x, y, nrows, ncols, batch, sb, G);
+        const dim3 gs((unsigned)nb, (unsigned)((batch + sb - 1) / sb));
+        if (merge)
+            k_apply<T, true><<<gs, bl, 0, s>>>(rowptr, col, w, x, y, nrows, ncols, batch, sb, G);
+        else
+            k_apply<T, false><<<gs, bl, 0, s>>>(rowptr, col, w, x, y, nrows, ncols, batch, sb, G);
     }
     RG_HIP(hipGetLastError());
     return RG_OK;

@@ -2935,10 +2935,11 @@ void weights_release(rg_weights* W)
     }
     dev_free(W->val_in_f32);
     dev_free(W->val_out_f32);
-    for (auto& pl : W->plan) {
-        dev_free(pl.box);
-        dev_free(pl.off);
-    }
+    for (auto& direction : W->plan)
+        for (auto& pl : direction) {
+            dev_free(pl.box);
+            dev_free(pl.off);
+        }
     delete W;
 }
 
