@@ -160,13 +160,14 @@ struct EmitSink {
 // wait on LDS only: first every 16th vertex in the whole part, then the others
 // between their neighbours'.  The vertices' results are shared between the two
 // cells of a vertex through LDS.  Each pass then moves little more than its
-// arrays: count 2.0 ms -> 31 us, emit 4.4 ms -> 97 us at 2048
+// arrays: count 2.0 ms -> 31 us, emit 4.4 ms -> 85 us at 2048
 // elements of 2049 -> 1537 vertices (7.3 M triples).
 constexpr int LINE_BLOCK = 256;
 constexpr int LINE_CELLS = 1024;
 constexpr int LINE_PER = LINE_CELLS / LINE_BLOCK;  // cells per thread
 constexpr int LINE_COARSE = 16;
-// 16 KiB, with the 4 KiB of results seven blocks per CU; an output grid of up
+// 16 KiB, with the 4 KiB of results seven blocks per CU (five in the emit pass,
+// whose entries take 8 KiB); an output grid of up
 // to this size is staged whole, without a search for the part the block meets
 // (two dependent memory round trips)
 constexpr int LINE_OUT = 2048;
@@ -346,56 +347,76 @@ __global__ __launch_bounds__(LINE_BLOCK) void k_line_count(
     }
 }
 
+// The block's cells hold one range of the entries.  A thread for each entry,
+// LINE_ENTRIES at a time, finds its cell in LDS, so that entries are computed
+// once each whatever their cells' counts (a wavefront of cells took the most
+// of 64, three steps where the mean is 1.7) and each array is written by
+// consecutive threads at consecutive entries, nontemporal: 99 -> 85 us at 2048
+// elements of 2049 -> 1537 vertices (105 us with ordinary stores), of which 30
+// are what the count pass takes too; 3 TB/s.  Entries four at a time or
+// starting at cache lines, and blocks of 512 cells or threads, measure the
+// same.
+constexpr int LINE_ENTRIES = 2 * LINE_CELLS;
+
 __global__ __launch_bounds__(LINE_BLOCK) void k_line_emit(
     const double* __restrict__ xin, int64_t n, const double* __restrict__ xout, int64_t m,
     int64_t nseg, int64_t block0, int32_t* __restrict__ bad, const double* __restrict__ wi,
-    const int64_t* __restrict__ off, const int32_t* __restrict__ cnt,
-    int64_t* __restrict__ ii, int64_t* __restrict__ io, double* __restrict__ w)
+    const int64_t* __restrict__ off, int64_t* __restrict__ ii, int64_t* __restrict__ io,
+    double* __restrict__ w)
 {
     __shared__ LineLds S;
+    __shared__ int32_t first[LINE_CELLS + 1];   // of each cell's entries, in storage order
+    __shared__ uint16_t owner[LINE_ENTRIES];    // cell of each entry
     const LineBlock L(xin, n, xout, m, nseg, block0 + blockIdx.x, bad, S);
     const int64_t row = L.d * (n - 1);
-    // the cells' loads in flight together
-    double xl[LINE_PER], xr[LINE_PER], size[LINE_PER], weight[LINE_PER];
-    int64_t p0[LINE_PER], room[LINE_PER];
+    const int64_t l0 = row + (L.xs.rev ? n - 1 - L.i0 - L.ncell : L.i0);
+    const int64_t e0 = off[l0];
 #pragma unroll
-    for (int t = 0; t < LINE_PER; t++) {
-        const int q = threadIdx.x + t * LINE_BLOCK;
-        room[t] = 0;
-        if (q >= L.ncell) continue;
-        const int64_t i = L.i0 + q, li = L.xs.rev ? n - 2 - i : i;
-        xl[t] = L.xs(i);
-        xr[t] = L.xs(i + 1);
-        // the reference divides by the ascending view's cell at the emitted
-        // (wrapped) index
-        size[t] = L.xs.rev ? L.xs(li + 1) - L.xs(li) : xr[t] - xl[t];
-        weight[t] = wi ? wi[row + li] : 1.0;
-        p0[t] = off[row + li];
-        room[t] = cnt[row + li];
+    for (int t = 0; t <= LINE_PER; t++) {
+        const int j = threadIdx.x + t * LINE_BLOCK;
+        // (more entries than this only in an element out of order, which
+        // sweep_1d writes again)
+        if (j <= L.ncell) first[j] = (int32_t)min(off[l0 + j] - e0, (int64_t)INT32_MAX);
     }
+    __syncthreads();
+    const int32_t total = first[L.ncell];
+    for (int64_t w0 = 0; w0 < total; w0 += LINE_ENTRIES) {
+        const int32_t in_window = (int32_t)min(total - w0, (int64_t)LINE_ENTRIES);
 #pragma unroll
-    for (int t = 0; t < LINE_PER; t++) {
-        const int q = threadIdx.x + t * LINE_BLOCK;
-        if (q >= L.ncell) break;
-        const int64_t i = L.i0 + q;
-        int64_t k0;
-        int64_t c = L.pieces(S, q, m, &k0);
-        // (an element out of order, written again by sweep_1d, stays in its
-        // counted range)
-        if (c > room[t]) c = room[t];
-        if (c == 0) continue;
-        double p1 = L.xt.base + (S.u[q] >> 1) > 0 ? xl[t] : L.xt(0);
-        for (int64_t k = 0; k < c; k++) {
-            const double ps = L.xt(k0 + k + 1);
-            const double p2 = ps < xr[t] ? ps : xr[t];
-            double ratio = (p2 - p1) / size[t];
-            if (wi) ratio = ratio * weight[t];
-            const int64_t p = p0[t] + (L.xt.g.rev ? c - 1 - k : k);
-            ii[p] = L.xs.rev ? ~i : i;
-            io[p] = L.xt.g.rev ? ~(k0 + k) : k0 + k;
-            w[p] = ratio;
-            p1 = p2;
+        for (int t = 0; t < LINE_PER; t++) {
+            const int j = threadIdx.x + t * LINE_BLOCK;
+            if (j >= L.ncell) break;
+            const int32_t a = (int32_t)max(first[j] - w0, (int64_t)0);
+            const int32_t b = (int32_t)min(first[j + 1] - w0, (int64_t)in_window);
+            for (int32_t e = a; e < b; e++) owner[e] = (uint16_t)j;
         }
+        __syncthreads();
+        for (int32_t e = threadIdx.x; e < in_window; e += LINE_BLOCK) {
+            const int j = owner[e], q = L.xs.rev ? L.ncell - 1 - j : j;
+            const int64_t i = L.i0 + q, at = w0 + e - first[j];
+            int64_t k0;
+            int64_t c = L.pieces(S, q, m, &k0);
+            // (an element out of order stays in its counted range)
+            if (c > first[j + 1] - first[j]) c = first[j + 1] - first[j];
+            if (at >= c) continue;
+            const int64_t k = L.xt.g.rev ? c - 1 - at : at;
+            const double xl = L.xs(i), xr = L.xs(i + 1);
+            // the reference divides by the ascending view's cell at the
+            // emitted (wrapped) index
+            const int64_t li = n - 2 - i;
+            const double size = L.xs.rev ? L.xs(li + 1) - L.xs(li) : xr - xl;
+            const bool leftmost = k == 0 && L.xt.base + (S.u[q] >> 1) > 0;
+            const double p1 = leftmost ? xl : L.xt(k0 + k);
+            const double ps = L.xt(k0 + k + 1);
+            const double p2 = ps < xr ? ps : xr;
+            double ratio = (p2 - p1) / size;
+            if (wi) ratio = ratio * wi[l0 + j];
+            const int64_t p = e0 + w0 + e;
+            __builtin_nontemporal_store(L.xs.rev ? ~i : i, &ii[p]);
+            __builtin_nontemporal_store(L.xt.g.rev ? ~(k0 + k) : k0 + k, &io[p]);
+            __builtin_nontemporal_store(ratio, &w[p]);
+        }
+        __syncthreads();
     }
 }
 
@@ -547,7 +568,7 @@ int rg_conservative_1d_emit(const double* x_input, int64_t n_input,
     k_zero_flags<<<grid_for(D, 256), 256, 0, s>>>(bad.p, D);
     for (int64_t b = 0; b < blocks; b += LINE_GRID)
         k_line_emit<<<(unsigned)std::min(blocks - b, LINE_GRID), LINE_BLOCK, 0, s>>>(
-            x_input, n_input, x_output, n_output, nseg, b, bad.p, weights_input, offsets, counts,
+            x_input, n_input, x_output, n_output, nseg, b, bad.p, weights_input, offsets,
             indices_input, indices_output, values);
     k_cons1d_emit<<<grid_for(D, 64), 64, 0, s>>>(x_input, n_input, x_output, n_output,
                                                   D, bad.p, weights_input, offsets, counts,
