@@ -600,7 +600,8 @@ __global__ __launch_bounds__(APPLY_BLOCK) void k_apply_jobs(
 namespace {
 
 // Tile width, and how results are stored (launch_apply).  Where the rows of
-// the output are whole cache lines, tiles are 16 wide and stores nontemporal.
+// the output are whole cache lines, tiles are 16 wide (FP32 32, a line, unless
+// the input is much the finer grid) and stores nontemporal.
 // Elsewhere a tile's row ends in two lines that the neighbouring tiles also
 // write, and a nontemporal store sends each part to memory by itself: while
 // the images fit the Infinity Cache with room to spare, the parts are stored
@@ -615,8 +616,10 @@ namespace {
 //   900^2 -> 1537^2 adjoint FP64 190 / 348 / 183; 2049^2 -> 1537^2 (whole
 //   lines) FP64 232 / 285 / 239, adjoint 285 / 321 / 301
 //   1500^2 -> 2000^2 FP64, 3 images - / 60 / 81 (150 MB)
-// and FP32 beyond the limit, 16 / 32 / 64 wide nontemporal: 1500^2 -> 2000^2
-//   - / 183 / 154, 1600^2 -> 1600^2 - / 120 / 168, 1700^2 -> 1200^2 102 / 89 / -
+// FP32 with whole lines: 2049^2 -> 1537^2 152 us 16 wide, 121 us 32 wide (150
+// and 147 at another angle); without them, beyond the limit, 16 / 32 / 64 wide
+// nontemporal: 1500^2 -> 2000^2 - / 183 / 154, 1600^2 -> 1600^2 - / 120 / 168,
+// 1700^2 -> 1200^2 102 / 89 / -
 constexpr int64_t LINE = 128;
 constexpr double MERGE_BYTES_8 = 130e6, MERGE_BYTES_4 = 190e6;
 int g_tile_w = 16;
@@ -719,12 +722,14 @@ int launch_apply(rg_weights* W, int dir, const int32_t* rowptr,
     const bool small = (double)batch * (nrows + ncols) * sizeof(T) <=
                        (sizeof(T) < 8 ? MERGE_BYTES_4 : MERGE_BYTES_8);
     const bool merge = !lines && small;
+    const double c = (double)ncols / (double)nrows;
     int widen = 0;
-    if (!lines && !small) {
-        const double c = (double)ncols / (double)nrows;
-        if (sizeof(T) >= 8) widen = c <= 1.75;
-        else widen = c <= 0.75 ? 2 : c <= 2.2;
-    }
+    if (sizeof(T) >= 8)
+        widen = !lines && !small && c <= 1.75;
+    else if (lines)
+        widen = c <= 2.2;
+    else if (!small)
+        widen = c <= 0.75 ? 2 : c <= 2.2;
     const int64_t tile_w = std::min(g_tile_w << widen, APPLY_BLOCK);
     ApplyGrid G = make_grid(shape, nrows, tile_w);
     rg_weights::Plan* P = nullptr;
@@ -750,8 +755,8 @@ int launch_apply(rg_weights* W, int dir, const int32_t* rowptr,
         // rows of more than 8 entries would read the rest once per image
         // group: the adjoint of 1025^2 -> 1500^2 (7.6 a row where there are
         // any, at most 12), 16 images: FP64 265 -> 195 us, FP32 121 -> 93; at
-        // three or four a row the longer row costs 8 %, at five nothing
-        const bool long_rows = W->nnz >= 5 * nrows;
+        // three or four a row the longer row costs 8 %, at five 1 or 2 % in FP32
+        const bool long_rows = 2 * W->nnz >= 11 * nrows;
 #define RG_ROUNDS_K(D, E, M)                                                           \
     k_apply_rounds<T, D, E, M><<<g1, bl, (size_t)lds, s>>>(                            \
         rowptr, col, P->off, P->box, w, x, y, nrows, ncols, src_gy, batch, G, lds)
