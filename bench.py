@@ -257,7 +257,7 @@ def main() -> int:
          "achieved": round(walk_flop / (ms_walk * 1e-3) / 1e12, 3), "peak": FP64_PEAK_TFLOPS,
          "unit": "TFLOP/s", "frac": round(walk_flop / (ms_walk * 1e-3) / 1e12 / FP64_PEAK_TFLOPS, 4),
          "traffic": None, "flop_per_launch": walk_flop, "ms_per_launch": round(ms_walk, 5)},
-        {"kernel": "k_reduce_groups (bucket sort + reduceat in LDS)", "bound": "hbm",
+        {"kernel": "k_reduce_cells (bucket sort in registers + reduceat, with its larger classes)", "bound": "hbm",
          "achieved": round(reduce_bytes / (ms_reduce * 1e-3) / 1e9, 1), "peak": HBM_PEAK_GBPS,
          "unit": "GB/s", "frac": round(reduce_bytes / (ms_reduce * 1e-3) / 1e9 / HBM_PEAK_GBPS, 4),
          "traffic": None, "bytes_per_launch": reduce_bytes, "ms_per_launch": round(ms_reduce, 5)},
