@@ -31,6 +31,8 @@
 // output point, clamped linear / bilinear weights.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "rg_internal.hpp"
 
 namespace rg {
@@ -567,23 +569,10 @@ int fill_tiles(double* a, double* other, const uint8_t* where, GsTileLists* list
     return RG_OK;
 }
 
-}  // namespace
-
-}  // namespace rg
-
-using namespace rg;
-
-extern "C" {
-
-int rg_fill_gauss_seidel_2d(double* a, const uint8_t* where, int64_t T, int64_t ny,
-                            int64_t nx, int64_t num_iterations, void* stream)
+// T slices, each launch of them within LAUNCH_THREADS
+int fill_slices(double* a, const uint8_t* where, int64_t T, int64_t ny, int64_t nx,
+                int64_t num_iterations, GsCoef c, hipStream_t s)
 {
-    if (T < 0 || ny < 1 || nx < 1 || num_iterations < 0 || T > 0xffffffffLL)
-        return fail(RG_ERR_ARGUMENT, "invalid fill shape or iteration count");
-    if (T == 0 || num_iterations == 0) return RG_OK;
-    if (!a || !where) return fail(RG_ERR_ARGUMENT, "NULL array");
-    hipStream_t s = (hipStream_t)stream;
-    const GsCoef c = gs_coef(nx, ny);
     if (ny * nx <= GS_LDS_CELLS && ny > 1 && nx > 1) {
         const int64_t late = n_late(ny, nx) + 1;
         k_gs_lds<<<(unsigned)T, GS_BLOCK, 8 * ny * nx + 4 * late, s>>>(a, where, (int)ny, (int)nx,
@@ -607,6 +596,32 @@ int rg_fill_gauss_seidel_2d(double* a, const uint8_t* where, int64_t T, int64_t 
         }
     }
     RG_HIP(hipGetLastError());
+    return RG_OK;
+}
+
+}  // namespace
+
+}  // namespace rg
+
+using namespace rg;
+
+extern "C" {
+
+int rg_fill_gauss_seidel_2d(double* a, const uint8_t* where, int64_t T, int64_t ny,
+                            int64_t nx, int64_t num_iterations, void* stream)
+{
+    if (T < 0 || ny < 1 || nx < 1 || num_iterations < 0 || T > 0xffffffffLL)
+        return fail(RG_ERR_ARGUMENT, "invalid fill shape or iteration count");
+    if (T == 0 || num_iterations == 0) return RG_OK;
+    if (!a || !where) return fail(RG_ERR_ARGUMENT, "NULL array");
+    const GsCoef c = gs_coef(nx, ny);
+    const int64_t cells = ny * nx;
+    const int64_t threads =  // of a slice, on the way that takes the most
+        std::max(cells, GS_BLOCK * gs_tiles(ny, GS_IN_H) * gs_tiles(nx, GS_IN_W));
+    const int64_t most = std::max<int64_t>(1, (LAUNCH_THREADS - GS_BLOCK) / threads);
+    for (int64_t t = 0; t < T; t += most)
+        RG_TRY(fill_slices(a + t * cells, where + t * cells, std::min(T - t, most), ny, nx,
+                           num_iterations, c, (hipStream_t)stream));
     return RG_OK;
 }
 

@@ -111,6 +111,11 @@ inline unsigned grid_for(int64_t n, int block)
     return (unsigned)(g < 1 ? 1 : g);
 }
 
+// Threads of one launch, at most: the runtime counts them in 32 bits and
+// drops the blocks beyond without an error (17 million blocks of 256 threads
+// ran as 222784).
+constexpr int64_t LAUNCH_THREADS = UINT32_MAX;
+
 }  // namespace rg
 
 // The object behind rg_weights_t: sparse weights of one 2-D element, stored
