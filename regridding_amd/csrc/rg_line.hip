@@ -507,7 +507,7 @@ __global__ void k_zero_flags(int32_t* __restrict__ p, int64_t n)
     if (i < n) p[i] = 0;
 }
 
-constexpr int64_t LINE_GRID = (int64_t)1 << 30;  // blocks per launch
+constexpr int64_t LINE_GRID = LAUNCH_THREADS / LINE_BLOCK;  // blocks per launch
 
 int check_line(const double* xin, int64_t n, const double* xout, int64_t m, int64_t D)
 {
