@@ -632,6 +632,16 @@ int64_t g_lds_limit = 32 * 1024;
 bool g_use_plan = true;
 bool g_rounds = true;  // one block per tile looping over image groups
 std::mutex g_plan_mu;
+std::mutex g_use_mu;
+
+// Waits for the applies of W queued on streams other than its own.
+void wait_uses(rg_weights* W)
+{
+    std::lock_guard<std::mutex> lk(g_use_mu);
+    for (auto& u : W->uses)
+        if (hipEventSynchronize(u.second) != hipSuccess)
+            (void)hipGetLastError();  // (recorded in a capture: nothing to wait for)
+}
 
 ApplyGrid make_grid(const int64_t* shape, int64_t nrows, int64_t tile_w)
 {
@@ -673,7 +683,7 @@ ApplyGrid gather_grid(const int64_t* shape, int64_t nrows)
     return G;
 }
 
-// The plan of one direction for the current tile shape (made on first use
+// The plan of one direction for these tiles of these grids (made on first use
 // on stream s; later applies on other streams must be ordered after it).
 int ensure_plan(rg_weights* W, int dir, int widen, const int32_t* rowptr,
                 const int32_t* col, const ApplyGrid& G, int64_t src_gy,
@@ -689,7 +699,9 @@ int ensure_plan(rg_weights* W, int dir, int widen, const int32_t* rowptr,
         return RG_OK;
     std::lock_guard<std::mutex> lk(g_plan_mu);
     rg_weights::Plan& P = W->plan[dir][widen];
-    if (P.tile_w != G.tw || P.ntiles != G.ntiles) {
+    if (P.tile_w != G.tw || P.gx != G.gx || P.gy != G.gy || P.src_gy != src_gy) {
+        // (a plan that is replaced may still be read by applies on other streams)
+        if (P.box) wait_uses(W);
         dev_free(P.box);
         dev_free(P.off);
         P.box = nullptr;
@@ -705,7 +717,9 @@ int ensure_plan(rg_weights* W, int dir, int widen, const int32_t* rowptr,
         RG_HIP(hipGetLastError());
         RG_TRY(read_scalars(mx.p, &P.max_cells, sizeof(int64_t), s));
         P.tile_w = G.tw;
-        P.ntiles = G.ntiles;
+        P.gx = G.gx;
+        P.gy = G.gy;
+        P.src_gy = src_gy;
     }
     *out = &P;
     return RG_OK;
@@ -826,8 +840,6 @@ int ensure_f32(rg_weights* W, hipStream_t s)
     W->val_out_f32 = b;
     return RG_OK;
 }
-
-std::mutex g_use_mu;
 
 }  // namespace
 

@@ -189,10 +189,11 @@ struct rg_weights {
     // apply plans (see rg_apply.hip), made on first use, one per direction
     // and tile width (the usual one, twice and four times it)
     struct Plan {
-        int64_t tile_w = 0;        // tile shape the plan was made for
+        int64_t tile_w = 0;        // what the plan was made for: the tiles' width,
+        int64_t gx = 0, gy = 0;    // the grid they cover,
+        int64_t src_gy = 0;        // and the row length of the input grid
         int32_t* box = nullptr;    // per tile: i0, j0, rows, cols of the patch
         uint16_t* off = nullptr;   // per CSR entry: offset inside its patch
-        int64_t ntiles = 0;
         int64_t max_cells = 0;     // largest patch (cells)
     } plan[2][3];
     rg_build_stats stats = {};
