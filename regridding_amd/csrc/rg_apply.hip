@@ -707,6 +707,7 @@ int ensure_plan(rg_weights* W, int dir, int widen, const int32_t* rowptr,
         P.box = nullptr;
         P.off = nullptr;
         P.tile_w = 0;
+        if (s != W->home) W->off_home = true;
         RG_TRY(dev_alloc((void**)&P.box, 4 * sizeof(int32_t) * G.ntiles, s));
         RG_TRY(dev_alloc((void**)&P.off, sizeof(uint16_t) * W->nnz, s));
         k_plan<<<(unsigned)G.ntiles, APPLY_BLOCK, 0, s>>>(rowptr, col, G, src_gy,
@@ -823,6 +824,7 @@ int ensure_f32(rg_weights* W, hipStream_t s)
     std::lock_guard<std::mutex> lk(g_f32_mu);
     if (W->val_out_f32 || W->nnz == 0) return RG_OK;
     float *a = nullptr, *b = nullptr;
+    if (s != W->home) W->off_home = true;
     RG_TRY(dev_alloc((void**)&a, W->nnz * sizeof(float), s));
     int st = dev_alloc((void**)&b, W->nnz * sizeof(float), s);
     if (st != RG_OK) {
@@ -845,7 +847,7 @@ int ensure_f32(rg_weights* W, hipStream_t s)
 
 int note_use(rg_weights* W, hipStream_t s)
 {
-    if (s == W->home) return RG_OK;
+    if (s == W->home && !W->off_home) return RG_OK;
     std::lock_guard<std::mutex> lk(g_use_mu);
     hipEvent_t ev = nullptr;
     for (auto& u : W->uses)

@@ -7,6 +7,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
 #include <memory>
 #include <string>
 #include <vector>
@@ -204,11 +205,15 @@ struct rg_weights {
     // device memory goes back to the pool of the stream it was allocated
     // on, so release first waits for applies still queued elsewhere.
     hipStream_t home = nullptr;
+    // Set once a plan or a single-precision copy was made on another stream
+    // than `home`, to whose pool it returns: from then on applies on `home`
+    // are among `uses` too.
+    std::atomic<bool> off_home{false};
     std::vector<std::pair<hipStream_t, hipEvent_t>> uses;
 };
 
 namespace rg {
 // Notes an apply of W on stream s (after its launch): records s's event
-// unless s is the handle's own stream.
+// unless s is the handle's own stream and all its memory is that stream's.
 int note_use(rg_weights* W, hipStream_t s);
 }  // namespace rg
