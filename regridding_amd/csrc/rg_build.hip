@@ -1301,13 +1301,15 @@ __global__ __launch_bounds__(64, 3) void k_reduce_cells(RedArgs A, int64_t n_gro
         atomicAdd(mismatch, 1);
     const int64_t base = A.bucket_off[4 * grp], end = A.bucket_off[4 * grp + 4];
     if (grp == 0 && lane == 0) A.cell_off[n_groups * 64] = A.bucket_off[4 * n_groups];
-    if (end > red_cap) {
-        // past the records a capacity-mode build holds: nothing of it is kept
+    if (end > red_cap || *cap_flag) {
+        // past the records a capacity-mode build holds, or a replay that has
+        // outgrown some capacity (records it found no room for were never
+        // written): nothing of it is kept
         A.nnz_row[grp * 64 + lane] = 0;
         A.cell_off[grp * 64 + lane] = 0;
         if (lane == 0) {
             A.group_mode[grp] = 0;
-            atomicOr(cap_flag, CAP_TRIPLES);
+            if (end > red_cap) atomicOr(cap_flag, CAP_TRIPLES);
         }
         return;
     }
