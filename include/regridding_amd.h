@@ -209,7 +209,8 @@ int rg_weights_free(rg_weights_t w);
 
 /* Declares the 2-D cell shapes of imported weights (built weights know
  * them): the apply walks its outputs in 2-D tiles for cache locality.  Has
- * no effect on results. */
+ * no effect on results.  A plan made for another shape is replaced at the next
+ * apply, so not while a captured graph that applies the handle is in use. */
 int rg_weights_set_shape(rg_weights_t w, int64_t ncx_in, int64_t ncy_in,
                          int64_t ncx_out, int64_t ncy_out);
 
@@ -234,7 +235,13 @@ int rg_set_apply_tuning(int tile_w, int images_per_pass, int lds_kib, int rounds
  * transpose=1 applies the transposed weights, which is what the reference
  * computes for regrid_from_weights(*transpose_weights(weights), ...)
  * (_weights_transposed.py:13-50).  Each output is accumulated sequentially
- * in the reference's storage order, so the FP64 result is bit-identical. */
+ * in the reference's storage order, so the FP64 result is bit-identical.
+ * Several images of weights with 65536 outputs or more are applied by a plan
+ * (2 bytes a weight, kept with the handle), made by the first call that wants
+ * it: one per direction and tile width, which the image count and the kind of
+ * value decide.  Making it waits for the stream; under stream capture a call
+ * takes a plan that its direction has, whatever its width, or goes without,
+ * which is slower for four images or more. */
 int rg_apply_f64(rg_weights_t w, int transpose, const double* values_input,
                  double* values_output, int64_t batch, void* stream);
 

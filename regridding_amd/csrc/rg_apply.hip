@@ -683,13 +683,35 @@ ApplyGrid gather_grid(const int64_t* shape, int64_t nrows)
     return G;
 }
 
-// The plan of one direction for these tiles of these grids (made on first use
-// on stream s; later applies on other streams must be ordered after it).
+bool capturing(hipStream_t s)
+{
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+        (void)hipGetLastError();  // not this call's failure
+        return false;
+    }
+    return st != hipStreamCaptureStatusNone;
+}
+
+bool plan_fits(const rg_weights::Plan& P, const ApplyGrid& G, int64_t src_gy)
+{
+    return P.tile_w == G.tw && P.gx == G.gx && P.gy == G.gy && P.src_gy == src_gy;
+}
+
+// The plan of one direction for tiles g_tile_w << widen of the output grid
+// (made on first use on stream s; later applies on other streams must be
+// ordered after it), and the tiles.  A plan cannot be made under capture (it
+// ends in a host read): there, any plan the direction has serves, and without
+// one the apply goes without.
 int ensure_plan(rg_weights* W, int dir, int widen, const int32_t* rowptr,
-                const int32_t* col, const ApplyGrid& G, int64_t src_gy,
-                int64_t batch, hipStream_t s, rg_weights::Plan** out)
+                const int32_t* col, const int64_t* shape, int64_t nrows, int64_t src_gy,
+                int64_t batch, hipStream_t s, rg_weights::Plan** out, ApplyGrid* tiles)
 {
     *out = nullptr;
+    const auto grid = [&](int wide) {
+        return make_grid(shape, nrows, std::min(g_tile_w << wide, APPLY_BLOCK));
+    };
+    ApplyGrid G = grid(widen);
     // below PLAN_MIN_ROWS outputs the gathered input stays in L2 anyway and
     // a plan (two kernels and a host wait) would only add latency; one image
     // is faster without (2049^2 -> 1537^2 FP64 31 against 37 us, FP32 25
@@ -698,8 +720,15 @@ int ensure_plan(rg_weights* W, int dir, int widen, const int32_t* rowptr,
     if (!g_use_plan || batch == 1 || G.gx == 1 || W->nnz == 0 || G.gx * G.gy < PLAN_MIN_ROWS)
         return RG_OK;
     std::lock_guard<std::mutex> lk(g_plan_mu);
+    if (!plan_fits(W->plan[dir][widen], G, src_gy) && capturing(s)) {
+        widen = -1;
+        for (int k = 0; k < 3; k++)
+            if (plan_fits(W->plan[dir][k], grid(k), src_gy)) widen = k;
+        if (widen < 0) return RG_OK;
+        G = grid(widen);
+    }
     rg_weights::Plan& P = W->plan[dir][widen];
-    if (P.tile_w != G.tw || P.gx != G.gx || P.gy != G.gy || P.src_gy != src_gy) {
+    if (!plan_fits(P, G, src_gy)) {
         // (a plan that is replaced may still be read by applies on other streams)
         if (P.box) wait_uses(W);
         dev_free(P.box);
@@ -708,8 +737,14 @@ int ensure_plan(rg_weights* W, int dir, int widen, const int32_t* rowptr,
         P.off = nullptr;
         P.tile_w = 0;
         if (s != W->home) W->off_home = true;
-        RG_TRY(dev_alloc((void**)&P.box, 4 * sizeof(int32_t) * G.ntiles, s));
-        RG_TRY(dev_alloc((void**)&P.off, sizeof(uint16_t) * W->nnz, s));
+        int st = dev_alloc((void**)&P.box, 4 * sizeof(int32_t) * G.ntiles, s);
+        if (st == RG_OK) st = dev_alloc((void**)&P.off, sizeof(uint16_t) * W->nnz, s);
+        if (st == RG_ERR_MEMORY) {  // the apply works without
+            dev_free(P.box);
+            P.box = nullptr;
+            return RG_OK;
+        }
+        RG_TRY(st);
         k_plan<<<(unsigned)G.ntiles, APPLY_BLOCK, 0, s>>>(rowptr, col, G, src_gy,
                                                         P.box, P.off);
         DevBuf<int64_t> mx;
@@ -723,6 +758,7 @@ int ensure_plan(rg_weights* W, int dir, int widen, const int32_t* rowptr,
         P.src_gy = src_gy;
     }
     *out = &P;
+    *tiles = G;
     return RG_OK;
 }
 
@@ -745,10 +781,9 @@ int launch_apply(rg_weights* W, int dir, const int32_t* rowptr,
         widen = c <= 2.2;
     else if (!small)
         widen = c <= 0.75 ? 2 : c <= 2.2;
-    const int64_t tile_w = std::min(g_tile_w << widen, APPLY_BLOCK);
-    ApplyGrid G = make_grid(shape, nrows, tile_w);
+    ApplyGrid G;
     rg_weights::Plan* P = nullptr;
-    RG_TRY(ensure_plan(W, dir, widen, rowptr, col, G, src_gy, batch, s, &P));
+    RG_TRY(ensure_plan(W, dir, widen, rowptr, col, shape, nrows, src_gy, batch, s, &P, &G));
     int32_t sb = 0;
     if (!P) {
         G = gather_grid(shape, nrows);
