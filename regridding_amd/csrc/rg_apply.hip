@@ -683,16 +683,6 @@ ApplyGrid gather_grid(const int64_t* shape, int64_t nrows)
     return G;
 }
 
-bool capturing(hipStream_t s)
-{
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &st) != hipSuccess) {
-        (void)hipGetLastError();  // not this call's failure
-        return false;
-    }
-    return st != hipStreamCaptureStatusNone;
-}
-
 bool plan_fits(const rg_weights::Plan& P, const ApplyGrid& G, int64_t src_gy)
 {
     return P.tile_w == G.tw && P.gx == G.gx && P.gy == G.gy && P.src_gy == src_gy;

@@ -538,12 +538,7 @@ bool tiles_apply(int64_t T, int64_t ny, int64_t nx, int64_t iterations, hipStrea
 {
     if (ny < GS_MIN || nx < GS_MIN || iterations < GS_FEW || ny * nx >= INT32_MAX) return false;
     if (T * gs_tiles(ny, GS_IN_H) * gs_tiles(nx, GS_IN_W) >= INT32_MAX) return false;
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &st) != hipSuccess) {
-        (void)hipGetLastError();  // not this call's failure
-        return false;
-    }
-    return st == hipStreamCaptureStatusNone;
+    return !capturing(s);
 }
 
 int fill_tiles(double* a, double* other, const uint8_t* where, GsTileLists* lists, int64_t T,

@@ -93,6 +93,10 @@ int read_scalars_end(void* host, size_t bytes);
 // rg_find_cells_2d_noalloc (looked up once per device and kept).
 int find_cells_scratch(int64_t** out);
 
+// Whether work on s is being recorded into a graph: memory of the pool must
+// then not be taken (it would be handed out again while the graph lives).
+bool capturing(hipStream_t s);
+
 // ---- scans ---------------------------------------------------------------
 
 // out[0..n] = exclusive prefix sum of in[0..n), out[n] = total.  `in` and

@@ -213,7 +213,8 @@ struct OutRange {
 // Shared start of both passes: the block's element and cells, the output
 // vertices they meet, and for each of the cells' vertices 2 (u - base) + e
 // with u = #{xt <= vertex} and e = 1 when a vertex of the output equals it.
-// A vertex out of order (or NaN) in the element flags it for sweep_1d.
+// A vertex out of order (or NaN) in the element flags it for sweep_1d (where
+// there are flags).
 struct LineBlock {
     int64_t d, i0;  // element, first cell (ascending)
     int ncell;
@@ -285,7 +286,7 @@ struct LineBlock {
             for (int64_t k = seg * share + tid; k < k1 && k < m - 1; k += LINE_BLOCK)
                 ok = ok && g(k) < g(k + 1);
         }
-        if (!ok) bad[d] = 1;
+        if (!ok && bad) bad[d] = 1;
         const auto count = [&](double x, int lo, int hi) {  // #{xt <= x} in [lo, hi]
             while (lo < hi) {
                 const int mid = (lo + hi) >> 1;
@@ -451,6 +452,27 @@ __global__ void k_cons1d_emit(const double* __restrict__ xin, int64_t n,
     sweep_1d(xin + d * n, n, xo, m, wi ? wi + d * (n - 1) : nullptr, sink);
 }
 
+// The same without flags, a block per element that looks its vertices over
+// itself: for an emit under stream capture, whose replays find nothing of the
+// call's own memory.
+__global__ __launch_bounds__(LINE_BLOCK) void k_cons1d_emit_unordered(
+    const double* __restrict__ xin, int64_t n, const double* __restrict__ xout, int64_t m,
+    int64_t d0, const double* __restrict__ wi, const int64_t* __restrict__ off,
+    const int32_t* __restrict__ cnt, int64_t* __restrict__ ii, int64_t* __restrict__ io,
+    double* __restrict__ w)
+{
+    const int64_t d = d0 + blockIdx.x;
+    const double* xi = xin + d * n;
+    const double* xo = xout + d * m;
+    const Axis a{xi, n, !(xi[0] < xi[n - 1])}, b{xo, m, !(xo[0] < xo[m - 1])};
+    bool ok = m < ((int64_t)1 << 30);
+    for (int64_t k = threadIdx.x; k < n - 1; k += LINE_BLOCK) ok = ok && a(k) < a(k + 1);
+    for (int64_t k = threadIdx.x; k < m - 1; k += LINE_BLOCK) ok = ok && b(k) < b(k + 1);
+    if (__syncthreads_and(ok) || threadIdx.x != 0) return;
+    EmitSink sink{off + d * (n - 1), cnt + d * (n - 1), b.rev, ii, io, w};
+    sweep_1d(xi, n, xo, m, wi ? wi + d * (n - 1) : nullptr, sink);
+}
+
 __global__ void k_multilinear_1d(const double* __restrict__ xin, int64_t n,
                                  const double* __restrict__ xout, int64_t m,
                                  int64_t D, const int64_t* __restrict__ index,
@@ -564,15 +586,23 @@ int rg_conservative_1d_emit(const double* x_input, int64_t n_input,
     hipStream_t s = (hipStream_t)stream;
     const int64_t nseg = (n_input - 1 + LINE_CELLS - 1) / LINE_CELLS, blocks = D * nseg;
     DevBuf<int32_t> bad;
-    RG_TRY(bad.alloc(D, s));
-    k_zero_flags<<<grid_for(D, 256), 256, 0, s>>>(bad.p, D);
+    if (!capturing(s)) {
+        RG_TRY(bad.alloc(D, s));
+        k_zero_flags<<<grid_for(D, 256), 256, 0, s>>>(bad.p, D);
+    }
     for (int64_t b = 0; b < blocks; b += LINE_GRID)
         k_line_emit<<<(unsigned)std::min(blocks - b, LINE_GRID), LINE_BLOCK, 0, s>>>(
             x_input, n_input, x_output, n_output, nseg, b, bad.p, weights_input, offsets,
             indices_input, indices_output, values);
-    k_cons1d_emit<<<grid_for(D, 64), 64, 0, s>>>(x_input, n_input, x_output, n_output,
-                                                  D, bad.p, weights_input, offsets, counts,
-                                                  indices_input, indices_output, values);
+    if (bad.p)
+        k_cons1d_emit<<<grid_for(D, 64), 64, 0, s>>>(x_input, n_input, x_output, n_output,
+                                                      D, bad.p, weights_input, offsets, counts,
+                                                      indices_input, indices_output, values);
+    else
+        for (int64_t d = 0; d < D; d += LINE_GRID)
+            k_cons1d_emit_unordered<<<(unsigned)std::min(D - d, LINE_GRID), LINE_BLOCK, 0, s>>>(
+                x_input, n_input, x_output, n_output, d, weights_input, offsets, counts,
+                indices_input, indices_output, values);
     RG_HIP(hipGetLastError());
     return RG_OK;
 }

@@ -318,6 +318,16 @@ int read_scalars_end(void* host, size_t bytes)
     return RG_OK;
 }
 
+bool capturing(hipStream_t s)
+{
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+        (void)hipGetLastError();  // not this call's failure
+        return false;
+    }
+    return st != hipStreamCaptureStatusNone;
+}
+
 // ---- scans ---------------------------------------------------------------
 
 namespace {
