@@ -341,8 +341,9 @@ int rg_multilinear_1d(const double* x_input, int64_t n_input, const double* x_ou
                       int64_t* n_outside, void* stream);
 
 /* Test hook (no reference counterpart): make the next call that reaches the
- * named site ("build", "apply", "alloc") fail with RG_ERR_INJECTED.  NULL
- * clears pending injections. */
+ * named site ("build", "apply", "alloc") fail with RG_ERR_INJECTED; at
+ * "digest", a digest job run out of memory with threads started.  NULL clears
+ * pending injections. */
 int rg_inject_failure(const char* site);
 
 /* ---- one hipGraph for a batched build and apply ---------------------

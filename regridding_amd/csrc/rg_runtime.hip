@@ -515,6 +515,13 @@ __global__ void k_copy_f64(const double* __restrict__ a, double* __restrict__ b,
 struct DigestJob {
     std::vector<std::thread> threads;
     std::vector<uint64_t> digests;
+
+    // (a job that could not be started in full ends here with threads running)
+    ~DigestJob()
+    {
+        for (auto& t : threads)
+            if (t.joinable()) t.join();
+    }
 };
 
 // An array below this is hashed at once (about 30 us; a thread costs as much).
@@ -622,6 +629,7 @@ int rg_digest_start(const void* const* data, const size_t* bytes, int n, void** 
             const size_t len = bytes[k];
             bool inline_ = len < DIGEST_THREAD_BYTES;
             if (!inline_) {
+                if (k > 0 && injected_failure("digest")) throw std::bad_alloc();
                 try {
                     j->threads.emplace_back([=] { *out = digest_bytes(p, len); });
                 } catch (const std::system_error&) {
