@@ -507,11 +507,15 @@ __global__ void k_copy_f64(const double* __restrict__ a, double* __restrict__ b,
 
 // ---- content digests ---------------------------------------------------------
 //
-// Eight lanes of 64-bit words, each folded in by exclusive or, an odd multiplier
-// and a rotation, and the lanes by the finaliser of SplitMix64.  Every fold is a
-// bijection of its word and of its lane, so a change of one word always shows;
-// others collide about once in 2^64.  The lanes' multiplies are independent,
-// which lets one core read about 20 GB/s.
+// Eight lanes of 64-bit words.  A word goes into its lane by exclusive or and a
+// multiplication to 128 bits by an odd constant, whose halves are joined by
+// exclusive or: the high half carries every bit of the word, the top one
+// included, into bits that depend on the data, so no fixed second edit undoes a
+// first.  (Kept to 64 bits, a change of the top bit stays one of the top bit,
+// and the flip of one bit eight words on cancels it whatever the values.)  The
+// lanes are joined by the finaliser of SplitMix64.  Contents not made for it
+// collide about once in 2^64.  The lanes' multiplies are independent, which
+// lets one core read about 35 GB/s (with 64-bit products 27).
 struct DigestJob {
     std::vector<std::thread> threads;
     std::vector<uint64_t> digests;
@@ -524,7 +528,7 @@ struct DigestJob {
     }
 };
 
-// An array below this is hashed at once (about 30 us; a thread costs as much).
+// An array below this is hashed at once (about 15 us; a thread costs as much).
 constexpr size_t DIGEST_THREAD_BYTES = 512 << 10;
 
 static uint64_t digest_bytes(const void* data, size_t bytes)
@@ -538,8 +542,8 @@ static uint64_t digest_bytes(const void* data, size_t bytes)
         uint64_t w[LANES];
         std::memcpy(w, q, sizeof w);
         for (int k = 0; k < LANES; k++) {
-            const uint64_t v = (h[k] ^ w[k]) * ODD;
-            h[k] = v << 31 | v >> 33;
+            const unsigned __int128 v = (unsigned __int128)(h[k] ^ w[k]) * ODD;
+            h[k] = (uint64_t)v ^ (uint64_t)(v >> 64);
         }
     };
     size_t left = bytes;
