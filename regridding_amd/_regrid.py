@@ -197,18 +197,22 @@ def _block_diagonal(flat, n_in: int, n_out: int):
 
 
 def apply_device(handle: Weights, transposed: bool, x: np.ndarray, n_out: int,
-                 out: np.ndarray | None = None) -> np.ndarray:
+                 out: np.ndarray | None = None, pending=None) -> np.ndarray | None:
     """(D, n_in) host float64 -> (D, n_out) host float64 through the GPU, into
-    `out` where given (C-contiguous, D * n_out values)."""
+    `out` where given (C-contiguous, D * n_out values).  With ``pending`` (see
+    ``_cache.lookup_pending``), None and `out` untouched if the weights' arrays
+    have changed."""
     D = x.shape[0]
+    dy = None
+    if D and n_out:
+        dx = DeviceArray.from_host(x)
+        dy = DeviceArray.empty((D, n_out), np.float64)
+        check(lib().rg_apply_f64(handle.ptr, int(transposed), dx.ptr, dy.ptr, D, 0))
+    if pending is not None and not pending.unchanged():
+        return None
     if out is None:
         out = np.empty((D, n_out))
-    if D == 0 or n_out == 0:
-        return out
-    dx = DeviceArray.from_host(x)
-    dy = DeviceArray.empty((D, n_out), np.float64)
-    check(lib().rg_apply_f64(handle.ptr, int(transposed), dx.ptr, dy.ptr, D, 0))
-    return dy.to_host(out=out)
+    return out if dy is None else dy.to_host(out=out)
 
 
 def _check_sizes(handle: Weights, transposed: bool, n_in: int, n_out: int) -> None:
@@ -232,8 +236,8 @@ def _apply_element(element, x: np.ndarray, n_in: int, n_out: int,
             handle, transposed, pending = hit
             hin, hout = (handle.n_in, handle.n_out)[:: -1 if transposed else 1]
             if (hin, hout) == (n_in, n_out):
-                y = apply_device(handle, transposed, x, n_out, out)
-                if pending.unchanged():
+                y = apply_device(handle, transposed, x, n_out, out, pending)
+                if y is not None:
                     return y
             elif pending.unchanged():
                 _check_sizes(handle, transposed, n_in, n_out)
