@@ -7,7 +7,7 @@
 //             row); chunk c > 0: a guessed start from the cell search
 //   count     every chunk walks, counts its triples, records its end state,
 //             adds its triples to the (cell group, pass) histogram and stages
-//             up to `cap` (cin, cout, term) triples per walk thread
+//             up to its pass's capacity of (cin, cout, term) triples per walk thread
 //   fixup     per row: chunks whose start differs from the predecessor's end
 //             are walked again from the true state (histogram corrected,
 //             staging rewritten)
@@ -22,7 +22,6 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <cmath>
 #include <cstring>
 #include <memory>
 #include <string>
@@ -30,6 +29,7 @@
 
 #include "rg_internal.hpp"
 #include "rg_sweep.hpp"
+#include "rg_walk_shape.hpp"
 #include "rg_wave.hpp"
 
 namespace rg {
@@ -637,7 +637,7 @@ __global__ __launch_bounds__(WALK_MAX_BLOCK) void k_walk_count(const Build* __re
                              int32_t* __restrict__ end,
                              int32_t* __restrict__ count,
                              int32_t* __restrict__ hist,
-                             Triple* __restrict__ stage, int64_t cap)
+                             Triple* __restrict__ stage)
 {
     const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (t >= nthreads_all) return;
@@ -648,7 +648,8 @@ __global__ __launch_bounds__(WALK_MAX_BLOCK) void k_walk_count(const Build* __re
     const int64_t g = B.chunk_gbase + r.g;
     int64_t k0, k1;
     chunk_range(P, r.c, &k0, &k1);
-    StageSink sink{0, t, cap, stage, hist + 4 * (B.cell_gbase >> 6) + r.p, {}};
+    StageSink sink{0, t - B.thread_gbase - P.thread_base, P.cap, stage + P.stage_base,
+                   hist + 4 * (B.cell_gbase >> 6) + r.p, {}};
     end[g] = walk_chunk(B, P, r.row, k0, k1, start[g], sink);
     sink.flush();
     count[g] = sink.n;
@@ -665,7 +666,7 @@ __global__ __launch_bounds__(WALK_MAX_BLOCK) void k_fixup(const Build* __restric
                         int32_t* __restrict__ end, int32_t* __restrict__ count,
                         int32_t* __restrict__ hist_all, int32_t* __restrict__ nfix,
                         int32_t* __restrict__ failed,
-                        Triple* __restrict__ stage, int64_t cap)
+                        Triple* __restrict__ stage)
 {
     const int64_t gr = grid_wave();
     const int lane = threadIdx.x & 63;
@@ -694,8 +695,8 @@ __global__ __launch_bounds__(WALK_MAX_BLOCK) void k_fixup(const Build* __restric
         UncountSink undo{hist, {}};
         (void)walk_chunk(B, P, row, k0, k1, start[g], undo);
         undo.flush();
-        StageSink redo{0, B.thread_gbase + thread_of_chunk(P, row, c), cap, stage,
-                       hist, {}};
+        StageSink redo{0, thread_of_chunk(P, row, c) - P.thread_base, P.cap,
+                       stage + P.stage_base, hist, {}};
         end[g] = walk_chunk(B, P, row, k0, k1, truth, redo);
         redo.flush();
         count[g] = redo.n;
@@ -713,19 +714,25 @@ __global__ __launch_bounds__(WALK_MAX_BLOCK) void k_fixup(const Build* __restric
 // Triples beyond the staging capacity, per chunk (then scanned into the
 // chunks' ranges of the overflow buffer), and the bucket cursors' first
 // values.
-__global__ void k_prepare_emit(const int32_t* __restrict__ count, int64_t nchunks,
-                               int64_t cap, int32_t* __restrict__ ov,
+__global__ void k_prepare_emit(const Build* __restrict__ builds,
+                               const int32_t* __restrict__ pair_of_wave, int64_t nthreads_all,
+                               const int32_t* __restrict__ count, int32_t* __restrict__ ov,
                                unsigned long long* __restrict__ total,
                                const int64_t* __restrict__ bucket_off,
                                uint32_t* __restrict__ cursor, int64_t nb)
 {
-    const int64_t g = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     int64_t v = 0;
-    if (g < nchunks) {
-        v = count[g] > cap ? count[g] - cap : 0;
-        ov[g] = (int32_t)v;
+    if (t < nthreads_all) {
+        const Build& B = build_of_thread(builds, pair_of_wave, t);
+        const ChunkRef r = chunk_of_thread(B, t - B.thread_gbase);
+        if (r.valid) {
+            const int64_t g = B.chunk_gbase + r.g, cap = pass_of_wave(B, r).cap;
+            v = count[g] > cap ? count[g] - cap : 0;
+            ov[g] = (int32_t)v;
+        }
     }
-    if (g < nb) cursor[g] = (uint32_t)bucket_off[g];
+    if (t < nb) cursor[t] = (uint32_t)bucket_off[t];
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
     if ((threadIdx.x & 63) == 0 && v) atomicAdd(total, (unsigned long long)v);
@@ -739,7 +746,7 @@ __global__ __launch_bounds__(WALK_MAX_BLOCK) void k_restage(const Build* __restr
                           const int32_t* __restrict__ start,
                           const int32_t* __restrict__ count,
                           const int64_t* __restrict__ ov_off,
-                          Triple* __restrict__ overflow, int64_t cap, int64_t ov_cap,
+                          Triple* __restrict__ overflow, int64_t ov_cap,
                           int32_t* __restrict__ restaged)
 {
     const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
@@ -747,9 +754,9 @@ __global__ __launch_bounds__(WALK_MAX_BLOCK) void k_restage(const Build* __restr
     const Build& B = build_of_thread(builds, pair_of_wave, t);
     const ChunkRef r = chunk_of_thread(B, t - B.thread_gbase);
     if (!r.valid) return;
-    const int64_t g = B.chunk_gbase + r.g;
-    if (count[g] <= cap) return;
     const Pass& P = pass_of_wave(B, r);
+    const int64_t g = B.chunk_gbase + r.g, cap = P.cap;
+    if (count[g] <= cap) return;
     int64_t k0, k1;
     chunk_range(P, r.c, &k0, &k1);
     // (a capacity-mode build sizes the buffer in advance: a chunk past its
@@ -812,7 +819,7 @@ __global__ __launch_bounds__(WALK_MAX_BLOCK) void k_scatter(const Build* __restr
                           const int32_t* __restrict__ pair_of_wave,
                           int64_t nthreads_all,
                           const int32_t* __restrict__ count,
-                          const Triple* __restrict__ stage, int64_t cap,
+                          const Triple* __restrict__ stage_all,
                           const Triple* __restrict__ ovbuf,
                           const int64_t* __restrict__ ov_off, int64_t ov_cap,
                           const int64_t* __restrict__ chunk_off,
@@ -828,7 +835,10 @@ __global__ __launch_bounds__(WALK_MAX_BLOCK) void k_scatter(const Build* __restr
     ScatTable& H = ((ScatTable*)scat_lds)[threadIdx.x >> 6];
     const Build& B = build_of_thread(builds, pair_of_wave, t);
     const ChunkRef r = chunk_of_thread(B, t - B.thread_gbase);
-    const int64_t g = B.chunk_gbase + r.g;
+    const Pass& P = pass_of_wave(B, r);
+    const int64_t g = B.chunk_gbase + r.g, cap = P.cap;
+    const int64_t u = t - B.thread_gbase - P.thread_base;
+    const Triple* const stage = stage_all + P.stage_base;
     // the pass's cursors: every lane of the wave sweeps one pass
     uint32_t* cursor = cursor_all + 4 * (B.cell_gbase >> 6) + r.p;
     int32_t n = r.valid ? count[g] : 0;
@@ -850,7 +860,7 @@ __global__ __launch_bounds__(WALK_MAX_BLOCK) void k_scatter(const Build* __restr
     Triple en[SCAT_R];
 #pragma unroll
     for (int k = 0; k < SCAT_R; k++)
-        if (k < n) en[k] = k < cap ? stage[stage_index(t, k, cap)] : ov[k - cap];
+        if (k < n) en[k] = k < cap ? stage[stage_index(u, k, cap)] : ov[k - cap];
     for (int32_t q0 = 0; q0 < mx; q0 += SCAT_R) {
         Triple e[SCAT_R];
 #pragma unroll
@@ -858,7 +868,7 @@ __global__ __launch_bounds__(WALK_MAX_BLOCK) void k_scatter(const Build* __restr
 #pragma unroll
         for (int k = 0; k < SCAT_R; k++) {
             const int32_t q = q0 + SCAT_R + k;
-            if (q < n) en[k] = q < cap ? stage[stage_index(t, q, cap)] : ov[q - cap];
+            if (q < n) en[k] = q < cap ? stage[stage_index(u, q, cap)] : ov[q - cap];
         }
         int32_t slot[SCAT_R], local[SCAT_R];
 #pragma unroll
@@ -2026,93 +2036,6 @@ __global__ void k_graph_jobs(JobDesc* __restrict__ jobs, const int32_t* __restri
     jobs[j].w = v_out + bases[2 * k];
 }
 
-// The split of the sweep rows into chunks, one walk thread each, and the
-// triples staged per thread.
-//
-// A chunk is a serial chain of dependent loads and divisions, whose time grows
-// with its triples (t of them), and costs a start search, whose time grows
-// with the number of chunks (all triples W / t): their sum is least at a t
-// that grows as sqrt(W).  A pass's edges emit about 2 (1 + c) triples each
-// when they cross c static cell edges, c from the grids' cell counts (they
-// are taken to cover each other, at a mean angle), and a pass's chunk is as
-// many edges as make t.  Build times, 16 edges for every pass -> this rule:
-//   67 x 190 -> 81 x 125 vertices   813 -> 389 us (the walk alone 469 -> 68)
-//   129^2 -> 101^2                  721 -> 322
-//   257^2 -> 193^2                  610 -> 354 (2 edges 359)
-//   513^2 -> 385^2                  692 -> 485 (2 edges 483, 4 edges 478)
-//   1025^2 -> 769^2                1013 -> 930 (4 edges 939, 8 edges 922)
-// (below ONE_EDGE_WORK triples, about 270^2 -> 200^2, every chunk is one edge)
-// and from about 2000^2 on t is at its bound, MAX_TRIPLES, and the chunks
-// are the 16 edges they were.  Coarse sweeps over fine static grids get
-// shorter chunks than the others, so that one staging capacity, 1.8 times
-// the expected triples, serves all: with 8 triples per edge for every pass
-// chunks of mixed batches overflowed and walked twice (64 pairs of 33 to
-// 1025 vertices per axis: the build 6.84 -> 5.56 ms).
-//
-// An explicit edges_per_lane or stage_per_edge applies to every pass as given
-// (a missing one of the two is 16 edges, or 8 triples).
-struct WalkShape {
-    static constexpr double MAX_TRIPLES = 72, ONE_EDGE_WORK = 1e6;
-    static constexpr int64_t MAX_EDGES = 32, MIN_CAP = 16, MAX_CAP = 128;
-    int64_t K;           // edges per chunk of every pass; 0: by expected work
-    double target = 1;   // expected triples of a chunk
-    int64_t cap;         // triples staged per walk thread
-
-    struct Dims {
-        int64_t rows, edges;  // sweep rows, edges per row
-        double per_edge;      // expected triples per edge
-    };
-
-    static Dims dims(const rg_pair_desc& d, int p)
-    {
-        const bool in = p >= 2;
-        const int64_t nxs = in ? d.nxi : d.nxo, nys = in ? d.nyi : d.nyo;
-        const int64_t nxt = in ? d.nxo : d.nxi, nyt = in ? d.nyo : d.nyi;
-        Dims q;
-        q.rows = (p & 1) ? nxs : nys;
-        q.edges = ((p & 1) ? nys : nxs) - 1;
-        // 2 / pi: the mean of |cos| and |sin| over the angle
-        const double c = 0.64 * (double)(nxt - 1 + nyt - 1) / (double)q.edges;
-        q.per_edge = 2 * (1 + c);
-        return q;
-    }
-
-    WalkShape(const rg_pair_desc* pairs, int64_t npairs, int64_t edges, int64_t per_edge)
-    {
-        if (edges > 0 || per_edge > 0) {
-            K = edges > 0 ? edges : 16;
-            cap = K * (per_edge > 0 ? per_edge : 8);
-            return;
-        }
-        K = 0;
-        double work = 0;
-        for (int64_t k = 0; k < npairs; k++)
-            for (int p = 0; p < 4; p++) {
-                const Dims q = dims(pairs[k], p);
-                work += (double)q.rows * (double)q.edges * q.per_edge;
-            }
-        target = work < ONE_EDGE_WORK ? 1 : std::min(std::sqrt(work) / 105, MAX_TRIPLES);
-        double most = 0;
-        for (int64_t k = 0; k < npairs; k++)
-            for (int p = 0; p < 4; p++)
-                most = std::max(most, (double)edges_per_chunk(pairs[k], p) *
-                                          dims(pairs[k], p).per_edge);
-        cap = std::min(MAX_CAP, std::max(MIN_CAP, (int64_t)(1.8 * most) + 1));
-    }
-
-    // Edges per chunk of pass p of a pair: the target's, spread evenly over
-    // the chunks of a row.
-    int64_t edges_per_chunk(const rg_pair_desc& d, int p) const
-    {
-        if (K > 0) return K;
-        const Dims q = dims(d, p);
-        int64_t e = (int64_t)(target / q.per_edge + 0.5);
-        e = std::max<int64_t>(1, std::min({e, MAX_EDGES, q.edges}));
-        const int64_t chunks = (q.edges + e - 1) / e;
-        return (q.edges + chunks - 1) / chunks;
-    }
-};
-
 int build_batched(const rg_pair_desc* pairs, int64_t npairs,
                   const rg_tuning* tuning, rg_weights** out, hipStream_t s,
                   CaptureCaps* caps);
@@ -2247,7 +2170,7 @@ int build_batched(const rg_pair_desc* pairs, int64_t npairs,
     std::vector<Build> builds(npairs);
     std::vector<int64_t> wave_pf(npairs + 1), row_pf(npairs + 1),
         ing_pf(npairs + 1), outg_pf(npairs + 1);
-    int64_t cell_tot = 0, out_tot = 0, thr_tot = 0, chunk_tot = 0, row_tot = 0;
+    int64_t cell_tot = 0, out_tot = 0, thr_tot = 0, chunk_tot = 0, row_tot = 0, stage_tot = 0;
     bool any_wi = false;
     for (int64_t k = 0; k < npairs; k++) {
         const rg_pair_desc& d = pairs[k];
@@ -2286,6 +2209,9 @@ int build_batched(const rg_pair_desc* pairs, int64_t npairs,
             Q.K = shape.edges_per_chunk(d, p);
             Q.cpr = std::max<int64_t>(1, (Q.nk - 1 + Q.K - 1) / Q.K);
             B.K = std::max(B.K, Q.K);
+            Q.cap = shape.staged(d, p);
+            Q.stage_base = stage_tot;
+            stage_tot += threads_of_pass(Q.nrows, Q.cpr) * Q.cap;
             Q.chunk_base = chunk;
             Q.thread_base = threads;
             B.row_base[p] = rows;
@@ -2444,19 +2370,18 @@ int build_batched(const rg_pair_desc* pairs, int64_t npairs,
     tm.mark();  // 2
 
     // ---- count (staging the triples)
-    const int64_t cap = shape.cap;
     DevBuf<Triple> stage;
-    RG_TRY(stage.alloc((size_t)thr_tot * cap, s));
+    RG_TRY(stage.alloc((size_t)stage_tot, s));
     k_walk_count<<<grid_for(thr_tot, block), block, 0, s>>>(
         d_builds, pair_of_wave.p, thr_tot, start.p, end.p, count.p, hist.p,
-        stage.p, cap);
+        stage.p);
     RG_HIP(hipGetLastError());
     tm.mark();  // 3
 
     // ---- fix-up
     k_fixup<<<grid_for(row_tot * 64, 256), 256, 0, s>>>(
         d_builds, pair_of_row.p, row_tot, start.p, end.p, count.p, hist.p,
-        counters.p + 1, counters.p + 2, stage.p, cap);
+        counters.p + 1, counters.p + 2, stage.p);
     RG_HIP(hipGetLastError());
     DevBuf<int64_t> chunk_off, bucket_off;
     RG_TRY(chunk_off.alloc(chunk_tot + 1, s));
@@ -2467,8 +2392,8 @@ int build_batched(const rg_pair_desc* pairs, int64_t npairs,
     DevBuf<int32_t> ov;
     RG_TRY(ov.alloc(chunk_tot, s));
     uint32_t* cursor = (uint32_t*)hist.p;  // reused: one word per bucket
-    k_prepare_emit<<<grid_for(std::max(chunk_tot, 4 * n_groups), 256), 256, 0, s>>>(
-        count.p, chunk_tot, cap, ov.p, (unsigned long long*)(counters.p + 6), bucket_off.p,
+    k_prepare_emit<<<grid_for(std::max(thr_tot, 4 * n_groups), 256), 256, 0, s>>>(
+        d_builds, pair_of_wave.p, thr_tot, count.p, ov.p, (unsigned long long*)(counters.p + 6), bucket_off.p,
         cursor, 4 * n_groups);
     RG_HIP(hipGetLastError());
     int64_t tot[2];
@@ -2526,13 +2451,13 @@ int build_batched(const rg_pair_desc* pairs, int64_t npairs,
         // the chunks' ranges of the overflow buffer
         RG_TRY(scan_i32_to_i64(ov.p, ov_off.p, chunk_tot, s));
         k_restage<<<grid_for(thr_tot, block), block, 0, s>>>(
-            d_builds, pair_of_wave.p, thr_tot, start.p, count.p, ov_off.p, ovbuf.p, cap,
+            d_builds, pair_of_wave.p, thr_tot, start.p, count.p, ov_off.p, ovbuf.p,
             ov_tot, counters.p + 4);
         RG_HIP(hipGetLastError());
     }
     k_scatter<<<grid_for(thr_tot, SCAT_BLOCK), SCAT_BLOCK, (SCAT_BLOCK / 64) * sizeof(ScatTable),
                 s>>>(
-        d_builds, pair_of_wave.p, thr_tot, count.p, stage.p, cap, ovbuf.p,
+        d_builds, pair_of_wave.p, thr_tot, count.p, stage.p, ovbuf.p,
         ov_off.p, ov_tot, chunk_off.p, cursor, rec.p, rcell.p, (uint32_t)T, counters.p + 2);
     RG_HIP(hipGetLastError());
     tm.mark();  // 6

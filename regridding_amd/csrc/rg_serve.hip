@@ -28,6 +28,7 @@
 #include <vector>
 
 #include "rg_internal.hpp"
+#include "rg_walk_shape.hpp"
 
 namespace rg {
 int build_batched(const rg_pair_desc* pairs, int64_t npairs,
@@ -68,16 +69,18 @@ int64_t cells_in(const rg_serve_request& r) { return (r.nxi - 1) * (r.nyi - 1); 
 int64_t cells_out(const rg_serve_request& r) { return (r.nxo - 1) * (r.nyo - 1); }
 
 // Device bytes a request holds while in a group: its values and results,
-// and for a build its coordinates plus the build's working set (staging,
-// buckets, records, both CSR layouts: about 400 bytes per sweep edge of a
-// large group; the one-edge chunks of a small one take up to 500).
+// and for a build its coordinates plus the build's working set.
 int64_t footprint(const rg_serve_request& r, bool build)
 {
     const int64_t es = r.dtype == RG_F32 ? 4 : 8;
     int64_t b = r.batch * (cells_in(r) + cells_out(r)) * es;
     if (build) {
-        const int64_t vi = r.nxi * r.nyi, vo = r.nxo * r.nyo;
-        b += 16 * (vi + vo) + 500 * 2 * (vi + vo);
+        rg_pair_desc d = {};
+        d.nxi = r.nxi;
+        d.nyi = r.nyi;
+        d.nxo = r.nxo;
+        d.nyo = r.nyo;
+        b += 16 * (r.nxi * r.nyi + r.nxo * r.nyo) + build_bytes(d);
     }
     return b;
 }

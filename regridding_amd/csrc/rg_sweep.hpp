@@ -76,6 +76,8 @@ struct Pass {
     int64_t chunk_base;      // global id of the first chunk of this pass
     int64_t cpr;             // chunks per row
     int64_t thread_base;     // first walk thread of this pass
+    int64_t cap;             // triples staged per walk thread
+    int64_t stage_base;      // first staged triple of the pass in a build's staging
 };
 
 struct Build {

@@ -15,6 +15,7 @@
 #include <vector>
 
 #include "../../regridding_amd/csrc/rg_layout.hpp"
+#include "../../regridding_amd/csrc/rg_walk_shape.hpp"
 #include "../../regridding_amd/csrc/rg_sweep.hpp"
 
 using namespace rg;
@@ -530,6 +531,28 @@ void rge_secant_pair(const double* x, const double* y, int64_t nx, int64_t ny,
         a[q] = index_secant(x, y, nx, ny, px[q], py[q]);
         b[q] = index_secant_xy(xy.data(), nx, ny, px[q], py[q]);
     }
+}
+
+// The split of a batch of pairs, vertices (nxi, nyi, nxo, nyo) each: the bytes
+// its staging takes, and per pair the bytes its build is taken to need.
+int64_t rge_walk_shape(const int64_t* sizes, int64_t n, int64_t* bytes)
+{
+    std::vector<rg_pair_desc> pairs(n);
+    for (int64_t k = 0; k < n; k++) {
+        pairs[k].nxi = sizes[4 * k];
+        pairs[k].nyi = sizes[4 * k + 1];
+        pairs[k].nxo = sizes[4 * k + 2];
+        pairs[k].nyo = sizes[4 * k + 3];
+    }
+    const WalkShape shape(pairs.data(), n, 0, 0);
+    int64_t staging = 0;
+    for (int64_t k = 0; k < n; k++) {
+        for (int p = 0; p < 4; p++)
+            staging += shape.threads(pairs[k], p) * shape.staged(pairs[k], p) *
+                       (int64_t)sizeof(Triple);
+        bytes[k] = build_bytes(pairs[k]);
+    }
+    return staging;
 }
 
 }  // extern "C"
