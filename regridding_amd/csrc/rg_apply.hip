@@ -88,11 +88,66 @@ constexpr int PROD_SLOTS = 64 * ENTRIES_U + 1;  // the last one is 0
 // images of 129^2 -> 101^2 take 7.6 us in 40 blocks, 4.6 us in 320 (any
 // limit from 512 to 4096 measures the same).
 constexpr int64_t SPLIT_TILES = 1024;
+// Long rows.  Where a row is a good part of a chunk, a few of the 64 lanes add
+// up products one after another, an entry at a time taking the LDS's latency.
+// Rows of 64 entries on average, or of LONG_FEW in few rows (long_rows), get a
+// wavefront each, which is as many chains at once as there are rows and, with
+// several images, images (apply_long_row).  In a wavefront of 64 rows that holds
+// more than LONG_ENTRIES a row (weights of a small input on a large output grid)
+// the sums are pipelined, with several images in chunks of 128, where the
+// registers they take are free.  us for 1 / 8 images of FP64, a lane per row
+// from memory -> rows in chunks only -> this:
+//   1025^2 -> 65^2 (239 a row)     90 / 737 -> 423 / 345 -> 12 / 25
+//   2049^2 -> 9^2 (53045)          17456 / 79939 -> 80365 / 89562 -> 1350 / 980
+//   eight of 257^2 -> 17^2 (239)   73 / 645 -> 409 / 3226 -> 15 / 23
+//   513^2 -> 513^2, twenty times as wide (426 a row in 26^2 cells of the output)
+//                                  128 / 1665 -> 201 / 1664 -> 103 / 1660
+//   513^2 -> 86^2 (43), chunks     21 / 129 -> 21 / 20 (a wavefront a row 12 / 13,
+//     but 51 where chunks take 29 for eight such pairs of 1 image)
+constexpr int32_t LONG_ENTRIES = 64;
+constexpr int64_t LONG_FEW_ROWS = 4096, LONG_FEW_ONE = 40, LONG_FEW = 28;
+constexpr int LONG_IMAGES = 5;
+static_assert((LONG_IMAGES - 1) * 65 + 64 <= PROD_SLOTS, "the products of a long row's images");
+
+// acc + prod[s] + ... + prod[e - 1], one after another.  The last steps of four
+// read the zero past the products, which changes no sum (none is -0, as it
+// starts from +0).  PIPELINE: a long run's next eight are read while the last
+// eight are added, where an entry takes the LDS's latency otherwise.
+template <bool PIPELINE, class T>
+__device__ inline T add_products(const T* __restrict__ prod, int32_t s, int32_t e, T acc)
+{
+    if (PIPELINE && e - s >= 16) {
+        T p[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) p[u] = prod[s + u];
+#pragma unroll 1
+        for (; s + 16 <= e; s += 8) {
+            T n[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) n[u] = prod[s + 8 + u];
+#pragma unroll
+            for (int u = 0; u < 8; u++) acc = acc + p[u];
+#pragma unroll
+            for (int u = 0; u < 8; u++) p[u] = n[u];
+        }
+#pragma unroll
+        for (int u = 0; u < 8; u++) acc = acc + p[u];
+        s += 8;
+    }
+    for (int32_t q = s; q < e; q += 4) {
+        T p[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) p[u] = prod[q + u < e ? q + u : PROD_SLOTS - 1];
+#pragma unroll
+        for (int u = 0; u < 4; u++) acc = acc + p[u];
+    }
+    return acc;
+}
 
 // Entries [c0, c0 + 64 * U) of the wavefront's `total` for `images` images:
 // the products go to LDS in entry order, and each lane adds up those of its
 // row, entries [s, e), to y (from 0 where c0 is 0).
-template <bool MERGE, class T, int U>
+template <bool MERGE, bool PIPELINE, class T, int U>
 __device__ inline void apply_entries(const int32_t* __restrict__ col, const T* __restrict__ w,
                                      const T* __restrict__ x, T* __restrict__ y, int64_t nrows,
                                      int64_t ncols, int32_t images, int32_t c0, int32_t total,
@@ -122,34 +177,76 @@ __device__ inline void apply_entries(const int32_t* __restrict__ col, const T* _
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         if (stores) {
-            T acc = c0 ? *y : T(0);
-            // four at a time; past the row's end +0 is added, which changes
-            // no sum (none is -0, as it starts from +0)
-            for (int32_t q = s; q < e; q += 4) {
-                T p[4];
-#pragma unroll
-                for (int u = 0; u < 4; u++) p[u] = prod[q + u < e ? q + u : PROD_SLOTS - 1];
-#pragma unroll
-                for (int u = 0; u < 4; u++) acc = acc + p[u];
-            }
+            const T acc = add_products<PIPELINE>(prod, s, e, c0 ? *y : T(0));
             store_result<MERGE>(y, acc);
         }
         y += nrows;
     }
 }
 
+// One row of `total` entries for up to LONG_IMAGES images, by a wavefront: 64
+// entries at a time, their products for every image in LDS, added up by one
+// lane per image (image m's are at 65 m, so that the lanes' reads fall in
+// different banks).  The next entries are requested before the sums.
+template <bool MERGE, class T>
+__device__ inline void apply_long_row(const int32_t* __restrict__ col, const T* __restrict__ w,
+                                      const T* __restrict__ x, T* __restrict__ y, int64_t nrows,
+                                      int64_t ncols, int32_t images, int32_t total,
+                                      T* __restrict__ prod)
+{
+    const int32_t lane = threadIdx.x & 63;
+    uint32_t c = 0;
+    T wq = T(0), acc = T(0);
+    const auto request = [&](int32_t c0) {
+        const uint32_t t = min(c0 + lane, total - 1);
+        c = (uint32_t)col[t];
+        wq = w[t];
+    };
+    if (total > 0) request(0);
+    for (int32_t c0 = 0; c0 < total; c0 += 64) {
+        T xv[LONG_IMAGES];
+#pragma unroll
+        for (int m = 0; m < LONG_IMAGES; m++)
+            if (m < images) xv[m] = x[m * ncols + c];
+        __builtin_amdgcn_wave_barrier();  // the last products are read
+#pragma unroll
+        for (int m = 0; m < LONG_IMAGES; m++)
+            if (m < images) prod[m * 65 + lane] = wq * xv[m];
+        if (c0 + 64 < total) request(c0 + 64);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        if (lane < images) {
+            const T* const p = prod + lane * 65;
+            const int32_t n = min(64, total - c0);
+            int32_t k = 0;
+            for (; k + 8 <= n; k += 8) {
+                T v[8];
+#pragma unroll
+                for (int u = 0; u < 8; u++) v[u] = p[k + u];
+#pragma unroll
+                for (int u = 0; u < 8; u++) acc = acc + v[u];
+            }
+            for (; k < n; k++) acc = acc + p[k];
+        }
+    }
+    if (lane < images) store_result<MERGE>(y + lane * nrows, acc);
+}
+
 // Applies the CSR to one tile and `images` images, a wavefront for each 64
 // consecutive rows and by itself.  A tile is 64 columns of APPLY_BLOCK / 64
-// grid rows at (ib, jb) or, if `flat`, APPLY_BLOCK rows of one long row.
+// grid rows at (ib, jb); APPLY_BLOCK rows of one long row (`th` 1); or, of a
+// grid one column wide, APPLY_BLOCK / 64 rows, a wavefront each.
 template <bool MERGE, class T>
 __device__ inline void apply_rows(const int32_t* __restrict__ rowptr,
                                   const int32_t* __restrict__ col, const T* __restrict__ w,
                                   const T* __restrict__ x, T* __restrict__ y, int64_t nrows,
                                   int64_t ncols, int32_t images, int64_t gy, int64_t ib,
-                                  int64_t jb, bool flat, T* __restrict__ prod)
+                                  int64_t jb, int64_t th, T* __restrict__ prod)
 {
     const int32_t lane = threadIdx.x & 63;
     const int32_t wave = __builtin_amdgcn_readfirstlane((int32_t)threadIdx.x / 64);
+    const bool flat = th == 1;
     const int64_t i = ib + (flat ? 0 : wave), j = jb + (flat ? wave * 64 : 0);
     const int64_t r0 = i * gy + j;
     if (r0 >= nrows || j >= gy) return;
@@ -173,13 +270,31 @@ __device__ inline void apply_rows(const int32_t* __restrict__ rowptr,
             for (int32_t m = 0; m < images; m++) y[m * nrows] = T(0);
         return;
     }
-    if (total <= 64 * (ENTRIES_U / 2))
-        apply_entries<MERGE, T, ENTRIES_U / 2>(col, w, x, y, nrows, ncols, images, 0, total, s, e, valid,
-                                        prod);
-    else
+    if (images > 1 && rows == 1) {
+        // (eight images in two passes of four)
+        const int32_t step = images <= LONG_IMAGES ? images : (images + 1) / 2;
+        static_assert(JOB_DB <= 2 * LONG_IMAGES, "two passes");
+        for (int32_t m = 0; m < images; m += step)
+            apply_long_row<MERGE, T>(col, w, x + m * ncols, y + m * nrows, nrows, ncols,
+                                     min(step, images - m), total, prod);
+        return;
+    }
+    if (total <= 64 * (ENTRIES_U / 2)) {
+        apply_entries<MERGE, false, T, ENTRIES_U / 2>(col, w, x, y, nrows, ncols, images, 0, total,
+                                                      s, e, valid, prod);
+    } else if (images == 1) {
         for (int32_t c0 = 0; c0 < total; c0 += 64 * ENTRIES_U)
-            apply_entries<MERGE, T, ENTRIES_U>(col, w, x, y, nrows, ncols, images, c0, total, s, e,
-                                        valid, prod);
+            apply_entries<MERGE, true, T, ENTRIES_U>(col, w, x, y, nrows, ncols, 1, c0, total, s,
+                                                     e, valid, prod);
+    } else if (total <= LONG_ENTRIES * rows) {
+        for (int32_t c0 = 0; c0 < total; c0 += 64 * ENTRIES_U)
+            apply_entries<MERGE, false, T, ENTRIES_U>(col, w, x, y, nrows, ncols, images, c0,
+                                                      total, s, e, valid, prod);
+    } else {
+        for (int32_t c0 = 0; c0 < total; c0 += 64 * 2)
+            apply_entries<MERGE, true, T, 2>(col, w, x, y, nrows, ncols, images, c0,
+                                                         total, s, e, valid, prod);
+    }
 }
 
 template <class T, bool MERGE>
@@ -197,7 +312,7 @@ __global__ __launch_bounds__(APPLY_BLOCK) void k_apply(
     const int64_t d0 = (int64_t)blockIdx.y * db;
     const int64_t nd = batch - d0 < db ? batch - d0 : db;
     apply_rows<MERGE, T>(rowptr, col, w, x + d0 * ncols, y + d0 * nrows, nrows, ncols, (int32_t)nd, G.gy,
-                  ti * G.th, tj * G.tw, G.th == 1, prod[threadIdx.x / 64]);
+                  ti * G.th, tj * G.tw, G.th, prod[threadIdx.x / 64]);
 }
 
 // ---- the apply plan -------------------------------------------------------
@@ -594,7 +709,7 @@ __global__ __launch_bounds__(APPLY_BLOCK) void k_apply_jobs(
     const int64_t nd = J.batch - d0 < JOB_DB ? J.batch - d0 : JOB_DB;
     apply_rows<false, T>(J.rowptr, J.col, (const T*)J.w, (const T*)J.x + d0 * J.ncols,
                   (T*)J.y + d0 * J.nrows, J.nrows, J.ncols, (int32_t)nd, J.gy, ti * J.th,
-                  tj * J.tw, J.th == 1, prod[threadIdx.x / 64]);
+                  tj * J.tw, J.th, prod[threadIdx.x / 64]);
 }
 
 namespace {
@@ -660,13 +775,32 @@ ApplyGrid make_grid(const int64_t* shape, int64_t nrows, int64_t tile_w)
     return G;
 }
 
+// Whether an apply without a plan gives every row a wavefront: us of chunks /
+// of a wavefront a row, 1 image, 31 to 69 entries a row: 2601 rows 15 / 11, 1764
+// 22 / 11, 7225 21 / 12, 42025 12 / 23, 28900 18 / 18, 16384 42 / 14; eight
+// images 12 / 11, 19 / 11, 20 / 13, 31 / 50, 30 / 38, 38 / 38; eight jobs of 1764
+// rows and 1, 3 and 8 images 29 / 19, 62 / 18, 167 / 26, of 7225 rows 29 / 51, 60 /
+// 48, 143 / 71, of 2601 rows 18 / 22, 34 / 21, 94 / 31.
+bool long_rows(int64_t nrows, int64_t nnz, int64_t images)
+{
+    return nnz >= LONG_ENTRIES * nrows ||
+           (nrows <= LONG_FEW_ROWS && nnz >= (images > 1 ? LONG_FEW : LONG_FEW_ONE) * nrows);
+}
+
 // Tiles of an apply without a plan: 64 columns of four grid rows (16 or 32
 // columns of more rows measure the same).  Grids of narrow rows are taken as
 // one long row, where a block's consecutive rows are a compact patch too; so
-// are rows of unknown shape.
-ApplyGrid gather_grid(const int64_t* shape, int64_t nrows)
+// are rows of unknown shape.  Long rows are a grid one column wide.
+ApplyGrid gather_grid(const int64_t* shape, int64_t nrows, int64_t nnz, int64_t images)
 {
     ApplyGrid G;
+    if (long_rows(nrows, nnz, images)) {
+        G.gx = nrows;
+        G.gy = G.tw = G.ntx = 1;
+        G.th = APPLY_BLOCK / 64;
+        G.ntiles = (nrows + G.th - 1) / G.th;
+        return G;
+    }
     G.gx = shape[0];
     G.gy = shape[1];
     G.tw = 64;
@@ -776,7 +910,7 @@ int launch_apply(rg_weights* W, int dir, const int32_t* rowptr,
     RG_TRY(ensure_plan(W, dir, widen, rowptr, col, shape, nrows, src_gy, batch, s, &P, &G));
     int32_t sb = 0;
     if (!P) {
-        G = gather_grid(shape, nrows);
+        G = gather_grid(shape, nrows, W->nnz, batch);
         sb = (int32_t)std::min<int64_t>(batch, JOB_DB);
         while (sb > 1 && G.ntiles * ((batch + sb - 1) / sb) < SPLIT_TILES) sb = (sb + 1) / 2;
     }
@@ -941,7 +1075,7 @@ int launch_jobs_common(const rg_apply_job* jobs, int64_t njobs, bool f32,
         d.batch = jb.batch;
         if (d.nrows == 0 || d.batch == 0) continue;
         const int64_t* shape = jb.transpose ? W->shape_in : W->shape_out;
-        job_tiles(d, shape[0], shape[1]);
+        job_tiles(d, shape[0], shape[1], W->nnz);
         d.block_base = nblocks;
         prefix.push_back(nblocks);
         nblocks += d.nrt * ((d.batch + JOB_DB - 1) / JOB_DB);
@@ -1006,10 +1140,10 @@ int apply_jobs_device(const JobDesc* jobs, const int64_t* prefix, int njobs, int
     return RG_OK;
 }
 
-void job_tiles(JobDesc& d, int64_t gx, int64_t gy)
+void job_tiles(JobDesc& d, int64_t gx, int64_t gy, int64_t nnz)
 {
     const int64_t shape[2] = {gx, gy};
-    const ApplyGrid G = gather_grid(shape, d.nrows);
+    const ApplyGrid G = gather_grid(shape, d.nrows, nnz, d.batch);
     d.tw = (int32_t)G.tw;
     d.th = (int32_t)G.th;
     d.gy = G.gy;

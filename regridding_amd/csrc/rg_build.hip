@@ -1983,6 +1983,7 @@ struct CaptureCaps {
     // makes handles; true: the capacity mode described above
     bool capacity = false;
     int64_t T_seen = 0, ov_seen = 0, nnz_seen = 0;
+    std::vector<int64_t> pair_nnz;  // recorded with them: each pair's weights
     int64_t T_cap = 0, ov_cap = 0, nnz_cap = 0;
     void* meta_pinned = nullptr;  // caller-owned pinned snapshot of the tables
     size_t meta_pinned_cap = 0;
@@ -2271,7 +2272,7 @@ int build_batched(const rg_pair_desc* pairs, int64_t npairs,
             d.nrows = pcs[k].n_out;
             d.ncols = pcs[k].n_in;
             d.batch = J.batch;
-            job_tiles(d, pairs[k].nxo - 1, pairs[k].nyo - 1);
+            job_tiles(d, pairs[k].nxo - 1, pairs[k].nyo - 1, caps->pair_nnz[k]);
             d.block_base = gblocks;
             gprefix.push_back(gblocks);
             gblocks += d.nrt * ((d.batch + JOB_DB - 1) / JOB_DB);
@@ -2536,7 +2537,11 @@ int build_batched(const rg_pair_desc* pairs, int64_t npairs,
                                     "counted buckets (" + std::to_string(cnt2[2]) +
                                         " mismatches)");
         nnz = hbases[2 * npairs];
-        if (caps) caps->nnz_seen = nnz;
+        if (caps) {
+            caps->nnz_seen = nnz;
+            for (int64_t k = 0; k < npairs; k++)
+                caps->pair_nnz.push_back(hbases[2 * k + 2] - hbases[2 * k]);
+        }
         for (int64_t k = 0; k < npairs; k++)
             if (hbases[2 * k + 2] - hbases[2 * k] >= INT32_MAX)
                 return fail(RG_ERR_ARGUMENT, "more than 2^31 - 1 weights in one element");
@@ -2796,6 +2801,7 @@ int graph_create(const rg_pair_desc* pairs, int64_t npairs, const rg_tuning* tun
         const int st = build_batched(pairs, npairs, &t, hs.data(), s, &sizing);
         for (rg_weights* w : hs) weights_release(w);
         if (st != RG_OK) return st;
+        G->caps.pair_nnz = std::move(sizing.pair_nnz);
         G->caps.T_cap = with_slack(sizing.T_seen, slack, 4096);
         G->caps.ov_cap = with_slack(sizing.ov_seen, slack, 4096);
         G->caps.nnz_cap = with_slack(sizing.nnz_seen, slack, 4096);

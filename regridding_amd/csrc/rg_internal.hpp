@@ -163,8 +163,8 @@ struct JobDesc {
 constexpr int JOB_DB = 8;  // images per block
 // Tiles the job's rows, the cells of a (gx, gy) grid (gx * gy == nrows; any
 // other shape is taken as one long row), into blocks; sets gy, ntx, tw, th
-// and nrt.
-void job_tiles(JobDesc& d, int64_t gx, int64_t gy);
+// and nrt.  nnz: the job's entries, as far as known (0: short rows).
+void job_tiles(JobDesc& d, int64_t gx, int64_t gy, int64_t nnz);
 // Launches the FP64 batched apply over a device job table (block prefix
 // `prefix`, `nblocks` blocks in all); every block returns at once when
 // *abort_flag is nonzero (abort_flag may be null).
