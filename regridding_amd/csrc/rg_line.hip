@@ -12,7 +12,8 @@
 // input cells are independent (k_line_count, k_line_emit, one thread per
 // cell).  Any other element (repeated or unordered vertices, NaN) goes
 // through the reference's state machine, replayed by one thread per element
-// (sweep_1d), including its first-point search.  Both reverse descending
+// (sweep_1d), including its first-point search, and so do elements of a few
+// vertices (short_elements).  Both reverse descending
 // grids and emit the wraparound (negative) indices as the reference does.
 // The state machine alone is a serial chain of one memory round trip per
 // step on as many lanes as there are elements: 2048 elements of 2049 -> 1537
@@ -421,7 +422,7 @@ __global__ __launch_bounds__(LINE_BLOCK) void k_line_emit(
     }
 }
 
-// ---- any other element -------------------------------------------------------
+// ---- any other element (all of them, without flags) --------------------------
 
 __global__ void k_cons1d_count(const double* __restrict__ xin, int64_t n,
                                const double* __restrict__ xout, int64_t m,
@@ -429,7 +430,7 @@ __global__ void k_cons1d_count(const double* __restrict__ xin, int64_t n,
                                int32_t* __restrict__ cnt)
 {
     const int64_t d = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (d >= D || !bad[d]) return;
+    if (d >= D || (bad && !bad[d])) return;
     int32_t* c = cnt + d * (n - 1);
     for (int64_t i = 0; i < n - 1; i++) c[i] = 0;
     CountSink sink{c};
@@ -446,7 +447,7 @@ __global__ void k_cons1d_emit(const double* __restrict__ xin, int64_t n,
                               double* __restrict__ w)
 {
     const int64_t d = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (d >= D || !bad[d]) return;
+    if (d >= D || (bad && !bad[d])) return;
     const double* xo = xout + d * m;
     EmitSink sink{off + d * (n - 1), cnt + d * (n - 1), !(xo[0] < xo[m - 1]), ii, io, w};
     sweep_1d(xin + d * n, n, xo, m, wi ? wi + d * (n - 1) : nullptr, sink);
@@ -529,6 +530,15 @@ __global__ void k_zero_flags(int32_t* __restrict__ p, int64_t n)
     if (i < n) p[i] = 0;
 }
 
+// Elements so short that one thread sweeps them sooner than a block finds its
+// cells: us for both passes, serial / by cells, elements of n -> m vertices:
+//   100 to 1000 of 9 -> 7 41 / 48, of 13 -> 10 48 / 49, of 17 -> 13 57 / 48
+//   10^4 of 17 -> 13 59 / 91, of 25 -> 19 74 / 92, of 33 -> 25 89 / 93; 10^5 of 25
+//   -> 19 572 / 589, of 33 -> 25 796 / 594
+//   10^6 of 2 -> 2 57 / 4440, of 9 -> 7 1272 / 5061, of 17 -> 13 4091 / 5817, of 33
+//   -> 5 5342 / 5495, of 25 -> 19 6901 / 6033
+bool short_elements(int64_t n, int64_t m, int64_t D) { return n + m <= (D < 4096 ? 24 : 48); }
+
 constexpr int64_t LINE_GRID = LAUNCH_THREADS / LINE_BLOCK;  // blocks per launch
 
 int check_line(const double* xin, int64_t n, const double* xout, int64_t m, int64_t D)
@@ -558,13 +568,15 @@ int rg_conservative_1d_count(const double* x_input, int64_t n_input,
     *total = 0;
     const int64_t cells = D * (n_input - 1);
     if (cells == 0) return RG_OK;
-    const int64_t nseg = (n_input - 1 + LINE_CELLS - 1) / LINE_CELLS, blocks = D * nseg;
     DevBuf<int32_t> bad;
-    RG_TRY(bad.alloc(D, s));
-    k_zero_flags<<<grid_for(D, 256), 256, 0, s>>>(bad.p, D);
-    for (int64_t b = 0; b < blocks; b += LINE_GRID)
-        k_line_count<<<(unsigned)std::min(blocks - b, LINE_GRID), LINE_BLOCK, 0, s>>>(
-            x_input, n_input, x_output, n_output, nseg, b, bad.p, counts);
+    if (!short_elements(n_input, n_output, D)) {
+        const int64_t nseg = (n_input - 1 + LINE_CELLS - 1) / LINE_CELLS, blocks = D * nseg;
+        RG_TRY(bad.alloc(D, s));
+        k_zero_flags<<<grid_for(D, 256), 256, 0, s>>>(bad.p, D);
+        for (int64_t b = 0; b < blocks; b += LINE_GRID)
+            k_line_count<<<(unsigned)std::min(blocks - b, LINE_GRID), LINE_BLOCK, 0, s>>>(
+                x_input, n_input, x_output, n_output, nseg, b, bad.p, counts);
+    }
     k_cons1d_count<<<grid_for(D, 64), 64, 0, s>>>(x_input, n_input, x_output,
                                                    n_output, D, bad.p, counts);
     RG_HIP(hipGetLastError());
@@ -584,25 +596,28 @@ int rg_conservative_1d_emit(const double* x_input, int64_t n_input,
     if (!counts || !offsets || !indices_input || !indices_output || !values)
         return fail(RG_ERR_ARGUMENT, "NULL array");
     hipStream_t s = (hipStream_t)stream;
-    const int64_t nseg = (n_input - 1 + LINE_CELLS - 1) / LINE_CELLS, blocks = D * nseg;
     DevBuf<int32_t> bad;
-    if (!capturing(s)) {
-        RG_TRY(bad.alloc(D, s));
-        k_zero_flags<<<grid_for(D, 256), 256, 0, s>>>(bad.p, D);
+    const bool by_cells = !short_elements(n_input, n_output, D);
+    if (by_cells) {
+        const int64_t nseg = (n_input - 1 + LINE_CELLS - 1) / LINE_CELLS, blocks = D * nseg;
+        if (!capturing(s)) {
+            RG_TRY(bad.alloc(D, s));
+            k_zero_flags<<<grid_for(D, 256), 256, 0, s>>>(bad.p, D);
+        }
+        for (int64_t b = 0; b < blocks; b += LINE_GRID)
+            k_line_emit<<<(unsigned)std::min(blocks - b, LINE_GRID), LINE_BLOCK, 0, s>>>(
+                x_input, n_input, x_output, n_output, nseg, b, bad.p, weights_input, offsets,
+                indices_input, indices_output, values);
     }
-    for (int64_t b = 0; b < blocks; b += LINE_GRID)
-        k_line_emit<<<(unsigned)std::min(blocks - b, LINE_GRID), LINE_BLOCK, 0, s>>>(
-            x_input, n_input, x_output, n_output, nseg, b, bad.p, weights_input, offsets,
-            indices_input, indices_output, values);
-    if (bad.p)
-        k_cons1d_emit<<<grid_for(D, 64), 64, 0, s>>>(x_input, n_input, x_output, n_output,
-                                                      D, bad.p, weights_input, offsets, counts,
-                                                      indices_input, indices_output, values);
-    else
+    if (by_cells && !bad.p)
         for (int64_t d = 0; d < D; d += LINE_GRID)
             k_cons1d_emit_unordered<<<(unsigned)std::min(D - d, LINE_GRID), LINE_BLOCK, 0, s>>>(
                 x_input, n_input, x_output, n_output, d, weights_input, offsets, counts,
                 indices_input, indices_output, values);
+    else
+        k_cons1d_emit<<<grid_for(D, 64), 64, 0, s>>>(x_input, n_input, x_output, n_output,
+                                                      D, bad.p, weights_input, offsets, counts,
+                                                      indices_input, indices_output, values);
     RG_HIP(hipGetLastError());
     return RG_OK;
 }
