@@ -23,9 +23,9 @@
 // colour and step, and keeps each thread's share of the lists in registers.
 // A slice of up to GS_LDS_CELLS cells runs every iteration in one workgroup
 // in LDS (k_gs_lds).  A larger one runs GS_ITER iterations per launch in
-// tiles with a halo (k_gs_tile); very thin slices, and calls under stream
-// capture or without room for the second buffer, take one launch per step
-// (k_gs_color, k_gs_late).
+// tiles with a halo (k_gs_tile); thin slices too large for the LDS, and calls
+// under stream capture or without room for the second buffer, take one launch
+// per step (k_gs_color, k_gs_late).
 //
 // Linear interpolation (regridding/_interp_ndarray.py:172-269): one lane per
 // output point, clamped linear / bilinear weights.
@@ -152,14 +152,22 @@ __device__ inline void gs_append(E* list, int32_t* n, bool take, E entry, int la
 // entry is the cell (13 bits) and which of its neighbours lie across the
 // periodic wrap (4 bits).  Every thread visiting every cell of both colours,
 // with 64-bit remainders for its neighbours, 100 iterations of 3 slices of 58
-// x 43 took 692 us (4 % masked) and 752 (all); now 84 and 120.
+// x 43 took 692 us (4 % masked) and 752 (all); now 84 and 120.  Slices of one row
+// or column (their cells are their own neighbours across it, and all late) fit
+// the same lists: one of 1 x 1000 72 us, 1.5 ms in a launch per step.
 constexpr int GS_LDS_CELLS = 8192;
 constexpr int GS_LDS_PER = GS_LDS_CELLS / 2 / GS_BLOCK;  // cells per thread and colour
+// Slices of up to GS_SMALL_CELLS take a wavefront each, whose steps need no
+// barrier across wavefronts: 10^5 slices of 8 x 8 0.78 ms (7.1 in blocks of 512),
+// of 16 x 16 all masked 1.42 (7.6); one of 16 x 16 45 us (37).
+constexpr int GS_SMALL_BLOCK = 64, GS_SMALL_CELLS = 256;
+static_assert(GS_SMALL_CELLS / 2 <= GS_SMALL_BLOCK * GS_LDS_PER, "a thread's cells");
 
-// every cell of one slice of (ny, nx) <= GS_LDS_CELLS, both at least 2
-__global__ __launch_bounds__(GS_BLOCK) void k_gs_lds(double* __restrict__ a,
-                                                const uint8_t* __restrict__ where, int ny,
-                                                int nx, int64_t num_iterations, GsCoef c)
+// every cell of one slice of ny x nx <= GS_LDS_CELLS
+template <int BLOCK>
+__global__ __launch_bounds__(BLOCK) void k_gs_lds(double* __restrict__ a,
+                                                  const uint8_t* __restrict__ where, int ny,
+                                                  int nx, int64_t num_iterations, GsCoef c)
 {
     extern __shared__ double s[];
     __shared__ int32_t cnt[3];
@@ -171,7 +179,7 @@ __global__ __launch_bounds__(GS_BLOCK) void k_gs_lds(double* __restrict__ a,
     const uint8_t* wt = where + (int64_t)blockIdx.x * cells;
     if (tid < 3) cnt[tid] = 0;
     __syncthreads();
-    for (int q0 = 0; q0 < cells; q0 += GS_BLOCK) {  // uniform
+    for (int q0 = 0; q0 < cells; q0 += BLOCK) {  // uniform
         const int q = q0 + tid;
         const int j = (unsigned)q / (unsigned)nx, i = q - j * nx;
         const bool in = q < cells && wt[q];
@@ -190,12 +198,12 @@ __global__ __launch_bounds__(GS_BLOCK) void k_gs_lds(double* __restrict__ a,
     uint32_t e0[GS_LDS_PER], e1[GS_LDS_PER];
 #pragma unroll
     for (int t = 0; t < GS_LDS_PER; t++) {
-        const int k = tid + t * GS_BLOCK;
+        const int k = tid + t * BLOCK;
         e0[t] = k < n0 ? list[k] : 0;
         e1[t] = k < n1 ? list1[k] : 0;
     }
     __syncthreads();
-    for (int q = tid; q < cells; q += GS_BLOCK) s[q] = at[q];
+    for (int q = tid; q < cells; q += BLOCK) s[q] = at[q];
     __syncthreads();
     const auto update = [&](uint32_t e) {
         const int q = e & 8191;
@@ -212,16 +220,16 @@ __global__ __launch_bounds__(GS_BLOCK) void k_gs_lds(double* __restrict__ a,
             const int n = colour ? n1 : n0;
 #pragma unroll
             for (int t = 0; t < GS_LDS_PER; t++)
-                if (tid + t * GS_BLOCK < n) update(colour ? e1[t] : e0[t]);
+                if (tid + t * BLOCK < n) update(colour ? e1[t] : e0[t]);
             __syncthreads();
             for (int step = 1; step <= steps; step++) {
-                for (int q = tid; q < nl; q += GS_BLOCK)
+                for (int q = tid; q < nl; q += BLOCK)
                     if (late[q] >> 17 == (uint32_t)(colour | step << 1)) update(late[q]);
                 __syncthreads();
             }
         }
     }
-    for (int q = tid; q < cells; q += GS_BLOCK) at[q] = s[q];
+    for (int q = tid; q < cells; q += BLOCK) at[q] = s[q];
 }
 
 // ---- tiles -------------------------------------------------------------------
@@ -568,10 +576,14 @@ int fill_tiles(double* a, double* other, const uint8_t* where, GsTileLists* list
 int fill_slices(double* a, const uint8_t* where, int64_t T, int64_t ny, int64_t nx,
                 int64_t num_iterations, GsCoef c, hipStream_t s)
 {
-    if (ny * nx <= GS_LDS_CELLS && ny > 1 && nx > 1) {
-        const int64_t late = n_late(ny, nx) + 1;
-        k_gs_lds<<<(unsigned)T, GS_BLOCK, 8 * ny * nx + 4 * late, s>>>(a, where, (int)ny, (int)nx,
-                                                                       num_iterations, c);
+    if (ny * nx <= GS_LDS_CELLS) {
+        const size_t lds = 8 * ny * nx + 4 * (n_late(ny, nx) + 1);
+        if (ny * nx <= GS_SMALL_CELLS)
+            k_gs_lds<GS_SMALL_BLOCK><<<(unsigned)T, GS_SMALL_BLOCK, lds, s>>>(
+                a, where, (int)ny, (int)nx, num_iterations, c);
+        else
+            k_gs_lds<GS_BLOCK><<<(unsigned)T, GS_BLOCK, lds, s>>>(a, where, (int)ny, (int)nx,
+                                                                  num_iterations, c);
         RG_HIP(hipGetLastError());
         return RG_OK;
     }
