@@ -89,10 +89,6 @@ int read_scalars(const void* dev, void* host, size_t bytes, hipStream_t s);
 int read_scalars_begin(const void* dev, size_t bytes, hipStream_t s);
 int read_scalars_end(void* host, size_t bytes);
 
-// Device address, on the current device, of the fixed scratch array of
-// rg_find_cells_2d_noalloc (looked up once per device and kept).
-int find_cells_scratch(int64_t** out);
-
 // Whether work on s is being recorded into a graph: memory of the pool must
 // then not be taken (it would be handed out again while the graph lives).
 bool capturing(hipStream_t s);

@@ -5,7 +5,6 @@
 // the cell-area entry point.
 #include <hip/hip_runtime.h>
 
-#include <mutex>
 #include <string>
 
 #include "rg_internal.hpp"
@@ -20,21 +19,20 @@ constexpr int CELLS_BLOCK = 128;
 
 // One lane per point: the secant iteration of the reference, its cell written
 // as (i, j) or (INT64_MAX, INT64_MAX).  Points the reference would hand to
-// the exhaustive search are marked RG_SEARCH_BRUTE for k_cells_brute: in
-// `mark` (every entry written) when there is one, else in their own row.
+// the exhaustive search are marked RG_SEARCH_BRUTE in their own row for
+// k_cells_brute.
 // 2.36 M points in a 1025^2 vertex grid: 228 us reading every vertex where it
 // is used, 154 reading it once (secant_search).
 __global__ __launch_bounds__(CELLS_BLOCK) void k_cells_secant(
     const double* __restrict__ x, const double* __restrict__ y, int64_t nx, int64_t ny,
     const double* __restrict__ px, const double* __restrict__ py, int64_t n,
-    int64_t* __restrict__ ij, int64_t* __restrict__ mark)
+    int64_t* __restrict__ ij)
 {
     const int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (q >= n) return;
     int64_t ci = INT64_MAX, cj = INT64_MAX;
     const int64_t r = secant_search(VertexArrays{x, y}, nx, ny, px[q], py[q], &ci, &cj);
-    if (mark) mark[q] = r;
-    ij[2 * q] = !mark && r == RG_SEARCH_BRUTE ? RG_SEARCH_BRUTE : ci;
+    ij[2 * q] = r == RG_SEARCH_BRUTE ? RG_SEARCH_BRUTE : ci;
     ij[2 * q + 1] = cj;
 }
 
@@ -46,14 +44,13 @@ __global__ __launch_bounds__(CELLS_BLOCK) void k_cells_secant(
 __global__ __launch_bounds__(256) void k_cells_brute(
     const double* __restrict__ x, const double* __restrict__ y, int64_t nx, int64_t ny,
     const double* __restrict__ px, const double* __restrict__ py, int64_t n, int per,
-    int64_t* __restrict__ ij, const int64_t* __restrict__ mark)
+    int64_t* __restrict__ ij)
 {
     const int64_t q0 = grid_wave() * per;
     const int lane = threadIdx.x & 63;
     if (q0 >= n) return;  // uniform
     const int64_t ql = q0 + lane;
-    uint64_t marked = __ballot(lane < per && ql < n &&
-                               (mark ? mark[ql] : ij[2 * ql]) == RG_SEARCH_BRUTE);
+    uint64_t marked = __ballot(lane < per && ql < n && ij[2 * ql] == RG_SEARCH_BRUTE);
     while (marked) {  // uniform
         const int64_t q = q0 + __builtin_ctzll(marked);
         marked &= marked - 1;
@@ -129,60 +126,19 @@ int check_find_cells(const double* x, const double* y, int64_t nx, int64_t ny,
 
 int launch_find_cells(const double* x, const double* y, int64_t nx, int64_t ny,
                       const double* px, const double* py, int64_t n,
-                      int64_t* cell_ij, int64_t* mark, hipStream_t s)
+                      int64_t* cell_ij, hipStream_t s)
 {
     k_cells_secant<<<grid_for(n, CELLS_BLOCK), CELLS_BLOCK, 0, s>>>(x, y, nx, ny, px, py, n,
-                                                                    cell_ij, mark);
+                                                                    cell_ij);
     int per = 1;
     while (per < 64 && n / (2 * per) >= 8192) per *= 2;
     k_cells_brute<<<grid_for((n + per - 1) / per * 64, 256), 256, 0, s>>>(x, y, nx, ny, px, py, n,
-                                                                          per, cell_ij, mark);
+                                                                          per, cell_ij);
     RG_HIP(hipGetLastError());
     return RG_OK;
 }
 
 }  // namespace
-
-// ---- the cell search without allocation -------------------------------------
-//
-// rg_find_cells_2d_noalloc keeps its per-point scratch in this fixed array
-// (one copy per GPU, RG_FIND_CELLS_NOALLOC_MAX * 8 bytes = 16 MiB, held
-// until the process ends).  Host code never passes the symbol itself to a
-// kernel or copy: on the host it names a host-side stand-in, not device
-// memory.  Its device address is looked up once per device, with that device
-// current, and kept; calls on one GPU share the array, so calls that
-// overlap on one GPU race (issue them on one stream).  Nothing in it needs
-// clearing: the secant kernel writes every entry the exhaustive one reads.
-static __device__ __align__(256) int64_t scratch[RG_FIND_CELLS_NOALLOC_MAX];
-
-namespace {
-
-constexpr int SCRATCH_MAX_DEVICES = 64;
-std::mutex g_scratch_mu;
-int64_t* g_scratch_addr[SCRATCH_MAX_DEVICES] = {};
-
-}  // namespace
-
-int find_cells_scratch(int64_t** out)
-{
-    *out = nullptr;
-    int dev = 0;
-    RG_HIP(hipGetDevice(&dev));
-    if (dev < 0 || dev >= SCRATCH_MAX_DEVICES)
-        return fail(RG_ERR_ARGUMENT, "device " + std::to_string(dev) +
-                                         " beyond the scratch table");
-    std::lock_guard<std::mutex> lk(g_scratch_mu);
-    if (!g_scratch_addr[dev]) {
-        void* p = nullptr;
-        const hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
-        if (e != hipSuccess || !p)
-            return fail(RG_ERR_HIP, std::string("hipGetSymbolAddress(scratch): ") +
-                                        hipGetErrorString(e));
-        g_scratch_addr[dev] = (int64_t*)p;
-    }
-    *out = g_scratch_addr[dev];
-    return RG_OK;
-}
 
 }  // namespace rg
 
@@ -204,7 +160,7 @@ int rg_find_cells_2d(const double* x, const double* y, int64_t nx, int64_t ny,
 {
     if (n == 0) return RG_OK;
     RG_TRY(check_find_cells(x, y, nx, ny, px, py, cell_ij));
-    return launch_find_cells(x, y, nx, ny, px, py, n, cell_ij, nullptr, (hipStream_t)stream);
+    return launch_find_cells(x, y, nx, ny, px, py, n, cell_ij, (hipStream_t)stream);
 }
 
 int rg_find_cells_2d_noalloc(const double* x, const double* y, int64_t nx,
@@ -213,15 +169,14 @@ int rg_find_cells_2d_noalloc(const double* x, const double* y, int64_t nx,
 {
     if (n == 0) return RG_OK;
     RG_TRY(check_find_cells(x, y, nx, ny, px, py, cell_ij));
+    // (the size that its scratch had when there was one)
     if (n < 0 || n > RG_FIND_CELLS_NOALLOC_MAX)
         return fail(RG_ERR_ARGUMENT,
                     "rg_find_cells_2d_noalloc: " + std::to_string(n) +
-                        " points exceed its fixed scratch of " +
+                        " points exceed its fixed scratch size of " +
                         std::to_string((long long)RG_FIND_CELLS_NOALLOC_MAX) +
                         " points per call; search them in slices");
-    int64_t* cell = nullptr;
-    RG_TRY(find_cells_scratch(&cell));
-    return launch_find_cells(x, y, nx, ny, px, py, n, cell_ij, cell, (hipStream_t)stream);
+    return launch_find_cells(x, y, nx, ny, px, py, n, cell_ij, (hipStream_t)stream);
 }
 
 int rg_find_indices_1d(const double* x_input, int64_t m,
