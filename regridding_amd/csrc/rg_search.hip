@@ -36,24 +36,39 @@ __global__ __launch_bounds__(CELLS_BLOCK) void k_cells_secant(
     ij[2 * q + 1] = cj;
 }
 
-// The exhaustive lowest-index search for the marked points, one at a time
-// over a wavefront.  A wavefront looks at `per` points: one while that many
-// wavefronts fill the chip (a marked point costs a pass over the grid), up to
-// 64 of a long list (2.36 M points, none marked: a wavefront each took 217 us,
-// 64 each 6).
-__global__ __launch_bounds__(256) void k_cells_brute(
+// The exhaustive lowest-index search for the marked points, one at a time over
+// a wavefront (a pass over the grid each).  A block looks at BRUTE_WAVES * per
+// points, lists the marked ones and has its wavefronts take them in turn: one
+// point a wavefront while that many wavefronts fill the chip, up to 64 of a long
+// list (2.36 M points, none marked: a wavefront each took 217 us, 64 each 6).
+// Marked points tend to lie together (a masked region), so a block's points are
+// not consecutive: it takes a cache line of rows at a time, BRUTE_LINE points,
+// every gridDim.x lines.  400000 points in 257^2 vertices, the 10000 NaN ones in
+// a row: 2.1 ms a wavefront each, 22 in 64 consecutive ones, now 2.1.
+constexpr int BRUTE_WAVES = 8, BRUTE_LINE = 8;
+constexpr int BRUTE_BLOCK = 64 * BRUTE_WAVES;
+
+__global__ __launch_bounds__(BRUTE_BLOCK) void k_cells_brute(
     const double* __restrict__ x, const double* __restrict__ y, int64_t nx, int64_t ny,
     const double* __restrict__ px, const double* __restrict__ py, int64_t n, int per,
     int64_t* __restrict__ ij)
 {
-    const int64_t q0 = grid_wave() * per;
-    const int lane = threadIdx.x & 63;
-    if (q0 >= n) return;  // uniform
-    const int64_t ql = q0 + lane;
-    uint64_t marked = __ballot(lane < per && ql < n && ij[2 * ql] == RG_SEARCH_BRUTE);
-    while (marked) {  // uniform
-        const int64_t q = q0 + __builtin_ctzll(marked);
-        marked &= marked - 1;
+    __shared__ int32_t list[BRUTE_BLOCK];
+    __shared__ int32_t marked;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const auto point = [&](int t) {  // the block's t-th
+        return (blockIdx.x + (int64_t)(t / BRUTE_LINE) * gridDim.x) * BRUTE_LINE +
+               t % BRUTE_LINE;
+    };
+    if (tid == 0) marked = 0;
+    __syncthreads();
+    const int64_t own = point(tid);
+    if (tid < BRUTE_WAVES * per && own < n && ij[2 * own] == RG_SEARCH_BRUTE)
+        list[atomicAdd(&marked, 1)] = tid;
+    __syncthreads();
+    const int32_t nm = marked;
+    for (int32_t k = block_wave(); k < nm; k += BRUTE_WAVES) {  // uniform per wavefront
+        const int64_t q = point(__builtin_amdgcn_readfirstlane(list[k]));
         const int64_t c = wave_brute(x, y, nx, ny, px[q], py[q], lane);
         if (lane == 0) {
             ij[2 * q] = c >= 0 ? c / (ny - 1) : INT64_MAX;
@@ -131,9 +146,11 @@ int launch_find_cells(const double* x, const double* y, int64_t nx, int64_t ny,
     k_cells_secant<<<grid_for(n, CELLS_BLOCK), CELLS_BLOCK, 0, s>>>(x, y, nx, ny, px, py, n,
                                                                     cell_ij);
     int per = 1;
-    while (per < 64 && n / (2 * per) >= 8192) per *= 2;
-    k_cells_brute<<<grid_for((n + per - 1) / per * 64, 256), 256, 0, s>>>(x, y, nx, ny, px, py, n,
-                                                                          per, cell_ij);
+    while (per < 64 && n / (2 * per) >= 16384) per *= 2;
+    const int64_t lines = (n + BRUTE_LINE - 1) / BRUTE_LINE;
+    static_assert(BRUTE_WAVES == BRUTE_LINE, "a block of BRUTE_WAVES * per points is per lines");
+    k_cells_brute<<<grid_for(lines, per), BRUTE_BLOCK, 0, s>>>(x, y, nx, ny, px, py, n, per,
+                                                               cell_ij);
     RG_HIP(hipGetLastError());
     return RG_OK;
 }
