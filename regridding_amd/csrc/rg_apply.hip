@@ -694,12 +694,12 @@ __global__ void k_to_f32(const double* __restrict__ a, float* __restrict__ b,
 template <class T>
 __global__ __launch_bounds__(APPLY_BLOCK) void k_apply_jobs(
     const JobDesc* __restrict__ jobs, const int64_t* __restrict__ block_prefix,
-    int njobs, int64_t nblocks, const int32_t* __restrict__ abort_flag)
+    int njobs, int64_t first, int64_t nblocks, const int32_t* __restrict__ abort_flag)
 {
     __shared__ T prod[APPLY_BLOCK / 64][PROD_SLOTS];
     if (abort_flag && *abort_flag) return;  // uniform: one word for the grid
     const int64_t ng = gridDim.x;  // a multiple of NUM_XCD
-    const int64_t b = (blockIdx.x % NUM_XCD) * (ng / NUM_XCD) + blockIdx.x / NUM_XCD;
+    const int64_t b = first + (blockIdx.x % NUM_XCD) * (ng / NUM_XCD) + blockIdx.x / NUM_XCD;
     if (b >= nblocks) return;
     const JobDesc& J = jobs[seg_of(block_prefix, njobs, b)];
     const uint32_t lt = (uint32_t)(b - J.block_base), nrt = (uint32_t)J.nrt;
@@ -1042,6 +1042,21 @@ struct JobUpload {
     bool recorded = false;
 };
 
+// The blocks of a job table, in launches within LAUNCH_THREADS.
+template <class T>
+int launch_jobs(const JobDesc* jobs, const int64_t* prefix, int njobs, int64_t nblocks,
+                const int32_t* abort_flag, hipStream_t s)
+{
+    constexpr int64_t MOST = LAUNCH_THREADS / APPLY_BLOCK / NUM_XCD * NUM_XCD;
+    for (int64_t b = 0; b < nblocks; b += MOST) {
+        const int64_t n = std::min(MOST, (nblocks - b + NUM_XCD - 1) / NUM_XCD * NUM_XCD);
+        k_apply_jobs<T><<<(unsigned)n, APPLY_BLOCK, 0, s>>>(jobs, prefix, njobs, b, nblocks,
+                                                            abort_flag);
+    }
+    RG_HIP(hipGetLastError());
+    return RG_OK;
+}
+
 int launch_jobs_common(const rg_apply_job* jobs, int64_t njobs, bool f32,
                        hipStream_t s)
 {
@@ -1115,14 +1130,10 @@ int launch_jobs_common(const rg_apply_job* jobs, int64_t njobs, bool f32,
     up.recorded = true;
     const JobDesc* d_jobs = (const JobDesc*)dt.p;
     const int64_t* d_prefix = (const int64_t*)(dt.p + poff);
-    const unsigned grid = (unsigned)((nblocks + NUM_XCD - 1) / NUM_XCD * NUM_XCD);
     if (f32)
-        k_apply_jobs<float><<<grid, APPLY_BLOCK, 0, s>>>(d_jobs, d_prefix, (int)table.size(),
-                                                         nblocks, nullptr);
+        RG_TRY(launch_jobs<float>(d_jobs, d_prefix, (int)table.size(), nblocks, nullptr, s));
     else
-        k_apply_jobs<double><<<grid, APPLY_BLOCK, 0, s>>>(d_jobs, d_prefix, (int)table.size(),
-                                                          nblocks, nullptr);
-    RG_HIP(hipGetLastError());
+        RG_TRY(launch_jobs<double>(d_jobs, d_prefix, (int)table.size(), nblocks, nullptr, s));
     for (int64_t k = 0; k < njobs; k++) RG_TRY(note_use(jobs[k].weights, s));
     return RG_OK;  // dt returns to the stream's pool after the kernel
 }
@@ -1134,10 +1145,7 @@ int apply_jobs_device(const JobDesc* jobs, const int64_t* prefix, int njobs, int
 {
     if (njobs == 0 || nblocks == 0) return RG_OK;
     if (nblocks >= INT32_MAX) return fail(RG_ERR_ARGUMENT, "batched apply too large");
-    const unsigned grid = (unsigned)((nblocks + NUM_XCD - 1) / NUM_XCD * NUM_XCD);
-    k_apply_jobs<double><<<grid, APPLY_BLOCK, 0, s>>>(jobs, prefix, njobs, nblocks, abort_flag);
-    RG_HIP(hipGetLastError());
-    return RG_OK;
+    return launch_jobs<double>(jobs, prefix, njobs, nblocks, abort_flag, s);
 }
 
 void job_tiles(JobDesc& d, int64_t gx, int64_t gy, int64_t nnz)
