@@ -47,7 +47,8 @@ typedef struct rg_tuning {
                                multiple of 64, at most 512) */
     int32_t flags;          /* RG_TUNE_TIMINGS: record per-phase times;
                                RG_TUNE_GUESS_OUTSIDE, RG_TUNE_ROW_WAVES,
-                               RG_TUNE_REDUCE_GENERAL: test hooks */
+                               RG_TUNE_REDUCE_GENERAL, RG_TUNE_REDUCE_NEAR:
+                               test hooks */
     int32_t stage_per_edge; /* triples staged per sweep edge by the counting
                                walk (default: from the expected work, 8 when
                                edges_per_lane is given; 16 edges per lane
@@ -68,6 +69,10 @@ typedef struct rg_tuning {
  * otherwise for groups too large, or with keys too wide, to sort in registers;
  * the result is the same bits, only slower. */
 #define RG_TUNE_REDUCE_GENERAL 8
+/* Test hook: the register sort counts the output cells of a group from the
+ * group's smallest, in 13 bits (wider groups take the general reduction), as
+ * builds too large for whole output indices do in more bits; same bits. */
+#define RG_TUNE_REDUCE_NEAR 16
 
 /* Counters and (optionally) phase times of a build. */
 typedef struct rg_build_stats {

@@ -1021,15 +1021,25 @@ __device__ inline void put_reduced_cell(KV* __restrict__ dst, const uint64_t* K,
 // instructions where comparing and exchanging 64-bit keys with their values
 // takes eleven.  The values stay behind and are fetched by the sorted keys'
 // slots.
+//
+// Where the output cells of a pair are too many for the bits the ordinals leave
+// (35 million cells at 600 million triples), `near` counts a group's from its
+// smallest: 64 neighbouring input cells meet outputs within a few million of
+// each other, and 23 bits are there at the most triples a build can hold.  A
+// group of wider spread takes the general reduction.  (The reduction of 7701^2
+// -> 5801^2 vertices, 719 M triples: 5.2 ms by the kernels before these, 10.1
+// with every group general, now 4.4.)
 struct KeyBits {
-    int ord, out;  // widths of the ordinal and of the output cell; 0: they do not fit
+    int ord, out;  // widths of the ordinal and of the output cell; out 0: no sorting
+    bool near;     // output cells count from the group's smallest
     static constexpr int SLOT = 6;
-    __device__ uint64_t encode(uint64_t key, int slot) const
+    __device__ uint64_t encode(uint64_t key, int slot, uint32_t out0) const
     {
         // (a capacity-mode build past its capacity may hold wider ordinals:
         // cut, so that the output cell stays in range)
         const uint64_t o = key & (((uint64_t)1 << ord) - 1);
-        return (uint64_t)1 << 62 | ((key >> 32) << ord | o) << SLOT | (uint64_t)slot;
+        const uint32_t c = (uint32_t)(key >> 32) - out0;
+        return (uint64_t)1 << 62 | ((uint64_t)c << ord | o) << SLOT | (uint64_t)slot;
     }
     __device__ uint32_t output(uint64_t code) const
     {
@@ -1107,7 +1117,7 @@ struct RedArgs {
 template <int M, int N, class Values>
 __device__ inline int reduce_sorted(const RedArgs& A, double* __restrict__ slot, int64_t grp,
                                     int64_t base, int32_t* __restrict__ hist_out, int n,
-                                    const Values& values)
+                                    uint32_t out0, const Values& values)
 {
     const int lane = threadIdx.x & 63;
     double k[M];
@@ -1163,7 +1173,7 @@ __device__ inline int reduce_sorted(const RedArgs& A, double* __restrict__ slot,
     if (n > 0) pv[at] = one ? first : first + rest;
     wave_sync_lds();
     for (int e = lane; e < pairs; e += 64) {
-        const uint32_t o = po[e];
+        const uint32_t o = po[e] + out0;
         KV r;
         r.key = (uint64_t)o | (uint64_t)(uint32_t)atomicAdd(&hist_out[o], 1) << 32;
         r.val = pv[e];
@@ -1249,10 +1259,27 @@ __device__ inline int reduce_group(const RedArgs& A, CellSlots<N>& S, int64_t gr
     const int n = S.cnt[lane];
     const int nmax = wave_max(n);
     if (nmax > N) return group_class(total, nmax);  // uniform
+    uint32_t out0 = 0;
+    if (A.bits.near) {  // uniform
+        uint32_t lo = ~0u, hi = 0;
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const uint32_t o = (uint32_t)(rr[u].key >> 32);
+            lo = min(lo, o);
+            hi = max(hi, o);
+        }
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            lo = min(lo, (uint32_t)__shfl_xor((int)lo, o, 64));
+            hi = max(hi, (uint32_t)__shfl_xor((int)hi, o, 64));
+        }
+        out0 = __builtin_amdgcn_readfirstlane(lo);
+        if (((uint32_t)__builtin_amdgcn_readfirstlane(hi) - out0) >> A.bits.out) return 3;
+    }
     A.cell_off[i] = base + wave_exclusive(n, lane);
 #pragma unroll
     for (int u = 0; u < U; u++)
-        S.slot[place[u]] = __builtin_bit_cast(double, A.bits.encode(rr[u].key, place[u] >> 6));
+        S.slot[place[u]] = __builtin_bit_cast(double, A.bits.encode(rr[u].key, place[u] >> 6, out0));
     wave_sync_lds();
     const auto values = [&] {
 #pragma unroll
@@ -1269,7 +1296,7 @@ __device__ inline int reduce_group(const RedArgs& A, CellSlots<N>& S, int64_t gr
             __builtin_amdgcn_sched_barrier(0);
         }
     };
-#define RG_SORTED(M) reduce_sorted<M, N>(A, S.slot, grp, base, hist_out, n, values)
+#define RG_SORTED(M) reduce_sorted<M, N>(A, S.slot, grp, base, hist_out, n, out0, values)
     if constexpr (N <= 24) {
         if (nmax <= 8) return RG_SORTED(8);
         if (nmax <= 16) return RG_SORTED(16);
@@ -1324,7 +1351,7 @@ __global__ __launch_bounds__(64, 3) void k_reduce_cells(RedArgs A, int64_t n_gro
         return;
     }
     int cls = 3;
-    if (A.bits.out == 0 || end - base > LIST2_U * 64) {
+    if (end > base && (A.bits.out == 0 || end - base > LIST2_U * 64)) {
     } else if (end - base <= CELLS_U * 64) {
         cls = reduce_group<CELLS_U, CELLS_N>(A, S, grp);
     } else {
@@ -1880,18 +1907,19 @@ int fill_zero(int32_t* p, int64_t n, hipStream_t s)
     return RG_OK;
 }
 
-// The widths of the reduction's keys for T triples and `most_out` output
-// cells of a pair; none if they and a slot exceed the 61 bits there are.
-KeyBits key_bits(int64_t T, int64_t most_out)
+// The widths of the reduction's keys for T triples (fewer than 2^32) and
+// `most_out` output cells of a pair, in the 61 bits that they and a slot have.
+KeyBits key_bits(int64_t T, int64_t most_out, int32_t flags)
 {
     const auto width = [](int64_t values) {  // bits of 0 .. values - 1, at least one
         int b = 1;
         while (b < 63 && ((int64_t)1 << b) < values) b++;
         return b;
     };
-    KeyBits k = {width(T), width(most_out)};
-    if (k.ord + k.out + KeyBits::SLOT > 61) k = {0, 0};
-    return k;
+    if (flags & RG_TUNE_REDUCE_GENERAL) return {0, 0, false};
+    if (flags & RG_TUNE_REDUCE_NEAR) return {width(T), 13, true};
+    const int ord = width(T), out = width(most_out), room = 61 - KeyBits::SLOT - ord;
+    return {ord, std::min(out, room), out > room};
 }
 
 struct PhaseTimer {
@@ -2482,8 +2510,7 @@ int build_batched(const rg_pair_desc* pairs, int64_t npairs,
     const RedArgs red_args = {bucket_off.p, rec.p,        rcell.p, red.p,         cell_off.p,
                               vol.p,        wi_all.p,     nnz_row.p, group_mode.p, d_pcs,
                               pair_of_ing.p, hist_out.p,
-                              (flags & RG_TUNE_REDUCE_GENERAL) ? KeyBits{0, 0}
-                                                               : key_bits(T, most_out)};
+                              key_bits(T, most_out, flags)};
     DevBuf<int32_t> list1, list2;
     RG_TRY(list1.alloc(n_groups, s));
     RG_TRY(list2.alloc(n_groups, s));
