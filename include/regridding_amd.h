@@ -222,9 +222,9 @@ int rg_weights_set_shape(rg_weights_t w, int64_t ncx_in, int64_t ncy_in,
 /* Launch shape of the apply kernels that stage input patches (several images
  * of weights with 65536 outputs or more; process-wide; 0 keeps the current
  * value): tile_w output cells along the last axis per tile row of a
- * 256-cell tile, twice or four times that (up to 256) where the rows are not
- * whole cache lines and the images are many (default 16; negative: same
- * widths, staged input patches off),
+ * 256-cell tile (default 16; negative: same widths, staged input patches
+ * off), twice or four times that (up to 256) by the kind of value, the rows'
+ * alignment, the images' bytes and the grids' ratio,
  * images_per_pass images accumulated per pass over the weights (1, 2, 4, 8
  * or 16), lds_kib the staged patch size per block (KiB, 1..64) above which
  * fewer images are staged per pass, and rounds (1: one block per tile loops

@@ -26,8 +26,8 @@
 // round-robin) sweeps one contiguous band of tiles, keeping the patches of
 // neighbouring tiles in that XCD's L2.
 //
-// The results are stored nontemporal, where a tile's rows end at cache lines or
-// the images are too many to merge there (launch_apply): each is written once
+// The results are stored nontemporal, except where a tile's rows end inside
+// 64-byte pieces that the caches can merge (planned_shape): each is written once
 // and not read back by the launch, so written through the caches they would
 // only evict the input patches that neighbouring tiles share (at 2049^2 ->
 // 1537^2 and 16 images: FP64 0.239 -> 0.232 ms, FP32 0.164 -> 0.150 ms, FP64
@@ -714,29 +714,58 @@ __global__ __launch_bounds__(APPLY_BLOCK) void k_apply_jobs(
 
 namespace {
 
-// Tile width, and how results are stored (launch_apply).  Where the rows of
-// the output are whole cache lines, tiles are 16 wide (FP32 32, a line, unless
-// the input is much the finer grid) and stores nontemporal.
-// Elsewhere a tile's row ends in two lines that the neighbouring tiles also
-// write, and a nontemporal store sends each part to memory by itself: while
-// the images fit the Infinity Cache with room to spare, the parts are stored
-// through the caches, which merge them; beyond that, tiles are two or four
-// times as wide (fewer parts), the less the more input cells there are to an
-// output, as a wider tile's patch leaves fewer images per pass.
-// us, 16 wide nontemporal / 32 wide nontemporal / 16 wide merged, 16 images:
-//   500^2 -> 999^2 FP64 73.8 / 52.6 / 35.0 (160 MB)
-//   1400^2 -> 1000^2 adjoint FP32 123 / 89.7 / 57.7 (189 MB)
-//   1200^2 -> 1200^2 FP32 92.7 / 65.4 / 50.7 (184 MB); FP64 138 / 103 / 133 (369 MB)
-//   1400^2 -> 1000^2 adjoint FP64 176 / 127 / 166 (379 MB); 8 images 76.7 / 59.6 / 72.1
-//   900^2 -> 1537^2 adjoint FP64 190 / 348 / 183; 2049^2 -> 1537^2 (whole
-//   lines) FP64 232 / 285 / 239, adjoint 285 / 321 / 301
-//   1500^2 -> 2000^2 FP64, 3 images - / 60 / 81 (150 MB)
-// FP32 with whole lines: 2049^2 -> 1537^2 152 us 16 wide, 121 us 32 wide (150
-// and 147 at another angle); without them, beyond the limit, 16 / 32 / 64 wide
-// nontemporal: 1500^2 -> 2000^2 - / 183 / 154, 1600^2 -> 1600^2 - / 120 / 168,
-// 1700^2 -> 1200^2 102 / 89 / -
-constexpr int64_t LINE = 128;
-constexpr double MERGE_BYTES_8 = 130e6, MERGE_BYTES_4 = 190e6;
+// Tile width, and how results are stored, for the apply with a plan.
+//
+// A nontemporal store sends what it holds of a 64-byte piece to memory by
+// itself.  Where the output's rows are whole pieces, so are a tile's, and its
+// results are stored nontemporal.  Elsewhere a tile's row ends in two pieces that
+// the neighbouring tiles also write: while the images fit the Infinity Cache with
+// room to spare, they are stored through the caches, which merge the parts;
+// beyond that, tiles are two or four times as wide (fewer parts), the less the
+// more input cells there are to an output, as a wider tile's patch leaves fewer
+// images per pass; and up to FEW_BYTES the parts cost less than the caches' way
+// (or are left to the wider tiles).  FP32 tiles are 32 wide, 128 bytes, unless the
+// input is much the finer grid or the parts are merged.  us, 16 wide nontemporal /
+// 32 wide nontemporal / 16 wide merged / 64 wide nontemporal, 16 images unless
+// given, where the grids' angles make a range:
+//   whole pieces
+//     2049^2 -> 1537^2 FP64 192-234 / 185-284 / 200-242, its adjoint 231-287 /
+//       212-324 / 231-302; FP32 144-150 / 109-151 / 138-166
+//     1401^2 -> 1001^2 adjoint FP64 72-89 / 70-99 / 119-165
+//     1501^2 -> 2001^2 FP32 81-103 / 76-109 / 149-184 / 77-152 (62.5 lines a row)
+//   others
+//     803^2 -> 642^2 adjoint FP64, 2 images 9.6-12.7 / 9.6-12.6 / 10.5-12.7 (17 MB);
+//       FP32 37 / 26-29 / 19-24 (67 MB)
+//     701^2 -> 1400^2 FP64 155-164 / 103-110 / 105-118 / 79-86 (313 MB); FP32
+//       109-117 / 70-79 / 37-40 / 49-59 (157 MB)
+//     1204^2 -> 903^2 FP64 74-78 / 56-84 / 79-91 (289 MB)
+//     1530^2 -> 1161^2 adjoint FP32 157-161 / 106-117 / 99-107 / 75-118 (236 MB)
+// (A tile as wide as it can be without its patch growing depends on the angle of
+// the grids, which is not known here.)
+constexpr int64_t LINE = 128, PIECE = 64;
+constexpr double FEW_BYTES = 50e6, MERGE_BYTES_8 = 130e6, MERGE_BYTES_4 = 190e6;
+
+struct PlannedShape {
+    int widen;   // tiles g_tile_w << widen
+    bool merge;  // results stored through the caches
+};
+
+PlannedShape planned_shape(int64_t row_bytes, int64_t value_bytes, double bytes, double c)
+{
+    const bool lines = row_bytes % LINE == 0, pieces = row_bytes % PIECE == 0;
+    const bool few = bytes <= FEW_BYTES;
+    const bool small = bytes <= (value_bytes < 8 ? MERGE_BYTES_4 : MERGE_BYTES_8);
+    if (value_bytes >= 8) {
+        if (pieces) return {!lines && !small && c <= 1.75, false};
+        const bool merge = small && !few;
+        return {!merge && c <= 1.9, merge};
+    }
+    if (lines) return {c <= 2.2, false};
+    if (few && c <= 2.2) return {1, false};
+    if (small) return {0, true};
+    return {c <= 0.75 && !pieces ? 2 : c <= 2.2, false};
+}
+
 int g_tile_w = 16;
 int g_images_per_pass = 8;
 // staged patch per block above which fewer images are staged per pass: at
@@ -893,21 +922,13 @@ int launch_apply(rg_weights* W, int dir, const int32_t* rowptr,
                  int64_t src_gy, int64_t batch, hipStream_t s)
 {
     if (nrows == 0 || batch == 0) return RG_OK;
-    const bool lines = shape[0] * shape[1] == nrows && shape[1] * (int64_t)sizeof(T) % LINE == 0;
-    const bool small = (double)batch * (nrows + ncols) * sizeof(T) <=
-                       (sizeof(T) < 8 ? MERGE_BYTES_4 : MERGE_BYTES_8);
-    const bool merge = !lines && small;
-    const double c = (double)ncols / (double)nrows;
-    int widen = 0;
-    if (sizeof(T) >= 8)
-        widen = !lines && !small && c <= 1.75;
-    else if (lines)
-        widen = c <= 2.2;
-    else if (!small)
-        widen = c <= 0.75 ? 2 : c <= 2.2;
+    const double bytes = (double)batch * (nrows + ncols) * sizeof(T);
+    // (a shape that is not known has no plan)
+    const PlannedShape planned = planned_shape(shape[1] * (int64_t)sizeof(T), sizeof(T), bytes,
+                                               (double)ncols / (double)nrows);
     ApplyGrid G;
     rg_weights::Plan* P = nullptr;
-    RG_TRY(ensure_plan(W, dir, widen, rowptr, col, shape, nrows, src_gy, batch, s, &P, &G));
+    RG_TRY(ensure_plan(W, dir, planned.widen, rowptr, col, shape, nrows, src_gy, batch, s, &P, &G));
     int32_t sb = 0;
     if (!P) {
         G = gather_grid(shape, nrows, W->nnz, batch);
@@ -929,8 +950,10 @@ int launch_apply(rg_weights* W, int dir, const int32_t* rowptr,
         // rows of more than 8 entries would read the rest once per image
         // group: the adjoint of 1025^2 -> 1500^2 (7.6 a row where there are
         // any, at most 12), 16 images: FP64 265 -> 195 us, FP32 121 -> 93; at
-        // three or four a row the longer row costs 8 %, at five 1 or 2 % in FP32
-        const bool long_rows = 2 * W->nnz >= 11 * nrows;
+        // three or four a row the longer row costs 8 % in FP32, at five 1 or 2 %;
+        // in FP64 it gains 0 to 8 % from 4.5 a row on
+        const bool long_rows = 2 * W->nnz >= (sizeof(T) < 8 ? 11 : 9) * nrows;
+        const bool merge = planned.merge;
 #define RG_ROUNDS_K(D, E, M)                                                           \
     k_apply_rounds<T, D, E, M><<<g1, bl, (size_t)lds, s>>>(                            \
         rowptr, col, P->off, P->box, w, x, y, nrows, ncols, src_gy, batch, G, lds)
@@ -967,7 +990,11 @@ int launch_apply(rg_weights* W, int dir, const int32_t* rowptr,
 #undef RG_PLANNED
     } else {
         const dim3 gs((unsigned)nb, (unsigned)((batch + sb - 1) / sb));
-        if (merge)
+        // (a wavefront stores 64 values of a row: ends at whole lines, or merged
+        // where the images fit the cache)
+        const bool lines = shape[0] * shape[1] == nrows &&
+                           shape[1] * (int64_t)sizeof(T) % LINE == 0;
+        if (!lines && bytes <= (sizeof(T) < 8 ? MERGE_BYTES_4 : MERGE_BYTES_8))
             k_apply<T, true><<<gs, bl, 0, s>>>(rowptr, col, w, x, y, nrows, ncols, batch, sb, G);
         else
             k_apply<T, false><<<gs, bl, 0, s>>>(rowptr, col, w, x, y, nrows, ncols, batch, sb, G);
