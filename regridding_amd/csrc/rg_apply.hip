@@ -725,7 +725,9 @@ namespace {
 // more input cells there are to an output, as a wider tile's patch leaves fewer
 // images per pass; and up to FEW_BYTES the parts cost less than the caches' way
 // (or are left to the wider tiles).  FP32 tiles are 32 wide, 128 bytes, unless the
-// input is much the finer grid or the parts are merged.  us, 16 wide nontemporal /
+// input is the finer grid or, with the parts merged, the images take several
+// passes (5 of 1202 x 1501 -> 1000 x 1334 24-26 us 16 wide, 22-25 32 wide, the
+// adjoint 25-28 and 25-28).  us, 16 wide nontemporal /
 // 32 wide nontemporal / 16 wide merged / 64 wide nontemporal, 16 images unless
 // given, where the grids' angles make a range:
 //   whole pieces
@@ -750,7 +752,8 @@ struct PlannedShape {
     bool merge;  // results stored through the caches
 };
 
-PlannedShape planned_shape(int64_t row_bytes, int64_t value_bytes, double bytes, double c)
+PlannedShape planned_shape(int64_t row_bytes, int64_t value_bytes, double bytes, double c,
+                           int64_t images)
 {
     const bool lines = row_bytes % LINE == 0, pieces = row_bytes % PIECE == 0;
     const bool few = bytes <= FEW_BYTES;
@@ -762,7 +765,7 @@ PlannedShape planned_shape(int64_t row_bytes, int64_t value_bytes, double bytes,
     }
     if (lines) return {c <= 2.2, false};
     if (few && c <= 2.2) return {1, false};
-    if (small) return {0, true};
+    if (small) return {(!pieces && c <= 0.75) || (images <= JOB_DB && c <= 1.5), true};
     return {c <= 0.75 && !pieces ? 2 : c <= 2.2, false};
 }
 
@@ -925,7 +928,7 @@ int launch_apply(rg_weights* W, int dir, const int32_t* rowptr,
     const double bytes = (double)batch * (nrows + ncols) * sizeof(T);
     // (a shape that is not known has no plan)
     const PlannedShape planned = planned_shape(shape[1] * (int64_t)sizeof(T), sizeof(T), bytes,
-                                               (double)ncols / (double)nrows);
+                                               (double)ncols / (double)nrows, batch);
     ApplyGrid G;
     rg_weights::Plan* P = nullptr;
     RG_TRY(ensure_plan(W, dir, planned.widen, rowptr, col, shape, nrows, src_gy, batch, s, &P, &G));
