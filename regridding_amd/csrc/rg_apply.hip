@@ -92,11 +92,13 @@ constexpr int64_t SPLIT_TILES = 1024;
 // up products one after another, an entry at a time taking the LDS's latency.
 // Rows of 64 entries on average, or of LONG_FEW in few rows (long_rows), get a
 // wavefront each, which is as many chains at once as there are rows and, with
-// several images, images (apply_long_row).  In a wavefront of 64 rows that holds
+// several images, images (apply_long_row).  A wavefront of 64 rows that holds
 // more than LONG_ENTRIES a row (weights of a small input on a large output grid)
-// the sums are pipelined, with several images in chunks of 128, where the
-// registers they take are free.  us for 1 / 8 images of FP64, a lane per row
-// from memory -> rows in chunks only -> this:
+// takes its rows one after another like that where there are several images
+// (four pairs of 2049^2 -> 1025^2, ten times as wide, 3 / 8 images: 2489 / 6060
+// us by a lane per row from memory, 3786 / 10063 by chunks of 128, 1395 / 2882
+// so); with one image its sums are pipelined.  us for 1 / 8 images of FP64, a
+// lane per row from memory -> rows in chunks only -> this:
 //   1025^2 -> 65^2 (239 a row)     90 / 737 -> 423 / 345 -> 12 / 25
 //   2049^2 -> 9^2 (53045)          17456 / 79939 -> 80365 / 89562 -> 1350 / 980
 //   eight of 257^2 -> 17^2 (239)   73 / 645 -> 409 / 3226 -> 15 / 23
@@ -263,6 +265,7 @@ __device__ inline void apply_rows(const int32_t* __restrict__ rowptr,
     e -= first;
     col += first;
     w += first;
+    T* const y0 = y + r0;
     y += r;
     if (lane == 0) prod[PROD_SLOTS - 1] = T(0);
     if (total == 0) {
@@ -270,13 +273,17 @@ __device__ inline void apply_rows(const int32_t* __restrict__ rowptr,
             for (int32_t m = 0; m < images; m++) y[m * nrows] = T(0);
         return;
     }
-    if (images > 1 && rows == 1) {
+    if (images > 1 && (rows == 1 || total > LONG_ENTRIES * rows)) {
         // (eight images in two passes of four)
         const int32_t step = images <= LONG_IMAGES ? images : (images + 1) / 2;
         static_assert(JOB_DB <= 2 * LONG_IMAGES, "two passes");
-        for (int32_t m = 0; m < images; m += step)
-            apply_long_row<MERGE, T>(col, w, x + m * ncols, y + m * nrows, nrows, ncols,
-                                     min(step, images - m), total, prod);
+        for (int32_t q = 0; q < rows; q++) {
+            const int32_t at = __builtin_amdgcn_readlane(s, q);
+            const int32_t n = __builtin_amdgcn_readlane(e, q) - at;
+            for (int32_t m = 0; m < images; m += step)
+                apply_long_row<MERGE, T>(col + at, w + at, x + m * ncols, y0 + q + m * nrows,
+                                         nrows, ncols, min(step, images - m), n, prod);
+        }
         return;
     }
     if (total <= 64 * (ENTRIES_U / 2)) {
@@ -286,14 +293,10 @@ __device__ inline void apply_rows(const int32_t* __restrict__ rowptr,
         for (int32_t c0 = 0; c0 < total; c0 += 64 * ENTRIES_U)
             apply_entries<MERGE, true, T, ENTRIES_U>(col, w, x, y, nrows, ncols, 1, c0, total, s,
                                                      e, valid, prod);
-    } else if (total <= LONG_ENTRIES * rows) {
+    } else {
         for (int32_t c0 = 0; c0 < total; c0 += 64 * ENTRIES_U)
             apply_entries<MERGE, false, T, ENTRIES_U>(col, w, x, y, nrows, ncols, images, c0,
                                                       total, s, e, valid, prod);
-    } else {
-        for (int32_t c0 = 0; c0 < total; c0 += 64 * 2)
-            apply_entries<MERGE, true, T, 2>(col, w, x, y, nrows, ncols, images, c0,
-                                                         total, s, e, valid, prod);
     }
 }
 
