@@ -530,14 +530,23 @@ __global__ void k_zero_flags(int32_t* __restrict__ p, int64_t n)
     if (i < n) p[i] = 0;
 }
 
-// Elements so short that one thread sweeps them sooner than a block finds its
-// cells: us for both passes, serial / by cells, elements of n -> m vertices:
-//   100 to 1000 of 9 -> 7 41 / 48, of 13 -> 10 48 / 49, of 17 -> 13 57 / 48
-//   10^4 of 17 -> 13 59 / 91, of 25 -> 19 74 / 92, of 33 -> 25 89 / 93; 10^5 of 25
-//   -> 19 572 / 589, of 33 -> 25 796 / 594
-//   10^6 of 2 -> 2 57 / 4440, of 9 -> 7 1272 / 5061, of 17 -> 13 4091 / 5817, of 33
-//   -> 5 5342 / 5495, of 25 -> 19 6901 / 6033
-bool short_elements(int64_t n, int64_t m, int64_t D) { return n + m <= (D < 4096 ? 24 : 48); }
+// Elements that one thread each sweeps sooner than a block each finds their
+// cells: few vertices, more of them where the elements are many (a block costs
+// 5.5 ns, what a thread's first 30 us are to 5000 elements), until the sweeps'
+// scattered reads and writes outgrow the caches.  us for both passes, serial /
+// by cells, D elements of n -> m vertices:
+//   300: 9 -> 7 42 / 75, 17 -> 13 58 / 74, 33 -> 5 65 / 65, 33 -> 25 86 / 72
+//   10^4: 33 -> 25 89 / 98, 2 -> 100 108 / 105, 17 -> 60 109 / 106, 60 -> 3 109 / 95
+//   45000: 2 -> 100 159 / 318, 33 -> 25 224 / 295, 2 -> 200 291 / 340, 49 -> 37 332 / 312
+//   10^5: 2 -> 200 561 / 692, 5 -> 60 360 / 644, 17 -> 13 316 / 581, 33 -> 5 384 / 552,
+//     33 -> 25 784 / 605
+//   10^6: 2 -> 50 1796 / 6062, 9 -> 50 6616 / 6439, 17 -> 13 4000 / 5840, 25 -> 19
+//     6780 / 6096, 33 -> 25 9500 / 6199
+bool short_elements(int64_t n, int64_t m, int64_t D)
+{
+    return D < 50000 ? 2 * n + m <= std::min<int64_t>(50 + D / 250, 150)
+                     : (n + m) * std::min<int64_t>(n, 12) <= 600;
+}
 
 constexpr int64_t LINE_GRID = LAUNCH_THREADS / LINE_BLOCK;  // blocks per launch
 

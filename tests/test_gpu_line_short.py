@@ -1,7 +1,7 @@
 """
-1-D conservative weights of short elements, which one thread sweeps, at the
-edges of what counts as short (24 vertices in all, 48 from 4096 elements on),
-next to those that are taken cell by cell: bit for bit against the oracle.
+1-D conservative weights of short elements, of 24 to 48 vertices in all at the
+most, in numbers around 4096: one thread sweeps each or a block takes it cell
+by cell.  Bit for bit against the oracle.
 """
 
 import ctypes
