@@ -9,9 +9,9 @@
 // order, which reproduces the reference bit for bit without atomics.
 //
 // One image, small weights and batched jobs read the entries as they lie and
-// gather from global memory (k_apply, k_apply_jobs).  Several images of large
-// weights stage patches of the input in LDS, DB images at a time, which
-// takes a plan (k_apply_rounds).
+// gather from global memory (k_apply, k_apply_jobs), long rows a wavefront
+// each (long_rows).  Several images of large weights stage patches of the
+// input in LDS, DB images at a time, which takes a plan (k_apply_rounds).
 //
 // The adjoint (transpose=1) is the same gather over the CSR by input, whose
 // rows hold the outputs in ascending order: exactly the order in which the
@@ -19,9 +19,9 @@
 //
 // Launch layout.  The rows of a CSR are the cells of a 2-D grid.  A block
 // of 256 lanes owns a tile of output cells (with a plan tile_w wide along the
-// grid's last axis and 256 / tile_w tall, otherwise 64 and 4), so the input cells it gathers form one
-// compact patch (a linear run of rows would be a thin band tilted across
-// the input grid, re-fetched by every neighbouring run).  Blocks are
+// grid's last axis and 256 / tile_w tall, otherwise 64 and 4), so the input
+// cells it gathers form one compact patch (a linear run of rows would be a thin
+// band tilted across the input grid, re-fetched by every neighbouring run).  Blocks are
 // renumbered so each of the 8 XCDs of the MI355X (blocks arrive
 // round-robin) sweeps one contiguous band of tiles, keeping the patches of
 // neighbouring tiles in that XCD's L2.
