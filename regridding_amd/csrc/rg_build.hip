@@ -1012,65 +1012,7 @@ __device__ inline void put_reduced_cell(KV* __restrict__ dst, const uint64_t* K,
     }
 }
 
-// ---- cells sorted in registers ------------------------------------------------
-//
-// A record's key -- output cell, emission ordinal -- and its place in its
-// cell's slots make one integer below 2^61, which, offset by 2^62, is the bit
-// pattern of a positive normal double: such doubles order as the integers do,
-// so a comparator of the sorting network is v_min_f64 and v_max_f64, two
-// instructions where comparing and exchanging 64-bit keys with their values
-// takes eleven.  The values stay behind and are fetched by the sorted keys'
-// slots.
-//
-// Where the output cells of a pair are too many for the bits the ordinals leave
-// (35 million cells at 600 million triples), `near` counts a group's from its
-// smallest: 64 neighbouring input cells meet outputs within a few million of
-// each other, and 23 bits are there at the most triples a build can hold.  A
-// group of wider spread takes the general reduction.  (The reduction of 7701^2
-// -> 5801^2 vertices, 719 M triples: 5.2 ms by the kernels before these, 10.1
-// with every group general, now 4.4.)
-struct KeyBits {
-    int ord, out;  // widths of the ordinal and of the output cell; out 0: no sorting
-    bool near;     // output cells count from the group's smallest
-    static constexpr int SLOT = 6;
-    __device__ uint64_t encode(uint64_t key, int slot, uint32_t out0) const
-    {
-        // (a capacity-mode build past its capacity may hold wider ordinals:
-        // cut, so that the output cell stays in range)
-        const uint64_t o = key & (((uint64_t)1 << ord) - 1);
-        const uint32_t c = (uint32_t)(key >> 32) - out0;
-        return (uint64_t)1 << 62 | ((uint64_t)c << ord | o) << SLOT | (uint64_t)slot;
-    }
-    __device__ uint32_t output(uint64_t code) const
-    {
-        return (uint32_t)(code >> (ord + SLOT)) & (uint32_t)(((uint64_t)1 << out) - 1);
-    }
-};
-
-// Batcher's odd-even merge sort of N doubles in registers (for N below a
-// power of two, that power's network without the comparators beyond N).
-template <int N>
-__device__ inline void sort_doubles(double* k)
-{
-#pragma unroll
-    for (int p = 1; p < N; p <<= 1) {
-#pragma unroll
-        for (int q = p; q > 0; q >>= 1) {
-#pragma unroll
-            for (int j = q % p; j + q < N; j += 2 * q) {
-#pragma unroll
-                for (int i = 0; i < q; i++) {
-                    const int a = i + j, b = i + j + q;
-                    if (b < N && a / (2 * p) == b / (2 * p)) {
-                        const double lo = fmin(k[a], k[b]);
-                        k[b] = fmax(k[a], k[b]);
-                        k[a] = lo;
-                    }
-                }
-            }
-        }
-    }
-}
+// ---- cells sorted in registers (KeyBits, sort_doubles: rg_sweep.hpp) -----------
 
 // One group's slots: entry d of cell c at d * 64 + c, so the lanes (one per
 // cell) touch consecutive words at every step.  Keys first, then values.  Row
@@ -1125,22 +1067,10 @@ __device__ inline int reduce_sorted(const RedArgs& A, double* __restrict__ slot,
     for (int j = 0; j < M; j++)
         k[j] = j < n ? slot[j * 64 + lane] : __builtin_bit_cast(double, 0x7fe0000000000000ull);
     sort_doubles<M>(k);
-    // the first record of each run of one output; from here on a record is
-    // its output and its slot
-    uint64_t heads = 0;
     uint32_t out[M];
     uint8_t from[M];
-#pragma unroll
-    for (int j = 0; j < M; j++) {
-        const uint64_t c = __builtin_bit_cast(uint64_t, k[j]);
-        out[j] = A.bits.output(c);
-        from[j] = (uint8_t)(c & 63);  // (0 past the cell's last)
-        if (j < n && (j == 0 || out[j] != out[j > 0 ? j - 1 : 0])) heads |= (uint64_t)1 << j;
-    }
-    uint64_t more = ~heads & (n < 64 ? ((uint64_t)1 << n) - 1 : ~(uint64_t)0);
-    more &= more >> 1;
-    more &= more >> 2;
-    more &= more >> 4;
+    uint64_t more;
+    const uint64_t heads = run_heads<M>(A.bits, k, n, out, from, &more);
     const int m = __popcll(heads);
     const int dst = wave_exclusive(m, lane);
     const int pairs = __builtin_amdgcn_readlane(dst + m, 63);
@@ -1153,24 +1083,9 @@ __device__ inline int reduce_sorted(const RedArgs& A, double* __restrict__ slot,
 #pragma unroll
     for (int j = 0; j < M; j++) v[j] = slot[(int)from[j] * 64 + lane];
     wave_sync_lds();  // every lane has its values: the slots take the pairs
-    // each run: its first term plus the sum of the others from -0.0
     double* const pv = slot;
     uint32_t* const po = reinterpret_cast<uint32_t*>(slot + room);
-    int at = dst - 1;
-    double first = 0, rest = -0.0;
-    bool one = true;
-#pragma unroll
-    for (int j = 0; j < M; j++) {
-        const bool head = heads >> j & 1;
-        if (head) {
-            if (j > 0) pv[at] = one ? first : first + rest;
-            po[++at] = out[j];
-        }
-        first = head ? v[j] : first;
-        rest = head ? -0.0 : (j < n ? rest + v[j] : rest);
-        one = head || (one && j >= n);
-    }
-    if (n > 0) pv[at] = one ? first : first + rest;
+    sum_runs<M>(v, out, heads, n, pv + dst, po + dst);
     wave_sync_lds();
     for (int e = lane; e < pairs; e += 64) {
         const uint32_t o = po[e] + out0;
@@ -1907,19 +1822,11 @@ int fill_zero(int32_t* p, int64_t n, hipStream_t s)
     return RG_OK;
 }
 
-// The widths of the reduction's keys for T triples (fewer than 2^32) and
-// `most_out` output cells of a pair, in the 61 bits that they and a slot have.
 KeyBits key_bits(int64_t T, int64_t most_out, int32_t flags)
 {
-    const auto width = [](int64_t values) {  // bits of 0 .. values - 1, at least one
-        int b = 1;
-        while (b < 63 && ((int64_t)1 << b) < values) b++;
-        return b;
-    };
     if (flags & RG_TUNE_REDUCE_GENERAL) return {0, 0, false};
-    if (flags & RG_TUNE_REDUCE_NEAR) return {width(T), 13, true};
-    const int ord = width(T), out = width(most_out), room = 61 - KeyBits::SLOT - ord;
-    return {ord, std::min(out, room), out > room};
+    if (flags & RG_TUNE_REDUCE_NEAR) return {KeyBits::width(T), 13, true};
+    return KeyBits::of(T, most_out);
 }
 
 struct PhaseTimer {

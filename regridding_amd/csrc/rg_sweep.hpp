@@ -875,6 +875,127 @@ RG_HD void sort_network(K* k, double* v)
     }
 }
 
+// ---- cells sorted in registers ------------------------------------------------
+//
+// A record's key -- output cell, emission ordinal -- and its place in its
+// cell's slots make one integer below 2^61, which, offset by 2^62, is the bit
+// pattern of a positive normal double: such doubles order as the integers do,
+// so a comparator of the sorting network is v_min_f64 and v_max_f64, two
+// instructions where comparing and exchanging 64-bit keys with their values
+// takes eleven.  The values stay behind and are fetched by the sorted keys'
+// slots.
+//
+// Where the output cells of a pair are too many for the bits the ordinals leave
+// (35 million cells at 600 million triples), `near` counts a group's from its
+// smallest: 64 neighbouring input cells meet outputs within a few million of
+// each other, and 23 bits are there at the most triples a build can hold.  A
+// group of wider spread takes the general reduction.  (The reduction of 7701^2
+// -> 5801^2 vertices, 719 M triples: 5.2 ms by the kernels before these, 10.1
+// with every group general, now 4.4.)
+struct KeyBits {
+    int ord, out;  // widths of the ordinal and of the output cell; out 0: no sorting
+    bool near;     // output cells count from the group's smallest
+    static constexpr int SLOT = 6;
+    // bits of 0 .. values - 1, at least one
+    RG_HD static int width(int64_t values)
+    {
+        int b = 1;
+        while (b < 63 && ((int64_t)1 << b) < values) b++;
+        return b;
+    }
+    // for T triples (fewer than 2^32) and `most_out` output cells of a pair, in
+    // the 61 bits that they and a slot have
+    RG_HD static KeyBits of(int64_t T, int64_t most_out)
+    {
+        const int ord = width(T), out = width(most_out), room = 61 - SLOT - ord;
+        return {ord, out < room ? out : room, out > room};
+    }
+    RG_HD uint64_t encode(uint64_t key, int slot, uint32_t out0) const
+    {
+        // (a capacity-mode build past its capacity may hold wider ordinals:
+        // cut, so that the output cell stays in range)
+        const uint64_t o = key & (((uint64_t)1 << ord) - 1);
+        const uint32_t c = (uint32_t)(key >> 32) - out0;
+        return (uint64_t)1 << 62 | ((uint64_t)c << ord | o) << SLOT | (uint64_t)slot;
+    }
+    RG_HD uint32_t output(uint64_t code) const
+    {
+        return (uint32_t)(code >> (ord + SLOT)) & (uint32_t)(((uint64_t)1 << out) - 1);
+    }
+};
+
+// Batcher's odd-even merge sort of N doubles in registers (for N below a
+// power of two, that power's network without the comparators beyond N).
+template <int N>
+RG_HD void sort_doubles(double* k)
+{
+#pragma unroll
+    for (int p = 1; p < N; p <<= 1) {
+#pragma unroll
+        for (int q = p; q > 0; q >>= 1) {
+#pragma unroll
+            for (int j = q % p; j + q < N; j += 2 * q) {
+#pragma unroll
+                for (int i = 0; i < q; i++) {
+                    const int a = i + j, b = i + j + q;
+                    if (b < N && a / (2 * p) == b / (2 * p)) {
+                        const double lo = fmin(k[a], k[b]);
+                        k[b] = fmax(k[a], k[b]);
+                        k[a] = lo;
+                    }
+                }
+            }
+        }
+    }
+}
+
+// A cell's sorted codes k[0 .. n): the bits of the first record of each run of
+// one output cell, every record's output cell and slot, and in *more whether a
+// run is too long for a sequential sum (numpy's pairwise order differs from 8
+// further terms on).
+template <int M>
+RG_HD uint64_t run_heads(const KeyBits& bits, const double* k, int n, uint32_t* out,
+                         uint8_t* from, uint64_t* more)
+{
+    uint64_t heads = 0;
+#pragma unroll
+    for (int j = 0; j < M; j++) {
+        const uint64_t c = __builtin_bit_cast(uint64_t, k[j]);
+        out[j] = bits.output(c);
+        from[j] = (uint8_t)(c & 63);  // (0 past the cell's last)
+        if (j < n && (j == 0 || out[j] != out[j > 0 ? j - 1 : 0])) heads |= (uint64_t)1 << j;
+    }
+    uint64_t m = ~heads & (n < 64 ? ((uint64_t)1 << n) - 1 : ~(uint64_t)0);
+    m &= m >> 1;
+    m &= m >> 2;
+    m &= m >> 4;
+    *more = m;
+    return heads;
+}
+
+// Each run's sum, its first term plus the sum of the others from -0.0, and its
+// output cell, to pv[0 ..] and po[0 ..].
+template <int M>
+RG_HD void sum_runs(const double* v, const uint32_t* out, uint64_t heads, int n, double* pv,
+                    uint32_t* po)
+{
+    int at = -1;
+    double first = 0, rest = -0.0;
+    bool one = true;
+#pragma unroll
+    for (int j = 0; j < M; j++) {
+        const bool head = heads >> j & 1;
+        if (head) {
+            if (j > 0) pv[at] = one ? first : first + rest;
+            po[++at] = out[j];
+        }
+        first = head ? v[j] : first;
+        rest = head ? -0.0 : (j < n ? rest + v[j] : rest);
+        one = head || (one && j >= n);
+    }
+    if (n > 0) pv[at] = one ? first : first + rest;
+}
+
 // Completion of a bucket left sorted (KV records, weights already divided)
 // by bucket_reduce: any run length; the values of each run are consumed in
 // place.

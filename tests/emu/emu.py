@@ -128,6 +128,23 @@ def bucket_reduce(keys, vals, stride: int = 1):
     return int(m), bool(lr.value), kb[: n * stride: stride].copy(), vb[: n * stride: stride].copy()
 
 
+def registers_reduce(m, triples, most_out, keys, vals, out0=0):
+    """One cell's records (any order) through the register reduction of size m:
+    (count or -1, near, output cells, sums)."""
+    keys = np.ascontiguousarray(keys, dtype=np.uint64)
+    vals = np.ascontiguousarray(vals, dtype=np.float64)
+    po, pv = np.zeros(64, np.uint32), np.full(64, np.nan)
+    near = ctypes.c_int32(0)
+    L = lib()
+    L.rge_registers_reduce.restype = _i64
+    L.rge_registers_reduce.argtypes = [ctypes.c_int, _i64, _i64, ctypes.c_void_p, _pd, ctypes.c_int,
+                                       ctypes.c_uint32, ctypes.POINTER(ctypes.c_int32),
+                                       ctypes.c_void_p, _pd]
+    c = L.rge_registers_reduce(m, triples, most_out, keys.ctypes.data, _d(vals), len(keys),
+                               int(out0), ctypes.byref(near), po.ctypes.data, _d(pv))
+    return int(c), bool(near.value), po[:max(c, 0)].copy(), pv[:max(c, 0)].copy()
+
+
 def reduceat_segment_inplace(a, stride: int = 1) -> float:
     """The stackless in-place variant (on a strided copy of ``a``)."""
     a = np.asarray(a, dtype=np.float64)

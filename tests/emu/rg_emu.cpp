@@ -438,6 +438,54 @@ void rge_sort_network(uint64_t* keys, double* vals, int64_t count, int n)
     }
 }
 
+// One cell's records (at most m = 8, 16, 24, 32, 48 or 64) through the register
+// reduction: keys of `triples` triples and `most_out` output cells, counted from
+// out0 where they are too many.  Returns the count of output cells, -1 if a run
+// is too long; *near says whether out0 counted.
+}  // extern "C"
+
+namespace {
+
+template <int M>
+int64_t registers_reduce(const KeyBits& bits, const uint64_t* keys, const double* vals, int n,
+                         uint32_t out0, uint32_t* po, double* pv)
+{
+    double k[M], v[M];
+    uint32_t out[M];
+    uint8_t from[M];
+    uint64_t more;
+    for (int j = 0; j < M; j++)
+        k[j] = __builtin_bit_cast(double, j < n ? bits.encode(keys[j], j, out0)
+                                                : (uint64_t)0x7fe0000000000000ull);
+    sort_doubles<M>(k);
+    const uint64_t heads = run_heads<M>(bits, k, n, out, from, &more);
+    if (more) return -1;
+    for (int j = 0; j < M; j++) v[j] = j < n ? vals[from[j]] : 0.0;
+    sum_runs<M>(v, out, heads, n, pv, po);
+    return __builtin_popcountll(heads);
+}
+
+}  // namespace
+
+extern "C" {
+
+int64_t rge_registers_reduce(int m, int64_t triples, int64_t most_out, const uint64_t* keys,
+                             const double* vals, int n, uint32_t out0, int32_t* near,
+                             uint32_t* po, double* pv)
+{
+    const KeyBits bits = KeyBits::of(triples, most_out);
+    *near = bits.near;
+    if (!bits.near) out0 = 0;
+    switch (m) {
+    case 8: return registers_reduce<8>(bits, keys, vals, n, out0, po, pv);
+    case 16: return registers_reduce<16>(bits, keys, vals, n, out0, po, pv);
+    case 24: return registers_reduce<24>(bits, keys, vals, n, out0, po, pv);
+    case 32: return registers_reduce<32>(bits, keys, vals, n, out0, po, pv);
+    case 48: return registers_reduce<48>(bits, keys, vals, n, out0, po, pv);
+    default: return registers_reduce<64>(bits, keys, vals, n, out0, po, pv);
+    }
+}
+
 double rge_reduceat_segment(const double* a, int64_t n)
 {
     return reduceat_segment(a, n);
